@@ -42,6 +42,7 @@ Scene::~Scene() {
 	if (fpart) hipFree(fpart);
 	if (dscal) hipFree(dscal);
 	if (code) hipFree(code);
+	if (res.words) hipFree(res.words);
 	if (hscal) hipHostFree(hscal);
 	if (ev) hipEventDestroy(ev);
 	if (evState) hipEventDestroy(evState);

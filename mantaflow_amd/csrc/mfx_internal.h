@@ -67,6 +67,14 @@ struct Dims {
 struct Grid;
 class MgHierarchy;
 
+// exchange words of the one-kernel CG (mfx_resident.h) and the first tag not
+// yet used on them
+struct ResWords {
+	unsigned long long* words = nullptr;
+	size_t count = 0;
+	unsigned next = 0;  // 0: the words have not been cleared
+};
+
 struct Scene {
 	Dims d;
 	int dim;
@@ -105,6 +113,7 @@ struct Scene {
 	long long micFix = -1;
 	uint64_t* dhash = nullptr;  // device word of the code hash
 	uint64_t* hhash = nullptr;  // its pinned host mirror
+	ResWords res;               // exchange words of the one-kernel CG
 	uint8_t* code = nullptr;    // per-cell Laplace matrix code of the current solve
 	std::vector<Grid*> grids;
 	~Scene();

@@ -45,6 +45,7 @@
 #include "mfx_internal.h"
 #include "mfx_mg.h"
 #include "mfx_prof.h"
+#include "mfx_resident.h"
 
 namespace mfx {
 
@@ -1690,6 +1691,8 @@ struct CgRun {
 	double* dpart = nullptr;
 	float* fpart = nullptr;
 	uint8_t* code = nullptr;
+	ResWords* res = nullptr;  // exchange words of the one-kernel CG (the scene's when pooled)
+	bool resident = false;    // the iterations ran, or run, as one kernel
 	int pc = 0, maxIter = 0;
 	bool pcNone = true;
 	MgHierarchy* mg = nullptr;
@@ -1803,6 +1806,51 @@ static void autotune_zmarch(Scene* s, const uint8_t* code) {
 
 static int precondition(CgRun& R);
 
+// doInit of the general kernels: x = 0, r = b, ||b||, sigma = dot(r, r)
+static void cg_init(CgRun& R) {
+	Scene* s = R.s;
+	hipLaunchKernelGGL(k_cg_init, dim3(R.nbU), dim3(kBlock), 0, s->stream, s->d, R.per, (const float*)R.rhs, R.x, R.r,
+	                   R.pcNone ? 1 : 0, R.dpart);
+	run_finalize_one(s->stream, FinP{R.st, R.dpart, R.fpart, (int)R.nbU, FIN_INIT, 0});
+}
+
+// Unpreconditioned solves of grids that fit the one-kernel CG: doInit and
+// every iteration as one launch.  Returns false where the general kernels
+// have to run.  At most 5 s may pass before a workgroup gives up waiting for
+// another (cg_verify then runs the solve on the general kernels).
+constexpr long long kResWaitTicks = 5ll * 100000000ll;
+static long long g_res_wait = kResWaitTicks;
+static bool cg_try_resident(CgRun& R) {
+	Scene* s = R.s;
+	if (!R.pcNone || R.gA0 || R.o.trueResidualEvery > 0) return false;
+	const ResPlan pl = cg_resident_plan(s->d);
+	if (!pl.V) return false;
+	ResWords& w = R.res ? *R.res : s->res;
+	if (pl.wg > 1 && !w.words) {
+		if (R.res) return false;
+		w.count = kResSlotWords + pl.words;
+		MFX_HIP(hipMalloc((void**)&w.words, sizeof(unsigned long long) * w.count));
+	}
+	ResP p;
+	p.d = s->d;
+	p.st = R.st;
+	p.code = R.code;
+	p.b = R.rhs;
+	p.x = R.x;
+	p.scaled = R.scaled;
+	p.scale = R.scale;
+	p.xs = w.words;
+	p.xr = w.words ? w.words + kResSlotWords : nullptr;
+	p.epoch = cg_resident_tags(w, s->stream, pl, R.maxIter);
+	p.limit = g_res_wait;
+	{
+		KtScope kt("cg_resident", s->stream);
+		cg_resident_run(s->stream, pl, p);
+	}
+	R.resident = true;
+	return true;
+}
+
 static void cg_setup(CgRun& R, Scene* s, Grid* flags, float* rhs, float* x, const mfx_pressure_opts& o,
                      bool batchInit = false, const BndDev* bnd = nullptr) {
 	R.t0 = std::chrono::steady_clock::now();
@@ -1907,9 +1955,9 @@ static void cg_setup(CgRun& R, Scene* s, Grid* flags, float* rhs, float* x, cons
 	}
 
 	// doInit: x = 0, r = b, bnorm; preconditioned: z = M r, sigma = dot(z, r)
-	hipLaunchKernelGGL(k_cg_init, dim3(R.nbU), dim3(kBlock), 0, s->stream, d, R.per, (const float*)rhs, x, R.r,
-	                   R.pcNone ? 1 : 0, R.dpart);
-	run_finalize_one(s->stream, FinP{R.st, R.dpart, R.fpart, (int)R.nbU, FIN_INIT, 0});
+	R.launched = 0;
+	if (cg_try_resident(R)) return;
+	cg_init(R);
 	if (R.gA0 && !R.pcNone) {
 		R.gS = s->getReal();
 		R.gT = s->getReal();
@@ -2069,6 +2117,13 @@ static void cg_iterate_finish(CgRun& R, double target) {
 }
 
 static void cg_verify(CgRun& R, double target) {
+	if (R.resident && ((const CgState*)R.s->hscal)->pad) {
+		// the one-kernel solve gave up: again, on the general kernels
+		R.resident = false;
+		R.launched = 0;
+		cg_init(R);
+		cg_iterate_finish(R, target);
+	}
 	for (int k = 0; k < kMaxRestarts && cg_needs_restart(R); k++) {
 		// iterations queued past convergence did nothing; the budget follows
 		// the device count (p = z after the restart, so the buffer parity is free)
@@ -2122,6 +2177,7 @@ static void solve_system(Scene* s, Grid* flags, float* rhs, float* x, const mfx_
 		R.z = bufs->r;
 		R.dpart = bufs->dpart;
 		R.fpart = bufs->fpart;
+		R.res = bufs->res;
 	}
 	cg_setup(R, s, flags, rhs, x, o, false, bnd);
 	cg_drive(R, o.relTol > 0 ? o.relTol : (double)o.cgAccuracy, stats);
@@ -2131,7 +2187,12 @@ static void solve_system(Scene* s, Grid* flags, float* rhs, float* x, const mfx_
 // stopping rule holds or maxIter is reached, then finish (statistics,
 // divergence error).  target: the stopping threshold the prediction aims at.
 static void cg_drive(CgRun& R, double target, mfx_solve_stats* stats) {
-	cg_iterate_finish(R, target);
+	if (R.resident) {
+		cg_true_residual_enqueue(R);
+		sync(R.s);
+	} else {
+		cg_iterate_finish(R, target);
+	}
 	cg_verify(R, target);
 	cg_release(R);
 	cg_finish_collect(R, stats);
@@ -2227,10 +2288,8 @@ static void solve_scaled(Scene* s, Grid* flags, float* rhs, float* x, int kind, 
 	R.pb = s->getReal();
 	R.q = s->getReal();
 	R.z = R.r;
-	hipLaunchKernelGGL(k_cg_init, dim3(R.nbU), dim3(kBlock), 0, s->stream, d, R.per, (const float*)rhs, x, R.r, 1,
-	                   R.dpart);
-	run_finalize_one(s->stream, FinP{R.st, R.dpart, R.fpart, (int)R.nbU, FIN_INIT, 0});
 	R.launched = 0;
+	if (!cg_try_resident(R)) cg_init(R);
 	cg_drive(R, (double)cgAccuracy, stats);
 }
 
@@ -2825,6 +2884,14 @@ extern "C" void mfx_testing_zmarch_chunks(int nx, int ny, int nz, int* mv, int* 
 	if (mv) *mv = t.mv;
 	if (l0) *l0 = t.l0;
 }
+// Testing hook: the longest wait of the one-kernel CG in wall clock ticks
+// (0: every solve of more than one workgroup gives up and runs on the general
+// kernels; < 0 restores the default).  Returns the previous value.
+extern "C" long long mfx_testing_resident_wait(long long ticks) {
+	const long long prev = g_res_wait;
+	g_res_wait = ticks < 0 ? kResWaitTicks : ticks;
+	return prev;
+}
 // Testing hook: set the plane chunks that single solves of a shape use
 // (multiples of 4 up to 64; 0,0 = autotune again).  Returns 0, or -1 for a
 // chunk the z-marching kernels do not accept.
@@ -3038,13 +3105,17 @@ constexpr size_t kNaVec = al256((size_t)kNoAllocMaxCells * sizeof(float));
 constexpr size_t kNaCode = al256((size_t)kNoAllocMaxCells);
 constexpr size_t kNaDPart = al256((3 * kNoAllocMaxPartBlocks + 16) * sizeof(double));
 constexpr size_t kNaFPart = al256((2 * kNoAllocMaxPartBlocks + 16) * sizeof(float));
-constexpr size_t kNoAllocBytes = 5 * kNaVec + kNaCode + kNaDPart + kNaFPart;
+// exchange words of the one-kernel CG (at most 8192 cells a workgroup)
+constexpr size_t kNaResWords = kResSlotWords + (size_t)kResMaxWG * 8192;
+constexpr size_t kNaRes = al256(kNaResWords * sizeof(unsigned long long));
+constexpr size_t kNoAllocBytes = 5 * kNaVec + kNaCode + kNaDPart + kNaFPart + kNaRes;
 }  // namespace
 
 static __device__ __align__(256) unsigned char scratch[kNoAllocBytes];
 
 static std::mutex g_scratch_mu;
 static void* g_scratch_dev[64];
+static ResWords g_scratch_res[64];
 
 // device address of `scratch` on device dev (looked up once per device, with
 // that device current)
@@ -3061,6 +3132,9 @@ static unsigned char* scratch_on(int dev) {
 		MFX_CHECK(e == hipSuccess && p != nullptr,
 		          std::string("solvePressureNoAlloc: hipGetSymbolAddress(scratch) failed: ") + hipGetErrorString(e));
 		g_scratch_dev[dev] = p;
+		g_scratch_res[dev].words =
+		    (unsigned long long*)((unsigned char*)p + 5 * kNaVec + kNaCode + kNaDPart + kNaFPart);
+		g_scratch_res[dev].count = kNaResWords;
 	}
 	return (unsigned char*)g_scratch_dev[dev];
 }
@@ -3127,6 +3201,7 @@ int mfx_solve_pressure_noalloc(mfx_grid* vel, mfx_grid* pressure, const mfx_grid
 	B.code = base + 5 * kNaVec;
 	B.dpart = (double*)(base + 5 * kNaVec + kNaCode);
 	B.fpart = (float*)(base + 5 * kNaVec + kNaCode + kNaDPart);
+	B.res = &g_scratch_res[dev];
 	compute_rhs(s, f, v, rhs, o.enforceCompatibility, B.dpart);
 	solve_system(s, f, rhs, p->real(), o, stats, &B);
 	correct_velocity(s, f, v, p->real());
