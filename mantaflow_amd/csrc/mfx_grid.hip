@@ -34,6 +34,7 @@ void set_last_error(const std::string& s) { g_err = s; }
 Scene::~Scene() {
 	if (stream) hipStreamSynchronize(stream);
 	mgStatic.reset();
+	mgDyn.reset();
 	mgMic.reset();
 	if (dhash) hipFree(dhash);
 	if (hhash) hipHostFree(hhash);

@@ -104,6 +104,7 @@ struct Scene {
 	hipGraphExec_t bexec = nullptr;
 	std::vector<long long> bkey, blastKey;
 	std::unique_ptr<MgHierarchy> mgStatic;
+	std::unique_ptr<MgHierarchy> mgDyn;  // PcMGDynamic: rebuilt by every solve, in the same memory
 	// multigrid hierarchy standing in for PcMIC (the reference's mIC keeps
 	// nothing between solves): rebuilt whenever the matrix code changes,
 	// checked by the flag grid's generation and a hash of the code

@@ -50,11 +50,16 @@ struct MgLevel {
 	bool hasCanon = false;
 };
 
+struct CanonSlot;
 class MgHierarchy {
 public:
+	MgHierarchy() = default;
+	MgHierarchy(const MgHierarchy&) = delete;
+	MgHierarchy& operator=(const MgHierarchy&) = delete;
 	~MgHierarchy();
 	// builds levels, coarse operators and the coarsest-level inverse from the
-	// level-0 matrix code
+	// level-0 matrix code; called again for another matrix of the same scene
+	// it works in the memory it has
 	void build(Scene* s, const uint8_t* code, int precision);
 	// z = V-cycle(r) from z = 0; kernels skip their work once st->done is set.
 	// Returns the number of partial sums of fl(z*r) the last kernel wrote into
@@ -67,7 +72,8 @@ public:
 	            bool tuned, int forceChunk = 0) const;
 	bool dim3d() const { return is3d; }
 	int levels() const { return (int)L.size(); }
-	int precision() const { return prec; }
+	// (-1: the last build did not finish)
+	int precision() const { return ready ? prec : -1; }
 
 private:
 	bool is3d = true;
@@ -75,13 +81,20 @@ private:
 	int prec = 0;                // 0: FP32 coefficients, 1: BF16 smoother/residual coefficients
 	std::vector<MgLevel> L;      // L[0] holds only r (x = z, b = rhs on the fly)
 	double* G = nullptr;         // dense generalized inverse of the coarsest operator
-	int* cidx = nullptr;         // active coarsest vertices
+	int* cidx = nullptr;         // active coarsest vertices, then (contiguous)
+	int* cpos = nullptr;         //   their numbers by vertex (-1 inactive)
+	int* cpin = nullptr;         //   and the pinned ones
 	int nc = 0;
-	float* bc = nullptr;         // gathered coarsest rhs (double via G)
-	std::vector<void*> allocs;
-	void* alloc(size_t bytes);
+	bool ready = false;
+	void* arena = nullptr;       // all of the hierarchy's device memory
+	void* hbuf = nullptr;        // pinned: what a build reads and writes on the host
+	size_t hostBytes = 0, readBytes = 0;
+	float* zero = nullptr;       // vectors that start a hierarchy at 0
+	long long nzero = 0;
+	CanonSlot* picks = nullptr;  // canonical stencils as picked, by level
+	double *sweepD = nullptr, *sweepW = nullptr, *sweepP = nullptr, *cdiag = nullptr;
+	void layout(Scene* s);
 	void build_coarsest(Scene* s, const uint8_t* code0);
-	void classify(Scene* s, int l);
 };
 
 }  // namespace mfx

@@ -21,6 +21,7 @@
 //    sequential FP64 Jacobi-PCG (:796-902).  This also makes the V-cycle well
 //    defined for pure-Neumann problems without pinning a pressure value.
 //  * level 0 is matrix-free: its stencil comes from the per-cell matrix code.
+#include <algorithm>
 #include <cmath>
 #include <cstring>
 #include <type_traits>
@@ -103,91 +104,130 @@ __global__ void k_mg_cover_done(LvDev c, uint8_t* __restrict__ ctype) {
 		if (ctype[v] == 3) ctype[v] = 1;
 }
 
-// fine-level matrix entry A(U, W) for W = U + off, off in [-1,1]^3;
-// level 0 from the code (7-point), coarse levels from the symmetric storage
+// the fine operator: level 0 from the code (7-point), coarse levels from the
+// symmetric storage
 struct FineOp {
 	const uint8_t* code;  // level 0 if non-null
 	const float* A;       // coarse storage otherwise
 	const uint8_t* type;
 	LvDev f;
-	int S, C;  // stencil size and centre index (14/13 in 3D, 5/4 in 2D)
-	int is3d;
 };
-__device__ inline float fine_entry(const FineOp& F, long long u, long long w, int dx, int dy, int dz) {
-	if (F.code) {
-		const int nz = (dx != 0) + (dy != 0) + (dz != 0);
-		if (nz == 0) return l0_diag(F.code[u]);
-		if (nz > 1) return 0.f;
-		if (dx == 1) return (F.code[u] & 8) ? -1.f : 0.f;
-		if (dx == -1) return (F.code[w] & 8) ? -1.f : 0.f;
-		if (dy == 1) return (F.code[u] & 16) ? -1.f : 0.f;
-		if (dy == -1) return (F.code[w] & 16) ? -1.f : 0.f;
-		if (dz == 1) return (F.code[u] & 32) ? -1.f : 0.f;
-		return (F.code[w] & 32) ? -1.f : 0.f;
-	}
-	const int s = F.is3d ? (dx + 1) + 3 * (dy + 1) + 9 * (dz + 1) : (dx + 1) + 3 * (dy + 1);
-	if (s >= F.C) return F.A[(long long)(s - F.C) * F.f.n + u];
-	return F.A[(long long)(F.C - s) * F.f.n + w];
-}
-__device__ inline bool fine_active(const FineOp& F, long long u) {
-	return F.code ? l0_active(F.code[u]) : F.type[u] != 0;
-}
 
-// Galerkin operator A_l = R A_{l-1} I at coarse vertex V (upper half), plus a
-// diagonal scale proxy used to drop vertices whose diagonal cancels
-__global__ void k_mg_galerkin(FineOp F, LvDev c, const uint8_t* __restrict__ ctype, float* __restrict__ Ac,
-                              float* __restrict__ proxyOut) {
-	for (long long v = blockIdx.x * (long long)blockDim.x + threadIdx.x; v < c.n;
-	     v += (long long)gridDim.x * blockDim.x) {
-		const int S = F.S, C = F.C;
-		if (!ctype[v]) {
-			for (int q = 0; q < S; q++) Ac[(long long)q * c.n + v] = 0.f;
-			proxyOut[v] = 0.f;
+// Interpolation along one axis seen from a fine vertex at offset dd (-1, 0,
+// 1) of coarse vertex V's injection point: the three couplings (lower, own,
+// upper) of the fine row onto the coarse offsets -1, 0, 1 of V.  A fine
+// vertex of even coordinate has one parent (weight 1), of odd coordinate two
+// (weight 1/2 each).
+struct AxisW {
+	double l0, c0, l1, c1, u1, c2, u2;
+	__device__ explicit AxisW(int dd)
+	    : l0(dd < 0 ? 1.0 : (dd == 0 ? 0.5 : 0.0)),
+	      c0(dd < 0 ? 0.5 : 0.0),
+	      l1(dd < 0 ? 0.0 : (dd == 0 ? 0.5 : 1.0)),
+	      c1(dd == 0 ? 1.0 : 0.5),
+	      u1(dd < 0 ? 1.0 : (dd == 0 ? 0.5 : 0.0)),
+	      c2(dd > 0 ? 0.5 : 0.0),
+	      u2(dd < 0 ? 0.0 : (dd == 0 ? 0.5 : 1.0)) {}
+	__device__ void fold(double& l, double& c, double& u) const {
+		const double a = l0 * l + c0 * c, b = l1 * l + c1 * c + u1 * u, e = c2 * c + u2 * u;
+		l = a;
+		c = b;
+		u = e;
+	}
+};
+
+// Galerkin operator A_l = R A_{l-1} I (upper half of the stencil), plus a
+// diagonal scale proxy used to drop vertices whose diagonal cancels.  A group
+// of 32 (2D: 16) lanes builds one coarse vertex: lane q < 27 (9) takes the
+// q-th fine vertex of its restriction support, loads that row, folds it onto
+// the 27 (9) coarse offsets axis by axis (three 3x3 products instead of up to
+// 8 parents for each of 27 couplings), and the group adds the lanes' rows in
+// lane order through LDS.  Bound by the loads of the fine rows (each row is
+// read by the up to 8 vertices it contributes to, from L2).  A thread that
+// built a whole vertex by itself ran its up to 27 x 27 x 8 terms one after
+// another: 95x70x83, all levels, 4610 -> 59 us.  The weights are powers of
+// two and the level-0 couplings small integers, so the double sums are exact
+// on the first levels whatever their order.
+template <bool IS3D, bool CODE>
+__global__ void __launch_bounds__(256) k_mg_galerkin(FineOp F, LvDev c, const uint8_t* __restrict__ ctype,
+                                                     float* __restrict__ Ac, float* __restrict__ proxyOut) {
+	constexpr int NL = IS3D ? 27 : 9, GL = IS3D ? 32 : 16, NG = 256 / GL, S = IS3D ? 14 : 5, C = S - 1;
+	__shared__ double sh[S + 1][NG][NL];
+	const int g = threadIdx.x / GL, q = threadIdx.x % GL;
+	const LvDev& f = F.f;
+	const long long v = (long long)blockIdx.x * NG + g;
+	const bool inv = v < c.n;
+	const unsigned vu = inv ? (unsigned)v : 0u, row = fastdiv(vu, c.fdx), vk = fastdiv(row, c.fdy);
+	const int vi = (int)(vu - row * (unsigned)c.nx), vj = (int)(row - vk * (unsigned)c.ny);
+	const bool act = inv && ctype[vu] != 0;
+	if (q < NL) {
+		const int dx = q % 3 - 1, dy = (q / 3) % 3 - 1, dz = IS3D ? q / 9 - 1 : 0;
+		const int ux = 2 * vi + dx, uy = 2 * vj + dy, uz = IS3D ? 2 * (int)vk + dz : 0;
+		const bool in = act && ux >= 0 && uy >= 0 && uz >= 0 && ux < f.nx && uy < f.ny && uz < f.nz;
+		const long long u = in ? ux + f.sy * uy + f.sz * uz : 0;
+		const bool ua = in && fine_active(F.code, F.type, u);
+		const double rw = (dx ? 0.5 : 1.0) * (dy ? 0.5 : 1.0) * (dz ? 0.5 : 1.0);
+		// couplings of the fine row, 0 towards inactive or outside vertices
+		double a[NL];
+#pragma unroll
+		for (int s = 0; s < NL; s++) a[s] = 0.0;
+		if (ua) {
+#pragma unroll
+			for (int s = 0; s < NL; s++) {
+				const int ex = s % 3 - 1, ey = (s / 3) % 3 - 1, ez = IS3D ? s / 9 - 1 : 0;
+				if (CODE && (ex != 0) + (ey != 0) + (ez != 0) > 1) continue;
+				const int wx = ux + ex, wy = uy + ey, wz = uz + ez;
+				const bool win = wx >= 0 && wy >= 0 && wz >= 0 && wx < f.nx && wy < f.ny && wz < f.nz;
+				const long long w = win ? u + ex + f.sy * ey + f.sz * ez : u;
+				float val;
+				bool wa;
+				if (CODE) {
+					const uint8_t cu = F.code[u], cw = F.code[w];
+					wa = l0_active(cw);
+					const int bit = ex ? 8 : (ey ? 16 : 32);
+					if (s == C) val = l0_diag(cu);
+					else val = (((s > C) ? cu : cw) & bit) ? -1.f : 0.f;
+				} else {
+					wa = F.type[w] != 0;
+					val = s >= C ? F.A[(long long)(s - C) * f.n + u] : F.A[(long long)(C - s) * f.n + w];
+				}
+				a[s] = win && wa ? (double)val : 0.0;
+			}
+		}
+		const double proxy = rw * fabs(a[C]) * rw;
+		const AxisW wx(dx), wy(dy), wz(dz);
+#pragma unroll
+		for (int s = 0; s < NL; s += 3) wx.fold(a[s], a[s + 1], a[s + 2]);
+#pragma unroll
+		for (int s = 0; s < NL; s += 9)
+#pragma unroll
+			for (int e = 0; e < 3; e++) wy.fold(a[s + e], a[s + 3 + e], a[s + 6 + e]);
+		if constexpr (IS3D) {
+#pragma unroll
+			for (int e = 0; e < 9; e++) wz.fold(a[e], a[9 + e], a[18 + e]);
+		}
+#pragma unroll
+		for (int s = 0; s < S; s++) sh[s][g][q] = rw * a[C + s];
+		sh[S][g][q] = proxy;
+	}
+	__syncthreads();
+	for (int t = threadIdx.x; t < (S + 1) * NG; t += 256) {
+		const int o = t / NG, h = t % NG;
+		const long long vv = (long long)blockIdx.x * NG + h;
+		if (vv >= c.n) continue;
+		double sum = 0.0;
+		for (int e = 0; e < NL; e++) sum += sh[o][h][e];
+		bool ok = ctype[vv] != 0;
+		if (o == S) {
+			proxyOut[vv] = ok ? (float)sum : 0.f;
 			continue;
 		}
-		const int vi = (int)(v % c.nx), vj = (int)((v / c.nx) % c.ny), vk = (int)(v / c.sz);
-		double acc[14];
-		for (int q = 0; q < 14; q++) acc[q] = 0.0;
-		double proxy = 0.0;
-		const LvDev f = F.f;
-		const int uk0 = F.is3d ? max(0, 2 * vk - 1) : 0, uk1 = F.is3d ? min(f.nz - 1, 2 * vk + 1) : 0;
-		for (int uz = uk0; uz <= uk1; uz++)
-			for (int uy = max(0, 2 * vj - 1); uy <= min(f.ny - 1, 2 * vj + 1); uy++)
-				for (int ux = max(0, 2 * vi - 1); ux <= min(f.nx - 1, 2 * vi + 1); ux++) {
-					const long long u = ux + f.sy * uy + f.sz * uz;
-					if (!fine_active(F, u)) continue;
-					const double rw = 1.0 / (double)(1 << oddc(ux, uy, uz));
-					const int dz0 = F.is3d ? -1 : 0, dz1 = F.is3d ? 1 : 0;
-					for (int dz = dz0; dz <= dz1; dz++)
-						for (int dy = -1; dy <= 1; dy++)
-							for (int dx = -1; dx <= 1; dx++) {
-								if (F.code && ((dx != 0) + (dy != 0) + (dz != 0)) > 1) continue;
-								const int wx = ux + dx, wy = uy + dy, wz = uz + dz;
-								if (wx < 0 || wy < 0 || wz < 0 || wx >= f.nx || wy >= f.ny || wz >= f.nz) continue;
-								const long long w = wx + f.sy * wy + f.sz * wz;
-								if (!fine_active(F, w)) continue;
-								const float a = fine_entry(F, u, w, dx, dy, dz);
-								if (a == 0.f) continue;
-								const double iw = 1.0 / (double)(1 << oddc(wx, wy, wz));
-								if (dx == 0 && dy == 0 && dz == 0) proxy += rw * fabs((double)a) * iw;
-								// parents N of W: [W/2, (W+1)/2]
-								for (int nz = wz / 2; nz <= (wz + 1) / 2; nz++)
-									for (int ny = wy / 2; ny <= (wy + 1) / 2; ny++)
-										for (int nx = wx / 2; nx <= (wx + 1) / 2; nx++) {
-											const int ox = nx - vi, oy = ny - vj, oz = nz - vk;
-											if (ox < -1 || ox > 1 || oy < -1 || oy > 1 || oz < -1 || oz > 1) continue;
-											const int s = F.is3d ? (ox + 1) + 3 * (oy + 1) + 9 * (oz + 1)
-											                     : (ox + 1) + 3 * (oy + 1);
-											if (s < C) continue;
-											if (nx >= c.nx || ny >= c.ny || nz >= c.nz) continue;
-											const long long nn = nx + c.sy * ny + c.sz * nz;
-											if (!ctype[nn]) continue;
-											acc[s - C] += rw * (double)a * iw;
-										}
-							}
-				}
-		for (int q = 0; q < S; q++) Ac[(long long)q * c.n + v] = (float)acc[q];
-		proxyOut[v] = (float)proxy;
+		const unsigned r2 = fastdiv((unsigned)vv, c.fdx), k2 = fastdiv(r2, c.fdy);
+		const int s = C + o, nx = (int)((unsigned)vv - r2 * (unsigned)c.nx) + s % 3 - 1;
+		const int ny = (int)(r2 - k2 * (unsigned)c.ny) + (s / 3) % 3 - 1, nz = (int)k2 + (IS3D ? s / 9 - 1 : 0);
+		ok = ok && nx >= 0 && ny >= 0 && nz >= 0 && nx < c.nx && ny < c.ny && nz < c.nz &&
+		     ctype[nx + c.sy * ny + c.sz * nz] != 0;
+		Ac[(long long)o * c.n + vv] = ok ? (float)sum : 0.f;
 	}
 }
 
@@ -224,25 +264,61 @@ __device__ inline bool mg_full_stencil(const LvDev& c, int is3d, int S, const fl
 	return ok;
 }
 
-// full stencils of a few sample vertices (for picking the canonical one)
-__global__ void k_mg_sample(LvDev c, int is3d, int S, const float* __restrict__ A, const uint8_t* __restrict__ type,
-                            const long long* __restrict__ samples, int ns, float* __restrict__ out,
-                            int* __restrict__ ok) {
-	const int t = blockIdx.x * blockDim.x + threadIdx.x;
-	if (t >= ns) return;
-	const long long v = samples[t];
-	float st[27];
-	for (int s = 0; s < 27; s++) st[s] = 0.f;
-	const bool good = type[v] && mg_full_stencil(c, is3d, S, A, type, v, st);
-	for (int s = 0; s < 27; s++) out[27 * t + s] = st[s];
-	ok[t] = good ? 1 : 0;
+// Pick the most frequent full stencil among a lattice of up to 64 sample
+// vertices whose neighbours are all active (the first of equally frequent
+// ones).  One block per level: a thread per stencil entry of a sample loads
+// it, then a thread per pair of samples compares them.
+struct CanonSlot {
+	Canon cn;
+	int has;
+};
+__global__ void __launch_bounds__(1024) k_mg_pick(LvDev c, int is3d, const float* __restrict__ A,
+                                                  const uint8_t* __restrict__ type, CanonSlot* __restrict__ out) {
+	__shared__ unsigned st[64][27];
+	__shared__ int bad[64], cnt[64];
+	const int t = threadIdx.x, per = is3d ? 4 : 8, ns = is3d ? 27 : 9, C = is3d ? 13 : 4;
+	if (t < 64) bad[t] = cnt[t] = 0;
+	__syncthreads();
+	for (int e = t; e < 64 * 27; e += 1024) {
+		const int o = e / 27, s = e % 27;
+		const int a = is3d ? o / (per * per) : o / per, b = is3d ? (o / per) % per : o % per, q = is3d ? o % per : 0;
+		const int i = (int)((c.nx - 2) * (a + 0.5) / per) + 1, j = (int)((c.ny - 2) * (b + 0.5) / per) + 1;
+		const int k = is3d ? (int)((c.nz - 2) * (q + 0.5) / per) + 1 : 0;
+		unsigned val = 0;
+		bool ok = i >= 1 && j >= 1 && i < c.nx - 1 && j < c.ny - 1 && (!is3d || (k >= 1 && k < c.nz - 1));
+		if (ok && s < ns) {
+			// (an inner vertex: every neighbour is inside)
+			const long long v = i + c.sy * j + c.sz * k;
+			const long long w = v + s % 3 - 1 + c.sy * ((s / 3) % 3 - 1) + (is3d ? c.sz * (s / 9 - 1) : 0);
+			ok = type[w] != 0;
+			val = __float_as_uint(s >= C ? A[(long long)(s - C) * c.n + v] : A[(long long)(C - s) * c.n + w]);
+		}
+		st[o][s] = val;
+		if (!ok) bad[o] = 1;
+	}
+	__syncthreads();
+	for (int e = t; e < 64 * 64; e += 1024) {
+		const int o = e >> 6, p = e & 63;
+		bool same = !bad[o] && !bad[p];
+		for (int s = 0; s < ns && same; s++) same = st[o][s] == st[p][s];
+		if (same) atomicAdd(&cnt[o], 1);
+	}
+	__syncthreads();
+	if (t >= 64) return;
+	// the largest count, of equal ones the lowest sample
+	int key = cnt[t] * 64 + (63 - t);
+	for (int o = 32; o > 0; o >>= 1) key = max(key, __shfl_xor(key, o, 64));
+	const int best = 63 - (key & 63), has = key >= 64 ? 1 : 0;
+	if (t == 0) out->has = has;
+	if (t < 27) out->cn.a[t] = has ? __uint_as_float(st[best][t]) : 0.f;
 }
 
-// type 2 = active, all neighbours active, stencil bitwise equal to cn.  Only
-// nonzero type values are ever written, so concurrent readers testing
-// type != 0 are unaffected.
+// type 2 = active, all neighbours active, stencil bitwise equal to the
+// picked one.  Only nonzero type values are ever written, so concurrent
+// readers testing type != 0 are unaffected.
 __global__ void k_mg_classify(LvDev c, int is3d, int S, const float* __restrict__ A, uint8_t* __restrict__ type,
-                              Canon cn) {
+                              const CanonSlot* __restrict__ pick) {
+	if (!pick->has) return;
 	const int ns = is3d ? 27 : 9;
 	for (long long v = blockIdx.x * (long long)blockDim.x + threadIdx.x; v < c.n;
 	     v += (long long)gridDim.x * blockDim.x) {
@@ -250,9 +326,171 @@ __global__ void k_mg_classify(LvDev c, int is3d, int S, const float* __restrict_
 		float st[27];
 		if (!mg_full_stencil(c, is3d, S, A, type, v, st)) continue;
 		bool same = true;
-		for (int s = 0; s < ns; s++) same = same && (__float_as_uint(st[s]) == __float_as_uint(cn.a[s]));
+		for (int s = 0; s < ns; s++) same = same && (__float_as_uint(st[s]) == __float_as_uint(pick->cn.a[s]));
 		if (same) type[v] = 2;
 	}
+}
+
+// ---------------------------------------------------------------------------
+// dense generalised inverse of the coarsest operator (FP64, on the device)
+// ---------------------------------------------------------------------------
+__global__ void k_fill_d(double* p, long long n) {
+	for (long long i = blockIdx.x * (long long)blockDim.x + threadIdx.x; i < n; i += (long long)gridDim.x * blockDim.x)
+		p[i] = 0.0;
+}
+__global__ void k_fill_f(float* p, long long n) {
+	for (long long i = blockIdx.x * (long long)blockDim.x + threadIdx.x; i < n; i += (long long)gridDim.x * blockDim.x)
+		p[i] = 0.f;
+}
+// M[a][b] = A(idx[a], idx[b]) (M cleared before), one thread per row and
+// stencil entry; code: the level-0 operator of a single-level hierarchy
+__global__ void __launch_bounds__(256) k_dense_assemble(LvDev c, int is3d, int S, int m, const int* __restrict__ idx,
+                                                        const int* __restrict__ pos, const float* __restrict__ A,
+                                                        const uint8_t* __restrict__ code, double* __restrict__ M,
+                                                        double* __restrict__ diag) {
+	const int t = blockIdx.x * 256 + threadIdx.x, a = t / 27, s = t % 27, C = S - 1;
+	if (a >= m || (!is3d && s >= 9)) return;
+	const int dx = s % 3 - 1, dy = (s / 3) % 3 - 1, dz = is3d ? s / 9 - 1 : 0;
+	const long long v = idx[a];
+	const int i = (int)(v % c.nx) + dx, j = (int)((v / c.nx) % c.ny) + dy, k = (int)(v / c.sz) + dz;
+	if (i < 0 || j < 0 || k < 0 || i >= c.nx || j >= c.ny || k >= c.nz) return;
+	const long long w = i + c.sy * j + c.sz * k;
+	if (pos[w] < 0) return;
+	float val;
+	if (code) {
+		const int nzc = (dx != 0) + (dy != 0) + (dz != 0);
+		if (nzc > 1) return;
+		const int bit = dx ? 8 : (dy ? 16 : 32);
+		val = s == C ? l0_diag(code[v]) : (((s > C ? code[v] : code[w]) & bit) ? -1.f : 0.f);
+	} else {
+		val = s >= C ? A[(long long)(s - C) * c.n + v] : A[(long long)(C - s) * c.n + w];
+	}
+	M[(long long)a * m + pos[w]] = (double)val;
+	if (s == C) diag[a] = (double)val;
+}
+
+// The inverse by sweeping blocks of kSweep pivots (the symmetric Gauss-Jordan
+// step, Goodnight 1979, in blocks): with D the swept pivot block (-its
+// inverse), P the matrix columns of the block and W = -P D,
+//   M_ij -= W_i P_j^T,  M_iK = W_i,  M_Kj = W_j^T,  M_KK = D;
+// after all pivots M is minus the inverse.  Pivots that are dropped (pinned,
+// or not positive beyond round-off) are not swept: their rows and columns
+// become 0.  Two launches per block: the panel (every workgroup sweeps the
+// pivot block for itself, then forms its rows of W) and the update.
+// On the host the same inverse (unblocked Cholesky) took about 3 ms at 294
+// and 75 ms at 729 unknowns; here 0.2 and 0.6 ms (a panel 19 us, an update
+// 6.5 us; blocks of 16 pivots: 8.4 and 4.9 us, twice as many).
+constexpr int kSweep = 32, kDTile = 32;
+__device__ inline double lane_d(double v, int lane) {
+	const unsigned long long u = __builtin_bit_cast(unsigned long long, v);
+	const unsigned lo = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)u, lane);
+	const unsigned hi = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)(u >> 32), lane);
+	return __builtin_bit_cast(double, ((unsigned long long)hi << 32) | lo);
+}
+__global__ void __launch_bounds__(256) k_sweep_panel(int m, int k0, const double* __restrict__ M,
+                                                     const double* __restrict__ diag,
+                                                     const int* __restrict__ pinned, double* __restrict__ D,
+                                                     double* __restrict__ W, double* __restrict__ Pc) {
+	__shared__ double d[kSweep][kSweep + 1];
+	__shared__ double p[kDTile][kSweep + 1];
+	__shared__ int drop[kSweep];
+	const int t = threadIdx.x, nk = min(kSweep, m - k0), i0 = (int)blockIdx.x * kDTile;
+	if (t < 64) {
+		// the first wavefront sweeps the pivot block: lane r holds row r, the
+		// pivot row comes by readlane (in LDS with two barriers per step a panel took
+		// 24 us instead of 19)
+		const int r = t & (kSweep - 1);
+		double a[kSweep];
+#pragma unroll
+		for (int q = 0; q < kSweep; q++) a[q] = r < nk && q < nk ? M[(long long)(k0 + r) * m + k0 + q] : 0.0;
+		const double og = r < nk ? diag[k0 + r] : 0.0;
+		const int pn = r < nk ? pinned[k0 + r] : 1;
+		unsigned dropped = 0;
+#pragma unroll
+		for (int k = 0; k < kSweep; k++) {
+			const double piv = lane_d(a[k], k), orig = lane_d(og, k);
+			if (__builtin_amdgcn_readlane(pn, k) || !(piv > 1e-10 * (orig > 0 ? orig : 1.0))) {
+				dropped |= 1u << k;
+				continue;
+			}
+			const double rp = 1.0 / piv;
+			const bool own = r == k;
+			const double cf = own ? -rp : a[k] * rp;
+#pragma unroll
+			for (int q = 0; q < kSweep; q++) {
+				if (q == k) continue;
+				a[q] = fma(-cf, lane_d(a[q], k), own ? 0.0 : a[q]);
+			}
+			a[k] = cf;
+		}
+		if (t < kSweep) {
+			drop[t] = (dropped >> t) & 1;
+#pragma unroll
+			for (int q = 0; q < kSweep; q++) d[t][q] = ((dropped >> t) | (dropped >> q)) & 1 ? 0.0 : a[q];
+		}
+	} else {
+		for (int e = t - 64; e < kDTile * kSweep; e += 192) {
+			const int r = e / kSweep, q = e % kSweep;
+			p[r][q] = i0 + r < m && q < nk ? M[(long long)(i0 + r) * m + k0 + q] : 0.0;
+		}
+	}
+	__syncthreads();
+	if (blockIdx.x == 0)
+		for (int e = t; e < kSweep * kSweep; e += 256) D[e] = d[e / kSweep][e % kSweep];
+	for (int e = t; e < kDTile * kSweep; e += 256) {
+		const int r = e / kSweep, q = e % kSweep;
+		if (i0 + r >= m) continue;
+		double w = 0.0;
+#pragma unroll
+		for (int l = 0; l < kSweep; l++) w -= p[r][l] * d[l][q];
+		W[(long long)(i0 + r) * kSweep + q] = w;
+		Pc[(long long)(i0 + r) * kSweep + q] = drop[q] ? 0.0 : p[r][q];
+	}
+}
+// last: the matrix is minus the result then
+__global__ void __launch_bounds__(256) k_sweep_update(int m, int k0, double* __restrict__ M,
+                                                      const double* __restrict__ D, const double* __restrict__ W,
+                                                      const double* __restrict__ Pc, int last) {
+	__shared__ double w[kDTile][kSweep + 1];
+	__shared__ double p[kDTile][kSweep + 1];
+	const int t = threadIdx.x, i0 = (int)blockIdx.y * kDTile, j0 = (int)blockIdx.x * kDTile;
+	for (int e = t; e < kDTile * kSweep; e += 256) {
+		const int r = e / kSweep, q = e % kSweep;
+		w[r][q] = i0 + r < m ? W[(long long)(i0 + r) * kSweep + q] : 0.0;
+		p[r][q] = j0 + r < m ? Pc[(long long)(j0 + r) * kSweep + q] : 0.0;
+	}
+	__syncthreads();
+	// rows ty + 16 u, columns tx + 16 q of the tile
+	constexpr int NU = kDTile / 16;
+	const int tx = t & 15, ty = t >> 4;
+	double acc[NU][NU] = {};
+#pragma unroll 4
+	for (int l = 0; l < kSweep; l++) {
+		double a[NU], b[NU];
+#pragma unroll
+		for (int u = 0; u < NU; u++) {
+			a[u] = w[ty + 16 * u][l];
+			b[u] = p[tx + 16 * u][l];
+		}
+#pragma unroll
+		for (int u = 0; u < NU; u++)
+#pragma unroll
+			for (int q = 0; q < NU; q++) acc[u][q] += a[u] * b[q];
+	}
+#pragma unroll
+	for (int u = 0; u < NU; u++)
+#pragma unroll
+		for (int q = 0; q < NU; q++) {
+			const int i = i0 + ty + 16 * u, j = j0 + tx + 16 * q;
+			if (i >= m || j >= m) continue;
+			const bool ik = i >= k0 && i < k0 + kSweep, jk = j >= k0 && j < k0 + kSweep;
+			double v;
+			if (ik && jk) v = D[(i - k0) * kSweep + j - k0];
+			else if (jk) v = w[ty + 16 * u][j - k0];
+			else if (ik) v = W[(long long)j * kSweep + i - k0];
+			else v = M[(long long)i * m + j] - acc[u][q];
+			M[(long long)i * m + j] = last ? -v : v;
+		}
 }
 
 // ---------------------------------------------------------------------------
@@ -1314,14 +1552,8 @@ __device__ __forceinline__ void body_coarsest(const CoarsestP& P, long long blk,
 // host
 // ---------------------------------------------------------------------------
 MgHierarchy::~MgHierarchy() {
-	for (void* p : allocs) (void)hipFree(p);
-}
-
-void* MgHierarchy::alloc(size_t bytes) {
-	void* p = nullptr;
-	MFX_HIP(hipMalloc(&p, bytes < 16 ? 16 : bytes));
-	allocs.push_back(p);
-	return p;
+	if (arena) (void)hipFree(arena);
+	if (hbuf) (void)hipHostFree(hbuf);
 }
 
 static unsigned nblk(long long n) {
@@ -1331,8 +1563,12 @@ static unsigned nblk(long long n) {
 	return (unsigned)b;
 }
 
-void MgHierarchy::build(Scene* s, const uint8_t* code, int precision) {
-	prec = precision;
+// Levels and their memory: one device block and one pinned block, laid out
+// once.  A hierarchy rebuilt for another matrix of the same grid (PcMGDynamic
+// in every solve, PcMIC when the flags changed) works in the same memory:
+// allocating its 30 to 40 arrays and freeing them again took about 1 ms a
+// solve.
+void MgHierarchy::layout(Scene* s) {
 	const Dims& d = s->d;
 	is3d = d.is3d != 0;
 	// the z-marching level-0 kernels keep in-plane offsets in 32 bits
@@ -1365,134 +1601,151 @@ void MgHierarchy::build(Scene* s, const uint8_t* code, int precision) {
 		n = c.n;
 		L.push_back(c);
 	}
-	L[0].r = (float*)alloc(sizeof(float) * (size_t)d.n);
-	L[0].x = (float*)alloc(sizeof(float) * (size_t)d.n);
-	for (size_t l = 1; l < L.size(); l++) {
+	const int nl = (int)L.size();
+	const size_t ncMax = (size_t)L[nl - 1].n;
+	// two passes over the same list: sizes, then addresses
+	size_t total = 0;
+	for (int pass = 0; pass < 2; pass++) {
+		size_t off = 0;
+		auto take = [&](auto*& p, size_t count) {
+			using T = std::remove_reference_t<decltype(*p)>;
+			off = (off + 255) & ~(size_t)255;
+			if (pass) p = (T*)((uint8_t*)arena + off);
+			off += sizeof(T) * count;
+		};
+		// vectors that start at 0 (inactive vertices keep it): one run
+		float* z0 = nullptr;
+		take(z0, 0);
+		const size_t zoff = off;
+		for (int l = 1; l < nl; l++) {
+			take(L[l].x, (size_t)L[l].n);
+			take(L[l].xp, (size_t)L[l].n);
+		}
+		if (pass) {
+			zero = (float*)((uint8_t*)arena + zoff);
+			nzero = (long long)((off - zoff) / sizeof(float));
+		}
+		// what the host reads: the picked stencils, the coarsest operator
+		CanonSlot* cs = nullptr;
+		take(cs, (size_t)nl);
+		picks = cs;
+		if (nl > 1) {
+			take(L[nl - 1].A, ncMax * (size_t)S);
+			take(L[nl - 1].type, ncMax);
+		}
+		if (pass) readBytes = (size_t)((uint8_t*)arena + off - (uint8_t*)picks);
+		take(L[0].r, (size_t)d.n);
+		take(L[0].x, (size_t)d.n);
+		for (int l = 1; l < nl; l++) {
+			MgLevel& c = L[l];
+			if (l < nl - 1) {
+				take(c.A, (size_t)(c.n * S));
+				take(c.type, (size_t)c.n);
+				if (prec == 1) take(c.Ah, (size_t)(c.n * S));
+			}
+			take(c.b, (size_t)c.n);
+			take(c.r, (size_t)c.n);
+		}
+		take(G, ncMax * ncMax);
+		take(sweepD, (size_t)kSweep * kSweep);
+		take(sweepW, ncMax * kSweep);
+		take(sweepP, ncMax * kSweep);
+		take(cdiag, ncMax);
+		// what the host writes
+		take(cidx, ncMax);
+		take(cpos, ncMax);
+		take(cpin, ncMax);
+		if (!pass) {
+			total = off;
+			MFX_HIP(hipMalloc(&arena, total));
+		}
+	}
+	hostBytes = std::max(readBytes, ncMax) + 256 + ((uint8_t*)(cpin + ncMax) - (uint8_t*)cidx);
+	MFX_HIP(hipHostMalloc(&hbuf, hostBytes, hipHostMallocDefault));
+}
+
+void MgHierarchy::build(Scene* s, const uint8_t* code, int precision) {
+	ready = false;
+	if (!arena || !hbuf || prec != precision) {
+		if (arena) MFX_HIP(hipFree(arena));
+		if (hbuf) MFX_HIP(hipHostFree(hbuf));
+		arena = hbuf = nullptr;
+		prec = precision;
+		layout(s);
+	}
+	hipStream_t q = s->stream;
+	const int nl = (int)L.size();
+	if (nzero) hipLaunchKernelGGL(k_fill_f, dim3(nblk(nzero)), dim3(256), 0, q, zero, nzero);
+	for (int l = 1; l < nl; l++) {
 		MgLevel& c = L[l];
-		c.A = (float*)alloc(sizeof(float) * (size_t)(c.n * S));
-		c.x = (float*)alloc(sizeof(float) * (size_t)c.n);
-		c.xp = (float*)alloc(sizeof(float) * (size_t)c.n);
-		c.b = (float*)alloc(sizeof(float) * (size_t)c.n);
-		c.r = (float*)alloc(sizeof(float) * (size_t)c.n);
-		c.type = (uint8_t*)alloc((size_t)c.n);
-		MFX_HIP(hipMemsetAsync(c.x, 0, sizeof(float) * (size_t)c.n, s->stream));
 		const MgLevel& f = L[l - 1];
-		hipLaunchKernelGGL(k_mg_activate, dim3(nblk(c.n)), dim3(256), 0, s->stream, lvdev(c), lvdev(f), (int)is3d,
-		                   l == 1 ? code : (const uint8_t*)nullptr, f.type, c.type);
-		hipLaunchKernelGGL(k_mg_cover, dim3(nblk(f.n)), dim3(256), 0, s->stream, lvdev(c), lvdev(f), (int)is3d,
-		                   l == 1 ? code : (const uint8_t*)nullptr, f.type, c.type);
-		hipLaunchKernelGGL(k_mg_cover_done, dim3(nblk(c.n)), dim3(256), 0, s->stream, lvdev(c), c.type);
-		FineOp F;
-		F.code = l == 1 ? code : nullptr;
-		F.A = l == 1 ? nullptr : f.A;
-		F.type = f.type;
-		F.f = lvdev(f);
-		F.S = S;
-		F.C = S - 1;
-		F.is3d = is3d;
-		hipLaunchKernelGGL(k_mg_galerkin, dim3(nblk(c.n)), dim3(256), 0, s->stream, F, lvdev(c),
-		                   (const uint8_t*)c.type, c.A, c.r);
-		hipLaunchKernelGGL(k_mg_drop, dim3(nblk(c.n)), dim3(256), 0, s->stream, lvdev(c), c.type, (const float*)c.A,
+		const uint8_t* fc = l == 1 ? code : nullptr;
+		hipLaunchKernelGGL(k_mg_activate, dim3(nblk(c.n)), dim3(256), 0, q, lvdev(c), lvdev(f), (int)is3d, fc, f.type,
+		                   c.type);
+		hipLaunchKernelGGL(k_mg_cover, dim3(nblk(f.n)), dim3(256), 0, q, lvdev(c), lvdev(f), (int)is3d, fc, f.type,
+		                   c.type);
+		hipLaunchKernelGGL(k_mg_cover_done, dim3(nblk(c.n)), dim3(256), 0, q, lvdev(c), c.type);
+		const FineOp F{fc, f.A, f.type, lvdev(f)};
+		const dim3 gb((unsigned)((c.n + (is3d ? 7 : 15)) / (is3d ? 8 : 16)));
+		auto* kern = is3d ? (fc ? k_mg_galerkin<true, true> : k_mg_galerkin<true, false>)
+		                  : (fc ? k_mg_galerkin<false, true> : k_mg_galerkin<false, false>);
+		hipLaunchKernelGGL(kern, gb, dim3(256), 0, q, F, lvdev(c), (const uint8_t*)c.type, c.A, c.r);
+		hipLaunchKernelGGL(k_mg_drop, dim3(nblk(c.n)), dim3(256), 0, q, lvdev(c), c.type, (const float*)c.A,
 		                   (const float*)c.r);
+		// the coarsest level is solved through G; the others get a canonical stencil
+		if (l == nl - 1) break;
+		hipLaunchKernelGGL(k_mg_pick, dim3(1), dim3(1024), 0, q, lvdev(c), (int)is3d, (const float*)c.A,
+		                   (const uint8_t*)c.type, picks + l);
+		hipLaunchKernelGGL(k_mg_classify, dim3(nblk(c.n)), dim3(256), 0, q, lvdev(c), (int)is3d, S, (const float*)c.A,
+		                   c.type, (const CanonSlot*)(picks + l));
 	}
 	build_coarsest(s, code);
-	// the coarsest level is solved through G; the others get a canonical stencil
-	for (int l = 1; l + 1 < (int)L.size(); l++) {
-		classify(s, l);
+	const CanonSlot* hp = (const CanonSlot*)hbuf;
+	for (int l = 1; l + 1 < nl; l++) {
+		MgLevel& c = L[l];
+		c.hasCanon = hp[l].has != 0;
+		c.canon = hp[l].cn;
 		if (prec == 1) {
 			// mixed precision: smoother and residual read BF16 coefficients; the
 			// canonical stencil is rounded the same way so that every coupling
 			// has one value seen from both of its vertices (symmetric V-cycle)
-			MgLevel& c = L[l];
-			c.Ah = (uint16_t*)alloc(sizeof(uint16_t) * (size_t)(c.n * S));
-			hipLaunchKernelGGL(k_to_bf16, dim3(nblk(c.n * S)), dim3(256), 0, s->stream, (const float*)c.A, c.Ah,
-			                   c.n * S);
-			for (int q = 0; q < 27; q++) c.canon.a[q] = from_bf16(to_bf16(c.canon.a[q]));
+			hipLaunchKernelGGL(k_to_bf16, dim3(nblk(c.n * S)), dim3(256), 0, q, (const float*)c.A, c.Ah, c.n * S);
+			for (int e = 0; e < 27; e++) c.canon.a[e] = from_bf16(to_bf16(c.canon.a[e]));
 		}
 	}
+	ready = true;
 }
 
-// Pick the most frequent full stencil among a lattice of sample vertices
-// (all neighbours active) and mark the vertices that share it bitwise.
-void MgHierarchy::classify(Scene* s, int l) {
-	MgLevel& c = L[l];
-	c.hasCanon = false;
-	const int per = is3d ? 4 : 8;
-	std::vector<long long> smp;
-	for (int a = 0; a < per; a++)
-		for (int b = 0; b < per; b++)
-			for (int e = 0; e < (is3d ? per : 1); e++) {
-				const int i = (int)((c.nx - 2) * (a + 0.5) / per) + 1, j = (int)((c.ny - 2) * (b + 0.5) / per) + 1;
-				const int k = is3d ? (int)((c.nz - 2) * (e + 0.5) / per) + 1 : 0;
-				if (i < 1 || j < 1 || i >= c.nx - 1 || j >= c.ny - 1 || (is3d && (k < 1 || k >= c.nz - 1))) continue;
-				smp.push_back(i + c.sy * j + c.sz * k);
-			}
-	const int ns = (int)smp.size();
-	if (ns == 0) return;
-	long long* dsmp = nullptr;
-	float* dout = nullptr;
-	int* dok = nullptr;
-	MFX_HIP(hipMalloc((void**)&dsmp, sizeof(long long) * ns));
-	MFX_HIP(hipMalloc((void**)&dout, sizeof(float) * 27 * ns));
-	MFX_HIP(hipMalloc((void**)&dok, sizeof(int) * ns));
-	MFX_HIP(hipMemcpyAsync(dsmp, smp.data(), sizeof(long long) * ns, hipMemcpyHostToDevice, s->stream));
-	hipLaunchKernelGGL(k_mg_sample, dim3((ns + 63) / 64), dim3(64), 0, s->stream, lvdev(c), (int)is3d, S,
-	                   (const float*)c.A, (const uint8_t*)c.type, (const long long*)dsmp, ns, dout, dok);
-	std::vector<float> out((size_t)27 * ns);
-	std::vector<int> ok(ns);
-	MFX_HIP(hipMemcpyAsync(out.data(), dout, sizeof(float) * 27 * ns, hipMemcpyDeviceToHost, s->stream));
-	MFX_HIP(hipMemcpyAsync(ok.data(), dok, sizeof(int) * ns, hipMemcpyDeviceToHost, s->stream));
-	sync(s);
-	MFX_HIP(hipFree(dsmp));
-	MFX_HIP(hipFree(dout));
-	MFX_HIP(hipFree(dok));
-	int best = -1, bestCount = 0;
-	for (int a = 0; a < ns; a++) {
-		if (!ok[a]) continue;
-		int cnt = 0;
-		for (int b = 0; b < ns; b++)
-			if (ok[b] && !memcmp(&out[27 * (size_t)a], &out[27 * (size_t)b], sizeof(float) * 27)) cnt++;
-		if (cnt > bestCount) {
-			bestCount = cnt;
-			best = a;
-		}
-	}
-	if (best < 0) return;
-	memcpy(c.canon.a, &out[27 * (size_t)best], sizeof(float) * 27);
-	c.hasCanon = true;
-	hipLaunchKernelGGL(k_mg_classify, dim3(nblk(c.n)), dim3(256), 0, s->stream, lvdev(c), (int)is3d, S,
-	                   (const float*)c.A, c.type, c.canon);
-}
-
-// dense generalised inverse of the coarsest operator (host, FP64)
+// Dense generalised inverse of the coarsest operator (FP64).  The host reads
+// the operator once (with the picked stencils, the only wait of a build),
+// numbers its active vertices and finds the singular blocks; the matrix is
+// assembled and inverted on the device.
 void MgHierarchy::build_coarsest(Scene* s, const uint8_t* code0) {
+	hipStream_t q = s->stream;
 	const int lc = (int)L.size() - 1;
 	const MgLevel& c = L[lc];
-	std::vector<uint8_t> type((size_t)c.n), hcode;
-	std::vector<float> A;
-	if (lc == 0) {
-		// single level: the dense operator comes from the level-0 matrix code
-		hcode.resize((size_t)c.n);
-		MFX_HIP(hipMemcpyAsync(hcode.data(), code0, (size_t)c.n, hipMemcpyDeviceToHost, s->stream));
-		sync(s);
-		for (long long v = 0; v < c.n; v++) type[v] = (hcode[v] & 7) ? 1 : 0;
-	} else {
-		MFX_HIP(hipMemcpyAsync(type.data(), c.type, (size_t)c.n, hipMemcpyDeviceToHost, s->stream));
-		A.resize((size_t)(c.n * S));
-		MFX_HIP(hipMemcpyAsync(A.data(), c.A, sizeof(float) * (size_t)(c.n * S), hipMemcpyDeviceToHost, s->stream));
-		sync(s);
+	uint8_t* hb = (uint8_t*)hbuf;
+	if (lc == 0) MFX_HIP(hipMemcpyAsync(hb, code0, (size_t)c.n, hipMemcpyDeviceToHost, q));
+	else MFX_HIP(hipMemcpyAsync(hb, picks, readBytes, hipMemcpyDeviceToHost, q));
+	sync(s);
+	const uint8_t* hcode = hb;
+	const float* A = lc ? (const float*)(hb + ((uint8_t*)c.A - (uint8_t*)picks)) : nullptr;
+	const uint8_t* type = lc ? hb + (c.type - (uint8_t*)picks) : nullptr;
+	// host copies of cidx, cpos, cpin, laid out as on the device
+	uint8_t* hw = hb + ((std::max(readBytes, (size_t)c.n) + 255) & ~(size_t)255);
+	int* idx = (int*)hw;
+	int* pos = (int*)(hw + ((uint8_t*)cpos - (uint8_t*)cidx));
+	int* pin = (int*)(hw + ((uint8_t*)cpin - (uint8_t*)cidx));
+	int m = 0;
+	for (long long v = 0; v < c.n; v++) {
+		const bool act = lc ? type[v] != 0 : (hcode[v] & 7) != 0;
+		pos[v] = act ? m : -1;
+		if (act) idx[m++] = (int)v;
 	}
-	std::vector<int> idx, pos((size_t)c.n, -1);
-	for (long long v = 0; v < c.n; v++)
-		if (type[v]) {
-			pos[v] = (int)idx.size();
-			idx.push_back((int)v);
-		}
-	nc = (int)idx.size();
-	const int m = nc;
-	std::vector<double> M((size_t)m * m, 0.0);
+	nc = m;
 	const int C = S - 1;
-	for (int a = 0; a < m; a++) {
+	// f(b, value) for the stored couplings of row a (b: the column)
+	auto row = [&](int a, auto&& f) {
 		const long long v = idx[a];
 		const int i = (int)(v % c.nx), j = (int)((v / c.nx) % c.ny), k = (int)(v / c.sz);
 		for (int dz = is3d ? -1 : 0; dz <= (is3d ? 1 : 0); dz++)
@@ -1500,114 +1753,69 @@ void MgHierarchy::build_coarsest(Scene* s, const uint8_t* code0) {
 				for (int dx = -1; dx <= 1; dx++) {
 					const int ni = i + dx, nj = j + dy, nk = k + dz;
 					if (ni < 0 || nj < 0 || nk < 0 || ni >= c.nx || nj >= c.ny || nk >= c.nz) continue;
-					const long long nn = ni + c.sy * nj + c.sz * nk;
-					if (pos[nn] < 0) continue;
+					const long long w = ni + c.sy * nj + c.sz * nk;
+					if (pos[w] < 0) continue;
+					const int si = is3d ? (dx + 1) + 3 * (dy + 1) + 9 * (dz + 1) : (dx + 1) + 3 * (dy + 1);
 					double val;
 					if (lc == 0) {
-						const int nzc = (dx != 0) + (dy != 0) + (dz != 0);
-						if (nzc > 1) continue;
-						const uint8_t cv = hcode[v], cn = hcode[nn];
-						if (nzc == 0) val = (cv & 128) ? (double)((float)(cv & 7) * 1e-6f) : (double)(cv & 7);
-						else if (dx == 1) val = (cv & 8) ? -1.0 : 0.0;
-						else if (dx == -1) val = (cn & 8) ? -1.0 : 0.0;
-						else if (dy == 1) val = (cv & 16) ? -1.0 : 0.0;
-						else if (dy == -1) val = (cn & 16) ? -1.0 : 0.0;
-						else if (dz == 1) val = (cv & 32) ? -1.0 : 0.0;
-						else val = (cn & 32) ? -1.0 : 0.0;
+						if ((dx != 0) + (dy != 0) + (dz != 0) > 1) continue;
+						const uint8_t cv = hcode[v], cw = hcode[w];
+						const int bit = dx ? 8 : (dy ? 16 : 32);
+						if (si == C) val = (cv & 128) ? (double)((float)(cv & 7) * 1e-6f) : (double)(cv & 7);
+						else val = ((si > C ? cv : cw) & bit) ? -1.0 : 0.0;
 					} else {
-						const int sidx = is3d ? (dx + 1) + 3 * (dy + 1) + 9 * (dz + 1) : (dx + 1) + 3 * (dy + 1);
-						val = sidx >= C ? A[(size_t)(sidx - C) * c.n + v] : A[(size_t)(C - sidx) * c.n + nn];
+						val = si >= C ? A[(size_t)(si - C) * c.n + v] : A[(size_t)(C - si) * c.n + w];
 					}
-					M[(size_t)a * m + pos[nn]] = val;
+					f(pos[w], val);
 				}
-	}
+	};
 	// Pure-Neumann blocks (fluid pockets enclosed by obstacles, or a closed
 	// domain) are singular; with float coefficients their last pivot is
 	// round-off rather than zero and would put ~1e7-sized entries into G.
 	// Pin one vertex of every connected component whose rows all sum to ~0.
-	std::vector<char> dropped(m, 0);
+	std::fill(pin, pin + m, 0);
 	{
-		std::vector<int> comp(m, -1), stack;
+		std::vector<char> seen((size_t)m, 0);
+		std::vector<int> stack, members;
 		for (int a0 = 0; a0 < m; a0++) {
-			if (comp[a0] >= 0) continue;
-			std::vector<int> members;
-			comp[a0] = a0;
+			if (seen[(size_t)a0]) continue;
+			members.clear();
+			seen[(size_t)a0] = 1;
 			stack.push_back(a0);
+			double maxSum = 0.0, maxDiag = 0.0;
+			int last = a0;
 			while (!stack.empty()) {
 				const int a = stack.back();
 				stack.pop_back();
 				members.push_back(a);
-				for (int b = 0; b < m; b++)
-					if (b != a && comp[b] < 0 && M[(size_t)a * m + b] != 0.0) {
-						comp[b] = a0;
+				last = std::max(last, a);
+				double rs = 0.0;
+				row(a, [&](int b, double val) {
+					rs += val;
+					if (b == a) maxDiag = std::max(maxDiag, val);
+					if (b != a && !seen[(size_t)b] && val != 0.0) {
+						seen[(size_t)b] = 1;
 						stack.push_back(b);
 					}
-			}
-			double maxSum = 0.0, maxDiag = 0.0;
-			for (int a : members) {
-				double rs = 0.0;
-				for (int b : members) rs += M[(size_t)a * m + b];
+				});
 				maxSum = std::max(maxSum, std::fabs(rs));
-				maxDiag = std::max(maxDiag, M[(size_t)a * m + a]);
 			}
-			if (members.size() > 1 && maxSum <= 1e-5 * maxDiag) {
-				int last = members[0];
-				for (int a : members) last = std::max(last, a);
-				dropped[last] = 1;
-			}
+			if (members.size() > 1 && maxSum <= 1e-5 * maxDiag) pin[last] = 1;
 		}
 	}
-	// Cholesky with dropped (pinned or non-positive) pivots
-	std::vector<double> Lm((size_t)m * m, 0.0);
-	for (int jj = 0; jj < m; jj++) {
-		double dval = M[(size_t)jj * m + jj];
-		for (int q = 0; q < jj; q++) dval -= Lm[(size_t)jj * m + q] * Lm[(size_t)jj * m + q];
-		const double orig = M[(size_t)jj * m + jj];
-		if (dropped[jj] || !(dval > 1e-10 * (orig > 0 ? orig : 1.0))) {
-			dropped[jj] = 1;
-			for (int q = 0; q < jj; q++) Lm[(size_t)jj * m + q] = 0.0;
-			Lm[(size_t)jj * m + jj] = 1.0;
-			continue;
-		}
-		const double ljj = std::sqrt(dval);
-		Lm[(size_t)jj * m + jj] = ljj;
-		for (int ii = jj + 1; ii < m; ii++) {
-			double sv = M[(size_t)ii * m + jj];
-			const double* li = &Lm[(size_t)ii * m];
-			const double* lj = &Lm[(size_t)jj * m];
-			for (int q = 0; q < jj; q++) sv -= li[q] * lj[q];
-			Lm[(size_t)ii * m + jj] = sv / ljj;
-		}
+	MFX_HIP(hipMemcpyAsync(cidx, hw, (size_t)((uint8_t*)(cpin + c.n) - (uint8_t*)cidx), hipMemcpyHostToDevice, q));
+	if (!m) return;
+	hipLaunchKernelGGL(k_fill_d, dim3(nblk((long long)m * m)), dim3(256), 0, q, G, (long long)m * m);
+	hipLaunchKernelGGL(k_dense_assemble, dim3((unsigned)((27 * m + 255) / 256)), dim3(256), 0, q, lvdev(c), (int)is3d, S,
+	                   m, (const int*)cidx, (const int*)cpos, (const float*)c.A, lc == 0 ? code0 : (const uint8_t*)nullptr,
+	                   G, cdiag);
+	const unsigned nt = (unsigned)((m + kDTile - 1) / kDTile);
+	for (int k0 = 0; k0 < m; k0 += kSweep) {
+		hipLaunchKernelGGL(k_sweep_panel, dim3(nt), dim3(256), 0, q, m, k0, (const double*)G, (const double*)cdiag,
+		                   (const int*)cpin, sweepD, sweepW, sweepP);
+		hipLaunchKernelGGL(k_sweep_update, dim3(nt, nt), dim3(256), 0, q, m, k0, G, (const double*)sweepD,
+		                   (const double*)sweepW, (const double*)sweepP, k0 + kSweep >= m ? 1 : 0);
 	}
-	for (int jj = 0; jj < m; jj++)
-		if (dropped[jj])
-			for (int ii = jj + 1; ii < m; ii++) Lm[(size_t)ii * m + jj] = 0.0;
-	// Linv (lower), then G = Linv^T Linv
-	std::vector<double> Li((size_t)m * m, 0.0);
-	for (int col = 0; col < m; col++) {
-		Li[(size_t)col * m + col] = 1.0 / Lm[(size_t)col * m + col];
-		for (int row = col + 1; row < m; row++) {
-			double sv = 0.0;
-			for (int q = col; q < row; q++) sv -= Lm[(size_t)row * m + q] * Li[(size_t)q * m + col];
-			Li[(size_t)row * m + col] = sv / Lm[(size_t)row * m + row];
-		}
-	}
-	std::vector<double> Gh((size_t)m * m, 0.0);
-	for (int a = 0; a < m; a++) {
-		if (dropped[a]) continue;
-		for (int b = a; b < m; b++) {
-			if (dropped[b]) continue;
-			double sv = 0.0;
-			for (int q = b; q < m; q++) sv += Li[(size_t)q * m + a] * Li[(size_t)q * m + b];
-			Gh[(size_t)a * m + b] = sv;
-			Gh[(size_t)b * m + a] = sv;
-		}
-	}
-	G = (double*)alloc(sizeof(double) * (size_t)m * m);
-	cidx = (int*)alloc(sizeof(int) * (size_t)m);
-	MFX_HIP(hipMemcpyAsync(G, Gh.data(), sizeof(double) * (size_t)m * m, hipMemcpyHostToDevice, s->stream));
-	MFX_HIP(hipMemcpyAsync(cidx, idx.data(), sizeof(int) * (size_t)m, hipMemcpyHostToDevice, s->stream));
-	sync(s);
 }
 
 // ---------------------------------------------------------------------------

@@ -1620,7 +1620,7 @@ static MgHierarchy* mic_hierarchy(Scene* s, const Grid* flags, const uint8_t* co
 	if (!sameKey) {
 		const uint64_t h = code_hash(s, code);
 		if (!(s->mgMic && s->mgMic->precision() == precision && s->micHash == h)) {
-			s->mgMic.reset(new MgHierarchy());
+			if (!s->mgMic) s->mgMic.reset(new MgHierarchy());
 			s->mgMic->build(s, code, precision);
 		}
 		s->micHash = h;
@@ -1696,7 +1696,6 @@ struct CgRun {
 	int pc = 0, maxIter = 0;
 	bool pcNone = true;
 	MgHierarchy* mg = nullptr;
-	std::unique_ptr<MgHierarchy> mgDyn;
 	float *r = nullptr, *pa = nullptr, *pb = nullptr, *q = nullptr, *z = nullptr;
 	CgState* st = nullptr;  // device
 	int launched = 0;
@@ -1932,9 +1931,9 @@ static void cg_setup(CgRun& R, Scene* s, Grid* flags, float* rhs, float* x, cons
 	if (!R.pcNone) {
 		if (o.preconditioner == MFX_PC_MGDYNAMIC) {
 			s->mgStatic.reset();
-			R.mgDyn.reset(new MgHierarchy());
-			R.mgDyn->build(s, R.code, o.precision);
-			R.mg = R.mgDyn.get();
+			if (!s->mgDyn) s->mgDyn.reset(new MgHierarchy());
+			s->mgDyn->build(s, R.code, o.precision);
+			R.mg = s->mgDyn.get();
 		} else if (o.preconditioner == MFX_PC_MIC) {
 			R.mg = mic_hierarchy(s, flags, R.code, R.fixing, o.precision);
 		} else {
@@ -3318,6 +3317,7 @@ int mfx_release_mg(mfx_scene* s) {
 	for (Scene* sc : all) {
 		sync(sc);
 		sc->mgStatic.reset();
+		sc->mgDyn.reset();
 		sc->mgMic.reset();
 	}
 	API_END
