@@ -236,8 +236,7 @@ int mfx_correct_velocity_bnd(mfx_grid* vel, const mfx_grid* pressure, const mfx_
 /* Batched solvePressure: count independent problems (vel[i], pressure[i],
  * flags[i]), each on its own scene (any mix of sizes, 2D and 3D), solved
  * together.  Every CG/multigrid phase is one launch whose work list holds the
- * tiles of all problems; two iterations are captured in a hipGraph and
- * replayed until every problem has met its stopping rule.  Results equal
+ * tiles of all problems, until every problem has met its stopping rule.  Results equal
  * per-problem mfx_solve_pressure calls up to the order of FP64 partial sums.
  * stats may be NULL or point to count entries.  No counterpart in the
  * reference (its callers loop over solvePressure, plugin/pressure.cpp:480). */

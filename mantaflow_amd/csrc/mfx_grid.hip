@@ -49,7 +49,6 @@ Scene::~Scene() {
 	if (evState) hipEventDestroy(evState);
 	if (arena) hipFree(arena);
 	if (hstage) hipHostFree(hstage);
-	if (bexec) hipGraphExecDestroy(bexec);
 	if (stream) hipStreamDestroy(stream);
 }
 

@@ -99,10 +99,6 @@ struct Scene {
 	size_t arenaCap = 0;
 	void* hstage = nullptr;     // pinned staging of the arena upload
 	size_t hstageCap = 0;
-	// two-iteration graph of the last batch composition led by this scene
-	// that was seen twice in a row (key: launch layout)
-	hipGraphExec_t bexec = nullptr;
-	std::vector<long long> bkey, blastKey;
 	std::unique_ptr<MgHierarchy> mgStatic;
 	std::unique_ptr<MgHierarchy> mgDyn;  // PcMGDynamic: rebuilt by every solve, in the same memory
 	// multigrid hierarchy standing in for PcMIC (the reference's mIC keeps

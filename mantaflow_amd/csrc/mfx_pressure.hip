@@ -1699,6 +1699,7 @@ struct CgRun {
 	float *r = nullptr, *pa = nullptr, *pb = nullptr, *q = nullptr, *z = nullptr;
 	CgState* st = nullptr;  // device
 	int launched = 0;
+	bool owesB = false;  // the last queued iteration's preconditioner part is not queued
 	int scaled = 0;     // scaled Laplace matrix (cgSolveDiffusion, cgSolveWE)
 	float scale = 0.f;
 	// float matrix of the second-order boundaries (fractions / ghost fluid),
@@ -1972,15 +1973,15 @@ static void cg_setup(CgRun& R, Scene* s, Grid* flags, float* rhs, float* x, cons
 
 // r = b - A x with FP64 row sums in place of the recursive residual (plus
 // the update's partials); returns the number of partial-sum slots written
-static int enqueue_replace_residual(CgRun& R) {
+static int enqueue_replace_residual(CgRun& R, hipStream_t q) {
 	Scene* s = R.s;
 	if (R.gA0) {
-		hipLaunchKernelGGL(k_replace_residual_gen, dim3(R.nbG), dim3(256), 0, s->stream, s->d, (const CgState*)R.st,
+		hipLaunchKernelGGL(k_replace_residual_gen, dim3(R.nbG), dim3(256), 0, q, s->d, (const CgState*)R.st,
 		                   (const uint8_t*)R.flags->f8, R.gen(), (const float*)R.rhs, (const float*)R.x, R.r,
 		                   R.pcNone ? 1 : 0, R.dpart, R.fpart);
 		return (int)R.nbG;
 	}
-	hipLaunchKernelGGL(k_cg_replace_residual, dim3(R.nbT), dim3(kBlock), 0, s->stream, s->d, R.t, (const CgState*)R.st,
+	hipLaunchKernelGGL(k_cg_replace_residual, dim3(R.nbT), dim3(kBlock), 0, q, s->d, R.t, (const CgState*)R.st,
 	                   R.code, (const float*)R.rhs, (const float*)R.x, R.r, R.pcNone ? 1 : 0, R.dpart, R.fpart);
 	return (int)R.nbT;
 }
@@ -2007,8 +2008,16 @@ static int precondition(CgRun& R) {
 	return np;
 }
 
-// GridCg::iterate (conjugategrad.cpp:238-299), queued on the scene stream
-static void cg_iteration(CgRun& R) {
+// GridCg::iterate (conjugategrad.cpp:238-299), queued on the scene stream in
+// two parts: up to the residual norm and the stopping rule, then the
+// preconditioner and beta
+static void cg_part_b(CgRun& R) {
+	if (!R.owesB) return;
+	R.owesB = false;
+	const int np = precondition(R);
+	run_finalize_one(R.s->stream, R.fin(np, FIN_BETA));
+}
+static void cg_part_a(CgRun& R) {
 	Scene* s = R.s;
 	const bool odd = (R.launched & 1) != 0;
 	if (R.gA0) {
@@ -2030,13 +2039,10 @@ static void cg_iteration(CgRun& R) {
 	int nbRes = (int)R.nbU;
 	if (R.o.trueResidualEvery > 0 && (R.launched + 1) % R.o.trueResidualEvery == 0) {
 		// FP64 residual replacement; its partials replace the update's
-		nbRes = enqueue_replace_residual(R);
+		nbRes = enqueue_replace_residual(R, s->stream);
 	}
 	run_finalize_one(s->stream, R.fin(nbRes, FIN_RES));
-	if (!R.pcNone) {
-		const int np = precondition(R);
-		run_finalize_one(s->stream, R.fin(np, FIN_BETA));
-	}
+	R.owesB = !R.pcNone;
 	R.launched++;
 }
 
@@ -2080,12 +2086,16 @@ static void cg_release(CgRun& R) {
 
 // CG restarted from the current x: r = b - A x (FP64 row sums), z = M r,
 // p = z on the next iteration; the iteration count and ||b|| carry on
+static int cg_restart_residual(CgRun& R, hipStream_t q) {
+	hipLaunchKernelGGL(k_cg_restart, dim3(1), dim3(64), 0, q, R.st);
+	return enqueue_replace_residual(R, q);
+}
 static void cg_restart(CgRun& R) {
 	Scene* s = R.s;
-	hipLaunchKernelGGL(k_cg_restart, dim3(1), dim3(64), 0, s->stream, R.st);
-	int np = enqueue_replace_residual(R);
+	int np = cg_restart_residual(R, s->stream);
 	if (!R.pcNone) np = precondition(R);
 	run_finalize_one(s->stream, R.fin(np, FIN_BETA0));
+	R.owesB = false;
 }
 
 // With relTol the stopping rule reads the recursively updated FP32 residual,
@@ -2101,18 +2111,74 @@ static bool cg_needs_restart(const CgRun& R) {
 	const double rel = bb > 0 ? std::sqrt(hs->trueRR / bb) : std::sqrt(hs->trueRR);
 	return rel > R.o.relTol;
 }
-static void cg_iterate(CgRun& R, double target);
+// Iterations still needed after those the state has seen, from the decay of
+// the residual norm (at least 1; 0 when the state says done; -1 without a
+// usable rate).  Plain CG's norm wanders: its mean decay counts too.
+static int cg_iters_left(const CgState& hs, double target, bool pcNone) {
+	if (hs.done) return 0;
+	const int it = hs.iter;
+	if (it < 2 || !(target > 0)) return -1;
+	const double b = hs.resNorm, h0 = hs.hist[0], a = it <= 64 ? hs.hist[it - 2] : 0.0;
+	const double mean = h0 > 0 && b > 0 ? std::pow(b / h0, 1.0 / (it - 1)) : 1.0;
+	double rate = a > 0 && b > 0 ? b / a : mean;
+	if (pcNone) rate = std::min(rate, mean);
+	if (!(rate > 0 && rate < 1)) return -1;
+	const double need = std::ceil(std::log(target / b) / std::log(rate));
+	return need < 1 ? 1 : (need > 1e6 ? 1000000 : (int)need);
+}
+// the next run of iterations: what is predicted, but not more than were run
+// so far (a prediction from few norms can be far off, and an iteration queued
+// past convergence still launches its kernels)
+static int cg_plan(int left, int launched) {
+	const int most = std::min(64, std::max(4, launched));
+	return left < 0 ? std::min(4, most) : std::min(std::max(left, 1), most);
+}
+
 // Iterations, then the FP64 true residual and the state copy, until the
-// copied state says done or maxIter iterations are queued.  The residual is
-// queued as soon as the iterations in flight are predicted to converge; if
-// they did not, it is superseded by the one after further iterations.
-static void cg_iterate_finish(CgRun& R, double target) {
+// copied state says done or maxIter iterations are queued.  Runs of `plan`
+// iterations are queued at a time; the host reads the state after the
+// next-to-last one's stopping rule while the GPU goes on, so the queue does
+// not drain there.  The preconditioner part of the iteration that is
+// predicted to converge is not queued: after convergence its 20 to 30
+// launches would do nothing, at 2 us each.  If the prediction was short it
+// follows, after the residual, with further iterations.
+static void cg_iterate_finish(CgRun& R, double target, int plan) {
+	Scene* s = R.s;
+	CgState* hs = (CgState*)s->hscal;
+	if (!s->evState) MFX_HIP(hipEventCreateWithFlags(&s->evState, hipEventDisableTiming));
 	while (true) {
-		cg_iterate(R, target);
+		const int nIt = std::min(plan, R.maxIter - R.launched);
+		for (int it = 0; it < nIt; it++) {
+			cg_part_b(R);
+			cg_part_a(R);
+			if (it == nIt - 2) {
+				MFX_HIP(hipMemcpyAsync(hs, R.st, sizeof(CgState), hipMemcpyDeviceToHost, s->stream));
+				MFX_HIP(hipEventRecord(s->evState, s->stream));
+			}
+		}
+		if (nIt >= 2 && R.launched < R.maxIter) {
+			MFX_HIP(hipEventSynchronize(s->evState));
+			const int left = cg_iters_left(*hs, target, R.pcNone);
+			if (left < 0 || left > 1) {
+				plan = cg_plan(left < 0 ? left : left - 1, R.launched);
+				continue;
+			}
+		}
+		if (R.launched >= R.maxIter) cg_part_b(R);  // (its divergence test)
 		cg_true_residual_enqueue(R);
-		sync(R.s);
-		if (((const CgState*)R.s->hscal)->done || R.launched >= R.maxIter) return;
+		sync(s);
+		if (hs->done || R.launched >= R.maxIter) return;
+		plan = cg_plan(cg_iters_left(*hs, target, R.pcNone), R.launched);
 	}
+}
+// iterations that a restart is expected to take: the true residual is mostly
+// a few per cent above the target, one iteration away
+static int cg_restart_plan(const CgState& hs, double target) {
+	const int it = std::min(hs.iter, 64);
+	if (it < 2 || !(hs.bnorm2 > 0)) return 1;
+	const double rate = std::pow((double)hs.hist[it - 1] / hs.hist[0], 1.0 / (it - 1));
+	const double need = std::log(target / std::sqrt(hs.trueRR / hs.bnorm2)) / std::log(rate);
+	return need > 1 && need < 4 ? (int)std::ceil(need) : 1;
 }
 
 static void cg_verify(CgRun& R, double target) {
@@ -2121,14 +2187,16 @@ static void cg_verify(CgRun& R, double target) {
 		R.resident = false;
 		R.launched = 0;
 		cg_init(R);
-		cg_iterate_finish(R, target);
+		cg_iterate_finish(R, target, 4);
 	}
 	for (int k = 0; k < kMaxRestarts && cg_needs_restart(R); k++) {
 		// iterations queued past convergence did nothing; the budget follows
 		// the device count (p = z after the restart, so the buffer parity is free)
-		R.launched = ((const CgState*)R.s->hscal)->iter;
+		const CgState* hs = (const CgState*)R.s->hscal;
+		R.launched = hs->iter;
+		const int plan = cg_restart_plan(*hs, target);
 		cg_restart(R);
-		cg_iterate_finish(R, target);
+		cg_iterate_finish(R, target, plan);
 	}
 }
 
@@ -2190,53 +2258,12 @@ static void cg_drive(CgRun& R, double target, mfx_solve_stats* stats) {
 		cg_true_residual_enqueue(R);
 		sync(R.s);
 	} else {
-		cg_iterate_finish(R, target);
+		cg_iterate_finish(R, target, 4);
 	}
 	cg_verify(R, target);
 	cg_release(R);
 	cg_finish_collect(R, stats);
 }
-
-// Queues iterations in batches sized from the residual history.  The host
-// reads the state of the next-to-last iteration of a batch while the GPU
-// runs the last one, so the queue does not drain at these checks; it
-// returns when the iterations queued are predicted to reach the target (or
-// to be done, or maxIter is reached), and the caller queues the finish.
-static void cg_iterate(CgRun& R, double target) {
-	Scene* s = R.s;
-	int batch = 4;
-	CgState* hs = (CgState*)s->hscal;
-	if (!s->evState) MFX_HIP(hipEventCreateWithFlags(&s->evState, hipEventDisableTiming));
-	while (true) {
-		const int nIt = std::min(batch, R.maxIter - R.launched);
-		for (int it = 0; it < nIt; it++) {
-			cg_iteration(R);
-			if (it == nIt - 2) {
-				MFX_HIP(hipMemcpyAsync(hs, R.st, sizeof(CgState), hipMemcpyDeviceToHost, s->stream));
-				MFX_HIP(hipEventRecord(s->evState, s->stream));
-			}
-		}
-		if (nIt < 2 || R.launched >= R.maxIter) return;
-		MFX_HIP(hipEventSynchronize(s->evState));
-		if (hs->done) return;  // the iteration in flight returns at once
-		// iterations still needed after the one in flight (without a usable
-		// rate: another batch of the same size)
-		int more = batch;
-		const int itNow = hs->iter;
-		if (itNow >= 2 && itNow <= 64) {
-			const double a = hs->hist[itNow - 2], b = hs->hist[itNow - 1];
-			if (a > 0 && b > 0 && b < a && target > 0) {
-				const double rate = b / a;
-				double need = std::log(target / b) / std::log(rate);
-				if (need < 1) need = 1;
-				more = (int)std::ceil(need) - 1;
-			}
-		}
-		if (more <= 0) return;
-		batch = std::min(more, 64);
-	}
-}
-
 
 // GridCg without preconditioner over a scaled Laplace matrix (the other
 // GridCg clients): kind 0 builds cgSolveDiffusion's matrix code, kind 1 the
@@ -2310,13 +2337,9 @@ static void correct_velocity(Scene* s, Grid* flags, Grid* vel, const float* pres
 // Batched solve: many independent pressure systems (one per scene, any mix
 // of sizes and 2D/3D).  Set-up and finish run per problem; every iteration
 // is one launch per CG/MG phase over a work list that holds the tiles of all
-// problems, so small problems share launches with large ones.  Iterations are
-// queued a few ahead of pipelined convergence checks.  When a batch has the
-// same launch layout as the previous batch led by the same scene, two
-// iterations (both parities of the search-direction buffers) and the done-flag
-// gather are captured once in a hipGraph and replayed from then on.  Each
-// problem keeps its own device CgState, so converged problems drop out at
-// once (their workgroups return on st->done).
+// problems, so small problems share launches with large ones.  Each problem
+// keeps its own device CgState, so converged problems drop out at once
+// (their workgroups return on st->done).
 // ---------------------------------------------------------------------------
 namespace {
 
@@ -2358,11 +2381,6 @@ struct Step {
 	unsigned n() const { return (unsigned)total; }
 };
 
-__global__ void k_gather_done(int np, CgState* const* __restrict__ st, int* __restrict__ done) {
-	const int i = blockIdx.x * blockDim.x + threadIdx.x;
-	if (i < np) done[i] = st[i]->done;
-}
-
 struct BatchSolve {
 	int P = 0;
 	bool bf16 = false;
@@ -2386,13 +2404,15 @@ struct BatchSolve {
 	bool anyMg = false;
 	uint8_t* dmem = nullptr;
 	CgState** dStates = nullptr;
-	int* dDone = nullptr;
 
-	void enqueue(hipStream_t s, int parity) {
+	// an iteration of every problem, in the two parts of a single solve's
+	void part_a(hipStream_t s, int parity) {
 		run_matvec_many(s, mv[parity].n(), mv[parity].dItems, mv[parity].dParams);
 		run_finalize_many(s, fa.n(), fa.dItems, fa.dParams);
 		run_update_many(s, up[parity].n(), up[parity].dItems, up[parity].dParams);
 		run_finalize_many(s, fr.n(), fr.dItems, fr.dParams);
+	}
+	void part_b(hipStream_t s) {
 		if (!anyMg) return;
 		enqueue_vcycle(s);
 		run_finalize_many(s, fb.n(), fb.dItems, fb.dParams);
@@ -2682,8 +2702,6 @@ static void solve_batch(const std::vector<Grid*>& vel, const std::vector<Grid*>&
 		std::vector<CgState*> states((size_t)P);
 		for (int i = 0; i < P; i++) states[(size_t)i] = R[(size_t)i].st;
 		const size_t stOff = A.add(states.data(), sizeof(CgState*) * (size_t)P);
-		std::vector<int> zeros((size_t)P, 0);
-		const size_t doneOff = A.add(zeros.data(), sizeof(int) * (size_t)P);
 		std::vector<CgState> gatherInit((size_t)P);
 		const size_t gatherOff = A.add(gatherInit.data(), sizeof(CgState) * (size_t)P);
 		Scene* s0 = vel[0]->s;
@@ -2710,7 +2728,6 @@ static void solve_batch(const std::vector<Grid*>& vel, const std::vector<Grid*>&
 		MFX_HIP(hipMemcpyAsync(B.dmem, s0->hstage, A.host.size(), hipMemcpyHostToDevice, q));
 		placeAll([&](auto& st) { st.bind(B.dmem); });
 		B.dStates = (CgState**)(B.dmem + stOff);
-		B.dDone = (int*)(B.dmem + doneOff);
 		// the batch stream waits for every problem's set-up
 		for (int i = 1; i < P; i++) MFX_HIP(hipStreamWaitEvent(q, vel[(size_t)i]->s->ev, 0));
 		// initial V-cycle of every preconditioned problem, sigma = dot(z, r)
@@ -2719,132 +2736,108 @@ static void solve_batch(const std::vector<Grid*>& vel, const std::vector<Grid*>&
 			run_finalize_many(q, B.fb0.n(), B.fb0.dItems, B.fb0.dParams);
 		}
 
-		// launch layout of one iteration; equal keys give identical launches
-		std::vector<long long> key = {P, B.bf16 ? 1 : 0, B.anyMg ? 1 : 0, (long long)(uintptr_t)s0->arena};
-		placeAll([&](auto& st) {
-			key.push_back(st.total);
-			key.push_back((long long)st.startOff);
-			key.push_back((long long)st.paramOff);
-		});
-		key.push_back((long long)stOff);
-		key.push_back((long long)doneOff);
-		hipGraphExec_t gexec = nullptr;
-		if (s0->bexec && s0->bkey == key) {
-			gexec = s0->bexec;
-		} else if (s0->blastKey == key) {
-			// second batch in a row with this layout: capture it once
-			hipGraph_t graph = nullptr;
-			MFX_HIP(hipStreamBeginCapture(q, hipStreamCaptureModeThreadLocal));
-			B.enqueue(q, 0);
-			B.enqueue(q, 1);
-			hipLaunchKernelGGL(k_gather_done, dim3((P + 255) / 256), dim3(256), 0, q, P, (CgState* const*)B.dStates,
-			                   B.dDone);
-			MFX_HIP(hipStreamEndCapture(q, &graph));
-			hipGraphExec_t e = nullptr;
-			const hipError_t ie = hipGraphInstantiate(&e, graph, nullptr, nullptr, 0);
-			(void)hipGraphDestroy(graph);
-			MFX_HIP(ie);
-			if (s0->bexec) (void)hipGraphExecDestroy(s0->bexec);
-			s0->bexec = e;
-			s0->bkey = key;
-			gexec = e;
-		}
-		s0->blastKey = key;
-		// Iterations are queued directly on the batch stream, a few ahead of
-		// the host: after every second iteration the done flags of all
-		// problems are copied to a pinned slot and an event recorded; the host
-		// waits only for the oldest outstanding check while later iterations
-		// are already queued.  Iterations queued after every problem has
-		// converged return at once (their kernels test the done flag).
-		constexpr int kAhead = 4;  // iterations queued beyond the last completed check
-		int* hdone = (int*)s0->hscal;  // pinned, 4 KiB: one slot of P flags per outstanding check
-		const int nslot = std::max(1, (int)(4096 / (sizeof(int) * (size_t)P)));
-		const bool pinned = nslot >= 2;
-		std::vector<int> done((size_t)P, 0);
-		struct Check {
-			int its;
-			int slot;
-			hipEvent_t ev;
+		// Iterations are queued as in a single solve (cg_iterate_finish), for
+		// all problems at once: a run is as long as the slowest problem is
+		// predicted to take, its next-to-last iteration's states are copied and
+		// read while the GPU goes on, and the last one's preconditioner part is
+		// left out.  Kernels of a converged problem return at once.
+		CgState* dGather = (CgState*)(B.dmem + gatherOff);
+		CgState* hst = (CgState*)s0->hstage;  // pinned, P states
+		const double target = o.relTol > 0 ? o.relTol : (double)o.cgAccuracy;
+		if (!s0->evState) MFX_HIP(hipEventCreateWithFlags(&s0->evState, hipEventDisableTiming));
+		auto copy_states = [&]() {
+			hipLaunchKernelGGL(k_gather_states, dim3((P + 255) / 256), dim3(256), 0, q, P, (CgState* const*)B.dStates,
+			                   dGather);
+			MFX_HIP(hipMemcpyAsync(hst, dGather, sizeof(CgState) * (size_t)P, hipMemcpyDeviceToHost, q));
 		};
-		std::vector<hipEvent_t> evPool;
-		std::deque<Check> pending;
-		int its = 0, checked = 0, nextSlot = 0;
-		auto take_event = [&]() {
-			hipEvent_t e;
-			if (!evPool.empty()) {
-				e = evPool.back();
-				evPool.pop_back();
-			} else {
-				MFX_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+		// the most iterations any problem still needs (-1: unknown for some)
+		auto iters_left = [&]() {
+			int most = 0;
+			for (int i = 0; i < P; i++) {
+				const int left = cg_iters_left(hst[i], target, R[(size_t)i].pcNone);
+				if (left < 0) return -1;
+				most = std::max(most, left);
 			}
-			return e;
+			return most;
 		};
-		bool converged = false;
-		const auto tIter = std::chrono::steady_clock::now();
-		try {
-			while (!converged) {
-				while (its < maxIt && its - checked < kAhead && (pinned ? (int)pending.size() < nslot : pending.empty())) {
-					if (gexec && maxIt - its >= 2) {
-						// (its is even here: the graph starts with parity 0)
-						MFX_HIP(hipGraphLaunch(gexec, q));
-						its += 2;
-					} else {
-						B.enqueue(q, its & 1);
-						its++;
-					}
-					if ((its & 1) == 0 || its == maxIt) {
-						const int slot = pinned ? nextSlot : 0;
-						nextSlot = (nextSlot + 1) % nslot;
-						if (!gexec || (its & 1))
-							hipLaunchKernelGGL(k_gather_done, dim3((P + 255) / 256), dim3(256), 0, q, P,
-							                   (CgState* const*)B.dStates, B.dDone);
-						MFX_HIP(hipMemcpyAsync(pinned ? hdone + (size_t)slot * P : done.data(), B.dDone,
-						                       sizeof(int) * (size_t)P, hipMemcpyDeviceToHost, q));
-						hipEvent_t e = take_event();
-						MFX_HIP(hipEventRecord(e, q));
-						pending.push_back(Check{its, slot, e});
+		int its = 0;
+		bool owesB = false;
+		auto iterate = [&](int plan, int limit) {
+			while (true) {
+				const int nIt = std::min(plan, limit - its);
+				for (int it = 0; it < nIt; it++) {
+					if (owesB) B.part_b(q);
+					B.part_a(q, its & 1);
+					owesB = true;
+					its++;
+					if (it == nIt - 2) {
+						copy_states();
+						MFX_HIP(hipEventRecord(s0->evState, q));
 					}
 				}
-				if (pending.empty()) break;
-				Check c = pending.front();
-				pending.pop_front();
-				MFX_HIP(hipEventSynchronize(c.ev));
-				evPool.push_back(c.ev);
-				checked = c.its;
-				const int* dn = pinned ? hdone + (size_t)c.slot * P : done.data();
-				bool all = true;
-				for (int i = 0; i < P && all; i++) all = dn[i] != 0;
-				converged = all || (its >= maxIt && pending.empty());
+				if (nIt >= 2 && its < limit) {
+					MFX_HIP(hipEventSynchronize(s0->evState));
+					const int left = iters_left();
+					if (left < 0 || left > 1) {
+						plan = cg_plan(left < 0 ? left : left - 1, its);
+						continue;
+					}
+				}
+				if (its >= limit && owesB) {
+					B.part_b(q);
+					owesB = false;
+				}
+				// every problem's true residual and its sum, all states to the host
+				run_true_residual_many(q, B.tres.n(), B.tres.dItems, B.tres.dParams);
+				run_reduce_true_rr_many(q, B.tred.n(), B.tred.dItems, B.tred.dParams);
+				copy_states();
+				sync(s0);
+				const int left = iters_left();
+				if (left == 0 || its >= limit) return;
+				plan = cg_plan(left, its);
 			}
-		} catch (...) {
-			for (auto& c : pending) evPool.push_back(c.ev);
-			for (hipEvent_t e : evPool) (void)hipEventDestroy(e);
-			throw;
-		}
-		for (auto& c : pending) evPool.push_back(c.ev);
-		for (hipEvent_t e : evPool) (void)hipEventDestroy(e);
+		};
+		const auto tIter = std::chrono::steady_clock::now();
+		iterate(4, maxIt);
 		batch_policy_done(tkey, policy,
 		                  std::chrono::duration<double>(std::chrono::steady_clock::now() - tIter).count());
-		for (int i = 0; i < P; i++) R[(size_t)i].launched = its;
-		// finish, batched: every problem's true residual and its sum, one
-		// copy of all CgStates to the host, each problem's state into its
-		// scene's host mirror (as a single solve leaves it)
-		run_true_residual_many(q, B.tres.n(), B.tres.dItems, B.tres.dParams);
-		run_reduce_true_rr_many(q, B.tred.n(), B.tred.dItems, B.tred.dParams);
-		CgState* dGather = (CgState*)(B.dmem + gatherOff);
-		hipLaunchKernelGGL(k_gather_states, dim3((P + 255) / 256), dim3(256), 0, q, P, (CgState* const*)B.dStates,
-		                   dGather);
-		MFX_HIP(hipMemcpyAsync(s0->hstage, dGather, sizeof(CgState) * (size_t)P, hipMemcpyDeviceToHost, q));
-		sync(s0);
-		for (int i = 0; i < P; i++)
-			std::memcpy(vel[(size_t)i]->s->hscal, (const CgState*)s0->hstage + i, sizeof(CgState));
-		// the relTol check on the true residual, as in a single solve; a
-		// problem that needs a restart continues alone on its own stream
-		// (and has synchronized it when cg_verify returns)
-		const double target = o.relTol > 0 ? o.relTol : (double)o.cgAccuracy;
+		// each problem's state into its scene's host mirror (as a single solve
+		// leaves it), then the relTol check on the true residual: the
+		// preconditioned problems that need it restart together
+		auto mirror = [&]() {
+			for (int i = 0; i < P; i++) {
+				std::memcpy(vel[(size_t)i]->s->hscal, hst + i, sizeof(CgState));
+				R[(size_t)i].launched = hst[i].iter;
+			}
+		};
+		mirror();
+		std::vector<char> again((size_t)P, 0);
+		for (int k = 0; k < kMaxRestarts; k++) {
+			int n = 0, plan = 1, limit = 0;
+			for (int i = 0; i < P; i++) {
+				CgRun& r = R[(size_t)i];
+				again[(size_t)i] = !r.pcNone && cg_needs_restart(r) ? 1 : 0;
+				if (!again[(size_t)i]) continue;
+				n++;
+				plan = std::max(plan, cg_restart_plan(hst[i], target));
+				limit = std::max(limit, r.maxIter - hst[i].iter);
+			}
+			if (!n) break;
+			for (int i = 0; i < P; i++)
+				if (again[(size_t)i]) cg_restart_residual(R[(size_t)i], q);
+			B.enqueue_vcycle(q);
+			run_finalize_many(q, B.fb0.n(), B.fb0.dItems, B.fb0.dParams);
+			owesB = false;
+			its = 0;
+			iterate(plan, limit);
+			mirror();
+		}
+		// what is left runs alone on its own stream (unpreconditioned restarts,
+		// one-kernel solves that gave up) and has synchronized it on return
 		for (int i = 0; i < P; i++) {
-			cg_verify(R[(size_t)i], target);
-			cg_release(R[(size_t)i]);
+			CgRun& r = R[(size_t)i];
+			if (r.pcNone) cg_verify(r, target);
+			cg_release(r);
 		}
 		run_correct_velocity_many(q, B.corr.n(), B.corr.dItems, B.corr.dParams);
 		sync(s0);
