@@ -1418,8 +1418,25 @@ __device__ __forceinline__ void body_smooth(const SmoothP& P, long long blk, lon
 	const int gx = ox + tx, gy = oy + ty, gz = oz + tz;
 	const bool valid = gx < c.nx && gy < c.ny && gz < c.nz;
 	const int v = valid ? gx + sy * gy + sz * gz : 0;
-	const uint8_t tv = valid ? type[v] : (uint8_t)0;
+	const uint8_t tl = type[v];
 	const float bv = b[v];
+	// post-smoothing: the region's old iterate and types, asked for before
+	// anything waits
+	constexpr int NIT = (RN + kSmoothNT - 1) / kSmoothNT;
+	float xr[NIT];
+	uint8_t tr[NIT];
+	if (POST) {
+#pragma unroll
+		for (int it = 0; it < NIT; it++) {
+			const int q = t + kSmoothNT * it;
+			const int hx = ox - 1 + q % RX, hy = oy - 1 + (q / RX) % RY, hzz = oz - hz + q / RXY;
+			const bool inb = q < RN && hx >= 0 && hy >= 0 && hzz >= 0 && hx < c.nx && hy < c.ny && hzz < c.nz;
+			const int g = inb ? hx + sy * hy + sz * hzz : 0;
+			xr[it] = xin[g];
+			tr[it] = type[g];
+		}
+	}
+	const uint8_t tv = valid ? tl : (uint8_t)0;
 	float a[NS];
 	float diag = 1.f;
 	if (tv == 2) {
@@ -1427,19 +1444,28 @@ __device__ __forceinline__ void body_smooth(const SmoothP& P, long long blk, lon
 #pragma unroll
 		for (int s = 0; s < NS; s++) a[s] = s == C ? 0.f : cn.a[s];
 	} else if (tv) {
-		diag = ldA(A, v);
-		int s = 0;
-		for (int dz = (IS3D ? -1 : 0); dz <= (IS3D ? 1 : 0); dz++)
-			for (int dy = -1; dy <= 1; dy++)
-				for (int dx = -1; dx <= 1; dx++, s++) {
-					float coef = 0.f;
-					const int nx = gx + dx, ny = gy + dy, nz = gz + dz;
-					if (s != C && nx >= 0 && ny >= 0 && nz >= 0 && nx < c.nx && ny < c.ny && nz < c.nz) {
-						const int nn = nx + sy * ny + sz * nz;
-						coef = s > C ? ldA(A, (long long)(s - C) * c.n + v) : ldA(A, (long long)(C - s) * c.n + nn);
-					}
-					a[s] = coef;
-				}
+		// all coefficients in flight at once: the upper ones are the vertex's
+		// own (0 towards neighbours outside the level), a lower one is its
+		// neighbour's; outside the level any valid address is read and 0 taken.
+		// With a branch and a wait per coefficient a small level's sweep was
+		// bound by them (17^3: 7.2 us before smoothing, 7.7 after; now 6.0 and
+		// 6.4; 65^3 after smoothing 13.6 -> 11.3, 129^3 41 -> 38.5).  What is
+		// left of a small level's 6 us: 1.8 in the colour phases, 1 in the
+		// loads' latency, 3 in the launch itself.
+		const bool in[3][3] = {{gx > 0, true, gx < c.nx - 1}, {gy > 0, true, gy < c.ny - 1}, {gz > 0, true, gz < c.nz - 1}};
+#pragma unroll
+		for (int s = 0; s < NS; s++) {
+			const int dx = s % 3 - 1, dy = (s / 3) % 3 - 1, dz = IS3D ? s / 9 - 1 : 0;
+			const bool ok = s >= C || (in[0][dx + 1] && in[1][dy + 1] && (!IS3D || in[2][dz + 1]));
+			const int nn = s >= C || !ok ? v : v + dx + sy * dy + sz * dz;
+			a[s] = ldA(A + (long long)(s >= C ? s - C : C - s) * c.n, nn);
+		}
+#pragma unroll
+		for (int s = 0; s < C; s++) {
+			const int dx = s % 3 - 1, dy = (s / 3) % 3 - 1, dz = IS3D ? s / 9 - 1 : 0;
+			if (!(in[0][dx + 1] && in[1][dy + 1] && (!IS3D || in[2][dz + 1]))) a[s] = 0.f;
+		}
+		diag = a[C];
 	}
 	if (POST) {
 		const int psy = (int)cp.sy, psz = (int)cp.sz;
@@ -1453,7 +1479,7 @@ __device__ __forceinline__ void body_smooth(const SmoothP& P, long long blk, lon
 		__syncthreads();
 	}
 #pragma unroll
-	for (int it = 0; it < (RN + kSmoothNT - 1) / kSmoothNT; it++) {
+	for (int it = 0; it < NIT; it++) {
 		const int q = t + kSmoothNT * it;
 		if (q >= RN) break;
 		const int rx = q % RX, ry = (q / RX) % RY, rz = q / RXY;
@@ -1461,10 +1487,8 @@ __device__ __forceinline__ void body_smooth(const SmoothP& P, long long blk, lon
 		const bool inb = hx >= 0 && hy >= 0 && hzz >= 0 && hx < c.nx && hy < c.ny && hzz < c.nz;
 		float x = 0.f;
 		if (POST) {
-			// branch-free: a valid address for every load, results selected
-			const int g = inb ? hx + sy * hy + sz * hzz : 0;
-			x = xin[g];
-			const uint8_t tp = type[g];
+			x = xr[it];
+			const uint8_t tp = tr[it];
 			// parents [s/2, (s+1)/2] per axis; with o even, s = o - 1 + r has
 			// parity (r + 1) & 1 and its first parent in LDS slot (r + 1) >> 1
 			const int odx = (rx + 1) & 1, ody = (ry + 1) & 1, odz = IS3D ? (rz + 1) & 1 : 0;
