@@ -600,27 +600,36 @@ __device__ __forceinline__ void body_dot(const DotP& P, long long blk, long long
 }
 
 // A: p_new = z + beta*p_old ; q = A p_new ; partial sums of fl(q*p_new).
-// z-marching form: a 64 x TY tile of columns walks a chunk of planes.  The
-// search direction of the current plane (tile + 1-cell ring) is staged in
-// LDS, the planes below and above stay in registers, so every value is read
-// from HBM once.  Row arithmetic and term order follow apply_row; neighbours
-// outside the grid contribute 0 (their coefficient is 0 there).
+// z-marching form: a 64 x TY tile of columns walks a chunk of planes, one
+// wavefront per row.  The search direction of the current plane (tile + ring)
+// is staged in LDS, the planes below and above stay in registers, so every
+// value is read from HBM once.  Row arithmetic and term order follow
+// apply_row; neighbours outside the grid contribute 0 (their coefficient is
+// 0 there).
 //
-// Loads run one plane ahead as raw values (z, p_old, code): p_new = z +
-// beta p_old is formed only when a plane enters LDS, so the loads of plane
-// k+2 are in flight during the whole step of plane k.
+// Loads run two planes ahead as raw values (z, p_old, code): p_new = z +
+// beta p_old is formed only when a plane enters LDS.  A wavefront's row is
+// one bounded buffer per plane (records: the row's cells inside the grid, 0
+// for a plane or row outside), so lanes outside read 0 and their stores are
+// dropped without any per-lane address or validity arithmetic, and nothing
+// between a plane's loads and their use depends on a branch: the wait for
+// them leaves the next plane's loads and the stores in flight.  The ring is
+// the work of the first three wavefronts (row below, row above, both sides).
+// A plane costs a workgroup 0.52 us with the machine otherwise idle, 0.60
+// with the loads one plane ahead and per-lane addresses; 192x160x129 15.3 ->
+// 14.1 us, 256^3 63.4 -> 61.6 us (4.6 TB/s, the rate of a large copy).
 template <int TY, bool SC = false>
 __device__ __forceinline__ void body_matvec(const MatvecP& P, long long blk, long long slot) {
-	constexpr int TX = 64, RX = TX + 2, RY = TY + 2, NH = 2 * RX + 2 * (RY - 2);
-	// plane buffers; the 64 slots past the ring take the writes of lanes
-	// that have no ring cell
-	__shared__ float ps[2][RX * RY + 64];
-	__shared__ uint8_t cs[2][RX * RY + 64];
+	constexpr int TX = 64, RX = TX + 2, RY = TY + 2;
+	static_assert(TY >= 3 && 2 * TY <= TX, "the ring's wavefronts");
+	// plane buffers; the slot past the ring takes the writes of lanes that
+	// have no ring cell
+	__shared__ float ps[2][RX * RY + 1];
+	__shared__ uint8_t cs[2][RX * RY + 1];
 	__shared__ double tab[kZmMaxGroups][TY];
 	const Dims& d = P.d;
 	const int kchunk = P.kchunk;
 	const CgState* __restrict__ st = P.st;
-	const uint8_t* __restrict__ code = P.code;
 	if (st->done) return;
 	const float beta = st->beta;
 	const bool first = st->first;
@@ -628,117 +637,133 @@ __device__ __forceinline__ void body_matvec(const MatvecP& P, long long blk, lon
 	// in the first iteration p_old is not used: its loads read z's lines
 	// (cache hits) instead of a second stream
 	const float* __restrict__ pold = first ? P.z : P.pold;
-	float* __restrict__ pnew = P.pnew;
-	float* __restrict__ q = P.q;
+	const uint8_t* __restrict__ code = P.code;
 	const unsigned ntx = (unsigned)(d.nx + TX - 1) / TX, nty = (unsigned)(d.ny + TY - 1) / TY;
 	const unsigned b32 = (unsigned)blk, rest = b32 / ntx;
 	const int ox = (int)(b32 - rest * ntx) * TX;
 	const int oy = (int)(rest % nty) * TY;
 	const int k0 = (int)(rest / nty) * kchunk, k1 = min(d.nz, k0 + kchunk);
-	const int tx = threadIdx.x & 63, ty = threadIdx.x >> 6;
-	const int gx = ox + tx, gy = oy + ty;
-	const bool in = gx < d.nx && gy < d.ny;
-	// one ring cell per thread (threads < NH)
-	static_assert(NH <= 64 * TY, "one ring cell per thread");
-	const int h = threadIdx.x;
-	int hx = 0, hy = 0;
-	if (h < RX) { hx = h; hy = 0; }
-	else if (h < 2 * RX) { hx = h - RX; hy = RY - 1; }
-	else if (h < 2 * RX + RY - 2) { hx = 0; hy = 1 + h - 2 * RX; }
-	else { hx = RX - 1; hy = 1 + h - 2 * RX - (RY - 2); }
+	const int tx = threadIdx.x & 63, ty = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+	// the wavefront's row: first cell of plane 0 and cells inside the grid
+	const long long row = ox + (long long)d.nx * (oy + ty);
+	const int nrow = oy + ty < d.ny ? min(TX, d.nx - ox) : 0;
+	const int vf = 4 * tx;
+	auto cells = [](const void* base, long long bytes, int records) {
+		return __builtin_amdgcn_make_buffer_rsrc((char*)base + bytes, 0, records, 0x00020000);
+	};
+	// the thread's ring cell (corners are no neighbours)
+	const bool ringWave = ty < 3;
+	const int hx = ty < 2 ? tx + 1 : (tx < TY ? 0 : RX - 1), hy = ty == 0 ? 0 : (ty == 1 ? RY - 1 : 1 + tx % TY);
 	const int hgx = ox - 1 + hx, hgy = oy - 1 + hy;
-	const bool hin = h < NH && hgx >= 0 && hgy >= 0 && hgx < d.nx && hgy < d.ny;
-	const long long gcol = in ? (long long)gx + (long long)d.nx * gy : 0;
+	const bool hcell = ty < 2 || tx < 2 * TY;
+	const bool hin = hcell && hgx >= 0 && hgy >= 0 && hgx < d.nx && hgy < d.ny;
 	const long long hcol = hin ? (long long)hgx + (long long)d.nx * hgy : 0;
-	// Raw values of one plane: own column (z, p_old, code) and ring cell
-	// (same).  The six loads are issued without branches (a plane outside
-	// the tile's planes k0-1..k1 or the grid reads a clamped plane, a lane
-	// outside the grid reads column 0; in the first iteration the p_old
-	// loads read z and are ignored), so the compiler can wait for one
-	// plane's loads while the next plane's stay in flight; validity is
-	// applied where the values are used.
+	const int L = (tx + 1) + RX * (ty + 1);
+	const int HS = hcell ? hx + RX * hy : RX * RY;  // ring slot or spare
 	struct Raw {
 		float z, po, hz, hpo;
 		uint8_t c, hc;
-		bool ok;
 	};
-	const int kLo = max(k0 - 1, 0), kHi = min(k1, d.nz - 1);
+	// cell offsets of the row in the plane to load and the plane to store
+	long long ol = row + d.sz * (k0 - 1), os = row + d.sz * k0;
+	const int kHi = min(k1, d.nz - 1);
+	// planes k0-1, k0, .. in turn (past k1 nothing is read)
 	auto load = [&](int kk, Raw& r) {
-		const long long pl = d.sz * min(max(kk, kLo), kHi);
-		r.z = z[gcol + pl];
-		r.po = pold[gcol + pl];
-		r.c = code[gcol + pl];
-		r.hz = z[hcol + pl];
-		r.hpo = pold[hcol + pl];
-		r.hc = code[hcol + pl];
-		r.ok = kk >= 0 && kk < d.nz;
+		const int n = kk >= 0 && kk <= kHi ? nrow : 0;
+		r.z = __int_as_float((int)__builtin_amdgcn_raw_buffer_load_b32(cells(z, 4 * ol, 4 * n), vf, 0, 0));
+		r.po = __int_as_float((int)__builtin_amdgcn_raw_buffer_load_b32(cells(pold, 4 * ol, 4 * n), vf, 0, 0));
+		r.c = __builtin_amdgcn_raw_buffer_load_b8(cells(code, ol, n), tx, 0, 0);
+		if (ringWave) {
+			const long long h = hcol + d.sz * min(max(kk, 0), kHi);
+			r.hz = z[h];
+			r.hpo = pold[h];
+			r.hc = code[h];
+		}
+		ol += d.sz;
 	};
 	auto pn = [&](float zv, float pv) -> float { return first ? zv : zv + beta * pv; };
-	auto own = [&](const Raw& r) -> float { return in && r.ok ? pn(r.z, r.po) : 0.f; };
-	auto ownc = [&](const Raw& r) -> uint8_t { return in && r.ok ? r.c : (uint8_t)0; };
-	auto ring = [&](const Raw& r) -> float { return hin && r.ok ? pn(r.hz, r.hpo) : 0.f; };
-	auto ringc = [&](const Raw& r) -> uint8_t { return hin && r.ok ? r.hc : (uint8_t)0; };
-	const int L = (tx + 1) + RX * (ty + 1);
-	const int HS = h < NH ? hx + RX * hy : RX * RY + tx;  // ring slot or spare
+	// plane kk's own cell and ring cell into LDS buffer b
+	float* __restrict__ psf = &ps[0][0];
+	uint8_t* __restrict__ csf = &cs[0][0];
+	constexpr int LB = RX * RY + 1;
+	auto stage = [&](const Raw& r, int b, bool ok, float& pv) {
+		pv = pn(r.z, r.po);
+		psf[b * LB + L] = pv;
+		csf[b * LB + L] = r.c;
+		if (ringWave) {
+			const bool in = hin && ok;
+			psf[b * LB + HS] = in ? pn(r.hz, r.hpo) : 0.f;
+			csf[b * LB + HS] = in ? r.hc : (uint8_t)0;
+		}
+	};
+	// x if bit B of the code is set, else +0
+	auto keep = [](float x, uint8_t c, int B) -> float {
+		return __int_as_float(__float_as_int(x) & __builtin_amdgcn_sbfe((int)c, B, 1));
+	};
 	float pPrev, pCur, pNext;
 	uint8_t cPrev, cCur, cNext;
-	Raw R;
+	Raw R[2];
 	{
-		load(k0 - 1, R);
-		pPrev = own(R);
-		cPrev = ownc(R);
-		load(k0, R);
-		pCur = own(R);
-		cCur = ownc(R);
-		ps[0][L] = pCur;
-		cs[0][L] = cCur;
-		ps[0][HS] = ring(R);
-		cs[0][HS] = ringc(R);
+		Raw r0, r1;
+		load(k0 - 1, r0);
+		load(k0, r1);
+		load(k0 + 1, R[0]);
+		load(k0 + 2, R[1]);
+		pPrev = pn(r0.z, r0.po);
+		cPrev = r0.c;
+		stage(r1, 0, true, pCur);
+		cCur = r1.c;
 	}
-	load(k0 + 1, R);
 	__syncthreads();
 	double acc = 0.0;
-	int b = 0;  // LDS buffer of plane k
-	for (int k = k0; k < k1; k++, b ^= 1) {
-		// R holds plane k+1: it goes to LDS buffer b^1 (whose plane k-1 was
+	const float nsc = -P.scale;
+	auto step = [&](int k, Raw& r, int b) {
+		// r holds plane k+1: it goes to LDS buffer b^1 (whose plane k-1 was
 		// last read before the previous barrier; after the last plane the
-		// write is unused) without a branch, and only then is R reloaded
-		// with plane k+2, so R keeps its registers across iterations
-		pNext = own(R);
-		cNext = ownc(R);
-		ps[b ^ 1][L] = pNext;
-		cs[b ^ 1][L] = cNext;
-		ps[b ^ 1][HS] = ring(R);
-		cs[b ^ 1][HS] = ringc(R);
+		// write is unused), and only then is r reloaded with plane k+3
+		stage(r, b ^ 1, k + 1 < d.nz, pNext);
+		cNext = r.c;
 		__builtin_amdgcn_sched_barrier(0);
-		load(k + 2, R);
-		if (in) {
-			const float* __restrict__ pp = ps[b];
-			const uint8_t* __restrict__ cp = cs[b];
-			float qv;
-			if (!(cCur & 64)) qv = pCur;
-			else if (SC) {
-				const float sc = P.scale;
-				qv = pCur * sA0(cCur, sc) + pp[L - 1] * sOff(cp[L - 1], 8, sc) + pp[L + 1] * sOff(cCur, 8, sc) +
-				     pp[L - RX] * sOff(cp[L - RX], 16, sc) + pp[L + RX] * sOff(cCur, 16, sc);
-				if (d.is3d) qv = qv + pPrev * sOff(cPrev, 32, sc) + pNext * sOff(cCur, 32, sc);
-			} else if (d.is3d)
-				qv = pCur * cA0(cCur) + pp[L - 1] * cAi(cp[L - 1]) + pp[L + 1] * cAi(cCur) + pp[L - RX] * cAj(cp[L - RX]) +
-				     pp[L + RX] * cAj(cCur) + pPrev * cAk(cPrev) + pNext * cAk(cCur);
-			else
-				qv = pCur * cA0(cCur) + pp[L - 1] * cAi(cp[L - 1]) + pp[L + 1] * cAi(cCur) + pp[L - RX] * cAj(cp[L - RX]) +
-				     pp[L + RX] * cAj(cCur);
-			const long long m = gcol + d.sz * k;
-			pnew[m] = pCur;
-			q[m] = qv;
-			acc += (double)(qv * pCur);
+		load(k + 3, r);
+		const float* __restrict__ pp = psf + b * LB;
+		const uint8_t* __restrict__ cp = csf + b * LB;
+		const uint8_t cw = cp[L - 1], cs_ = cp[L - RX];
+		const float pw = pp[L - 1], pe = pp[L + 1], po = pp[L - RX], pq = pp[L + RX];
+		float qv;
+		if (SC) {
+			qv = pCur * sA0(cCur, P.scale) + keep(pw, cw, 3) * nsc;
+			qv = qv + keep(pe, cCur, 3) * nsc;
+			qv = qv + keep(po, cs_, 4) * nsc;
+			qv = qv + keep(pq, cCur, 4) * nsc;
+			if (d.is3d) {
+				qv = qv + keep(pPrev, cPrev, 5) * nsc;
+				qv = qv + keep(pNext, cCur, 5) * nsc;
+			}
+		} else {
+			qv = pCur * cA0(cCur) - keep(pw, cw, 3);
+			qv = qv - keep(pe, cCur, 3);
+			qv = qv - keep(po, cs_, 4);
+			qv = qv - keep(pq, cCur, 4);
+			if (d.is3d) {
+				qv = qv - keep(pPrev, cPrev, 5);
+				qv = qv - keep(pNext, cCur, 5);
+			}
 		}
+		qv = (cCur & 64) ? qv : pCur;
+		__builtin_amdgcn_raw_buffer_store_b32((unsigned)__float_as_int(pCur), cells(P.pnew, 4 * os, 4 * nrow), vf, 0, 0);
+		__builtin_amdgcn_raw_buffer_store_b32((unsigned)__float_as_int(qv), cells(P.q, 4 * os, 4 * nrow), vf, 0, 0);
+		os += d.sz;
+		acc += (double)(qv * pCur);
 		if ((k + 1) % kDotGroup == 0 || k + 1 == k1) zm_dot_flush<TY>(acc, tab, k, k0);
 		__syncthreads();
 		pPrev = pCur;
 		cPrev = cCur;
 		pCur = pNext;
 		cCur = cNext;
+	};
+	for (int k = k0; k < k1; k += 2) {
+		step(k, R[0], 0);
+		if (k + 1 < k1) step(k + 1, R[1], 1);
 	}
 	(void)slot;
 	zm_dot_store<TY>(tab, d, zm_column(blk, d, TY), k0, k1, P.part);
@@ -1742,6 +1767,16 @@ static void autotune_zmarch(Scene* s, const uint8_t* code) {
 	const Dims& d = s->d;
 	if (!d.is3d) return;
 	if (!zm_claim_tuning(d)) return;
+	// At most one workgroup per CU even with the shortest chunk: that is the
+	// fastest one (a plane more costs a workgroup 0.5 us in the matvec, 0.8 and
+	// 1.1 us in the level-0 sweeps; 44x66x44 with 4 / 8 planes: 6.7 / 8.7, 10.6 /
+	// 14.1, 13.4 / 17.7 us), and launches this short are too close to the
+	// host's launch rate for the trials to tell.
+	int kc4 = 0;
+	if (matvec_tiles(d, &kc4, false, kDotGroup) <= 256) {
+		zm_set_tuned(d, ZmTune{kDotGroup, kDotGroup});
+		return;
+	}
 	float* a = s->getReal();
 	float* b = s->getReal();
 	float* c = s->getReal();

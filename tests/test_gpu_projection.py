@@ -163,3 +163,31 @@ def test_zmarch_result_independent_of_chunk(manta, oracle):
         assert setc(*shape, 6, 8) == -1 and setc(*shape, 8, 68) == -1 and setc(*shape, 0, 8) == -1
     finally:
         setc(*shape, 0, 0)
+
+
+@pytest.mark.parametrize("shape", [(5, 17, 9), (64, 16, 4), (65, 33, 7), (130, 4, 6), (63, 15, 21), (128, 49, 5)])
+def test_zmarch_matvec_tile_edges(manta, oracle, shape):
+    """Grids that end inside, at and just past a 64x16 column tile and a plane
+    chunk: the rows' bounded loads and stores reach exactly the grid, and the
+    chunk does not change a bit.  The solve stops at max |r| < 1e-4, so the
+    true relative residual (another kernel's) is below 1e-4 / rms(b), with a
+    divergence of rms above 0.1."""
+    _, setc = _zm_hooks()
+    rng = np.random.default_rng(sum(shape))
+    flags = obstacle_flags(oracle, shape, 0.05, rng)
+    vel = smooth_vel(rng, shape, passes=1)
+    oracle.set_wall_bcs(shape, flags, vel)
+    try:
+        res = []
+        for mv in (4, 8, 12):
+            assert setc(*shape, mv, 4) == 0
+            g = GpuScene(manta, shape)
+            f, v, p = g.flags(flags), g.mac(vel), g.real()
+            manta.solvePressure(flags=f, vel=v, pressure=p, cgAccuracy=1e-4, preconditioner=manta.PcMGStatic)
+            st = manta.lastSolveStats(g.s)
+            assert st["converged"] and st["relResidual"] <= 1e-3, st
+            res.append(p.toNumpy().copy())
+        np.testing.assert_array_equal(res[0], res[1])
+        np.testing.assert_array_equal(res[0], res[2])
+    finally:
+        setc(*shape, 0, 0)
