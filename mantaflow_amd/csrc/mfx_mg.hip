@@ -1557,19 +1557,31 @@ __device__ __forceinline__ void body_coarsest(const CoarsestP& P, long long blk,
 	const float* __restrict__ b = P.b;
 	const uint8_t* __restrict__ code = P.code;
 	float* __restrict__ x = P.x;
-	if (st->done) return;
+	// latency, not work: the state, the right-hand side's indices and the row
+	// of the inverse are asked for together, kN of each per lane at a time
+	// (past the end an index in range, and the value is not added)
+	constexpr int kN = 12;
+	const int done = st->done;
 	const int lane = threadIdx.x & 63;
 	const int row = (int)blk * 4 + (threadIdx.x >> 6);
 	if (row >= nc) return;
+	const int ov = cidx[row];
 	double acc = 0.0;
-#pragma unroll 4
-	for (int jj = lane; jj < nc; jj += 64) {
-		const int v = cidx[jj];
-		const double bv = code ? (double)(b[v] * l0_scale(code[v])) : (double)b[v];
-		acc += G[(long long)row * nc + jj] * bv;
+	for (int j0 = 0; j0 < nc; j0 += 64 * kN) {
+		int v[kN];
+		double g[kN], bv[kN];
+#pragma unroll
+		for (int e = 0; e < kN; e++) v[e] = cidx[min(j0 + 64 * e + lane, nc - 1)];
+#pragma unroll
+		for (int e = 0; e < kN; e++) g[e] = G[(long long)row * nc + min(j0 + 64 * e + lane, nc - 1)];
+#pragma unroll
+		for (int e = 0; e < kN; e++) bv[e] = code ? (double)(b[v[e]] * l0_scale(code[v[e]])) : (double)b[v[e]];
+#pragma unroll
+		for (int e = 0; e < kN; e++)
+			if (j0 + 64 * e + lane < nc) acc += g[e] * bv[e];
 	}
 	acc = wave_sum(acc);
-	if (lane == 0) x[cidx[row]] = (float)acc;
+	if (lane == 0 && !done) x[ov] = (float)acc;
 }
 
 // ---------------------------------------------------------------------------

@@ -844,52 +844,85 @@ __device__ __forceinline__ void body_update(const UpdateP& P, long long blk, lon
 	}
 }
 
-// single-block deterministic reduction of nb partial triples
-__device__ inline void reduce_parts(const double* __restrict__ part, int nb, int which, double* out, double* sh) {
-	double a = 0;
-	for (int b = threadIdx.x; b < nb; b += blockDim.x) a += part[3 * b + which];
-	a = wave_sum(a);
-	if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = a;
-	__syncthreads();
-	if (threadIdx.x == 0) {
-		double s = 0;
-		for (int q = 0; q < (int)(blockDim.x >> 6); q++) s += sh[q];
-		*out = s;
-	}
-	__syncthreads();
-}
-
+// Single-block deterministic reduction of nb partials and the scalar rule of
+// the phase.  Nothing here is work; the time is the chain of memory waits
+// between the launch and the last store, so everything is asked for at once -
+// the state's scalars, the sums and the extrema - and one barrier separates
+// the wavefronts' sums from the block's (one after another, with the state
+// read by thread 0 at the end: 4.9 us; at once: FIN_US us at 128^3).
+constexpr int kFinNT = 1024;
 __device__ __forceinline__ void body_finalize(const FinP& P, long long, long long) {
+	constexpr int NW = kFinNT / 64;
 	CgState* st = P.st;
 	const double* __restrict__ part = P.part;
 	const float* __restrict__ fpart = P.fpart;
 	const int nb = P.nb, phase = P.phase, pcNone = P.pcNone;
-	__shared__ double sh[16];
-	__shared__ double r0, r1;
-	__shared__ float smn[16], smx[16];
-	if (phase != FIN_INIT && st->done) return;
-	reduce_parts(part, nb, 0, &r0, sh);
-	if (phase == FIN_INIT || phase == FIN_RES) reduce_parts(part, nb, 1, &r1, sh);
+	__shared__ double sh0[NW], sh1[NW];
+	__shared__ float smn[NW], smx[NW];
+	const int done = st->done, iter = st->iter, maxIter = st->maxIter, useL2 = st->useL2;
+	const float sigma = st->sigma, prevNorm = st->resNorm, accuracy = st->acc;
+	const double relTol = st->relTol, bnorm2 = st->bnorm2;
+	const bool two = phase == FIN_INIT || phase == FIN_RES, extrema = phase == FIN_RES;
+	double a0 = 0, a1 = 0;
 	float mn = 3.402823466e+38f, mx = -3.402823466e+38f;
-	if (phase == FIN_RES) {
-		for (int b = threadIdx.x; b < nb; b += blockDim.x) {
-			mn = fminf(mn, fpart[2 * b]);
-			mx = fmaxf(mx, fpart[2 * b + 1]);
+	// kN partials per thread in flight (past the end one in range, not added)
+	auto gather = [&](auto twoC, auto exC) {
+		constexpr bool TWO = decltype(twoC)::value, EX = decltype(exC)::value;
+		constexpr int kN = EX ? 2 : 4;
+		for (int b0 = threadIdx.x; b0 < nb; b0 += kFinNT * kN) {
+			double v0[kN], v1[kN];
+			float f0[kN], f1[kN];
+#pragma unroll
+			for (int e = 0; e < kN; e++) {
+				const int b = min(b0 + kFinNT * e, nb - 1);
+				v0[e] = part[3 * b];
+				if (TWO) v1[e] = part[3 * b + 1];
+				if (EX) {
+					f0[e] = fpart[2 * b];
+					f1[e] = fpart[2 * b + 1];
+				}
+			}
+#pragma unroll
+			for (int e = 0; e < kN; e++) {
+				const bool ok = b0 + kFinNT * e < nb;
+				a0 = ok ? a0 + v0[e] : a0;
+				if (TWO) a1 = ok ? a1 + v1[e] : a1;
+				if (EX) {
+					mn = fminf(mn, f0[e]);
+					mx = fmaxf(mx, f1[e]);
+				}
+			}
 		}
+	};
+	if (extrema) gather(std::true_type{}, std::true_type{});
+	else if (two) gather(std::true_type{}, std::false_type{});
+	else gather(std::false_type{}, std::false_type{});
+	if (phase != FIN_INIT && done) return;
+	a0 = wave_sum(a0);
+	if (two) a1 = wave_sum(a1);
+	if (extrema) {
 		mn = wave_min(mn);
 		mx = wave_max(mx);
-		if ((threadIdx.x & 63) == 0) {
-			smn[threadIdx.x >> 6] = mn;
-			smx[threadIdx.x >> 6] = mx;
-		}
-		__syncthreads();
 	}
+	if ((threadIdx.x & 63) == 0) {
+		sh0[threadIdx.x >> 6] = a0;
+		sh1[threadIdx.x >> 6] = a1;
+		smn[threadIdx.x >> 6] = mn;
+		smx[threadIdx.x >> 6] = mx;
+	}
+	__syncthreads();
 	if (threadIdx.x != 0) return;
+	double r0 = 0, r1 = 0;
+#pragma unroll
+	for (int q = 0; q < NW; q++) {
+		r0 += sh0[q];
+		r1 += sh1[q];
+	}
 	if (phase == FIN_INIT) {
 		st->sigma = (float)r0;
 		st->bnorm2 = r1;
 		st->iter = 0;
-		st->done = st->maxIter <= 0 ? 1 : 0;
+		st->done = maxIter <= 0 ? 1 : 0;
 		st->converged = 0;
 		st->diverged = 0;
 		st->first = 1;
@@ -900,30 +933,31 @@ __device__ __forceinline__ void body_finalize(const FinP& P, long long, long lon
 	if (phase == FIN_ALPHA) {
 		const float dp = (float)r0;
 		float alpha = 0.f;
-		if (fabsf(dp) > 0.f) alpha = st->sigma / dp;
+		if (fabsf(dp) > 0.f) alpha = sigma / dp;
 		st->alpha = alpha;
 		st->first = 0;
 		return;
 	}
 	if (phase == FIN_RES) {
-		for (int q = 0; q < (int)(blockDim.x >> 6); q++) {
+#pragma unroll
+		for (int q = 0; q < NW; q++) {
 			mn = fminf(mn, smn[q]);
 			mx = fmaxf(mx, smx[q]);
 		}
-		st->iter += 1;
+		st->iter = iter + 1;
 		st->rr = r1;
 		float resNorm;
 		bool conv;
-		if (st->relTol > 0) {
-			resNorm = (float)sqrt(r1 / (st->bnorm2 > 0 ? st->bnorm2 : 1.0));
-			conv = sqrt(r1) <= st->relTol * sqrt(st->bnorm2);
+		if (relTol > 0) {
+			resNorm = (float)sqrt(r1 / (bnorm2 > 0 ? bnorm2 : 1.0));
+			conv = sqrt(r1) <= relTol * sqrt(bnorm2);
 		} else {
-			if (st->useL2) resNorm = (float)r1;
+			if (useL2) resNorm = (float)r1;
 			else resNorm = fmaxf(fabsf(mn), fabsf(mx));  // max(fabs(amin), fabs(amax))
-			conv = resNorm < st->acc;
+			conv = resNorm < accuracy;
 		}
 		st->resNorm = resNorm;
-		if (st->iter - 1 < 64) st->hist[st->iter - 1] = resNorm;
+		if (iter < 64) st->hist[iter] = resNorm;
 		if (conv) {
 			st->sigma = resNorm;
 			st->converged = 1;
@@ -932,28 +966,28 @@ __device__ __forceinline__ void body_finalize(const FinP& P, long long, long lon
 		}
 		if (pcNone) {
 			const float sigmaNew = (float)r0;
-			st->beta = sigmaNew / st->sigma;
+			st->beta = sigmaNew / sigma;
 			st->sigma = sigmaNew;
 			if (!(resNorm < 1e35f)) {
 				st->diverged = 1;
 				st->done = 1;
 				return;
 			}
-			if (st->iter >= st->maxIter) st->done = 1;
+			if (iter + 1 >= maxIter) st->done = 1;
 		}
 		return;
 	}
 	// FIN_BETA / FIN_BETA0 (preconditioned): sigmaNew = dot(z, r)
 	const float sigmaNew = (float)r0;
-	st->beta = sigmaNew / st->sigma;
+	st->beta = sigmaNew / sigma;
 	st->sigma = sigmaNew;
 	if (phase == FIN_BETA0) st->first = 1;
-	if (!(st->resNorm < 1e35f)) {
+	if (!(prevNorm < 1e35f)) {
 		st->diverged = 1;
 		st->done = 1;
 		return;
 	}
-	if (st->iter >= st->maxIter) st->done = 1;
+	if (iter >= maxIter) st->done = 1;
 }
 
 // Three consecutive floats at a 4-byte aligned address, read by one load.
@@ -1187,10 +1221,10 @@ void run_update_many(hipStream_t s, unsigned nb, WorkList items, const UpdateP* 
 	hipLaunchKernelGGL((k_many<UpdateP, body_update, kBlock>), dim3(nb), dim3(kBlock), 0, s, items, p);
 }
 void run_finalize_one(hipStream_t s, const FinP& p) {
-	hipLaunchKernelGGL((k_one<FinP, body_finalize, 1024>), dim3(1), dim3(1024), 0, s, p);
+	hipLaunchKernelGGL((k_one<FinP, body_finalize, kFinNT>), dim3(1), dim3(kFinNT), 0, s, p);
 }
 void run_finalize_many(hipStream_t s, unsigned nprob, WorkList items, const FinP* p) {
-	hipLaunchKernelGGL((k_many<FinP, body_finalize, 1024>), dim3(nprob), dim3(1024), 0, s, items, p);
+	hipLaunchKernelGGL((k_many<FinP, body_finalize, kFinNT>), dim3(nprob), dim3(kFinNT), 0, s, items, p);
 }
 void run_dot_one(hipStream_t s, unsigned nb, const DotP& p) {
 	hipLaunchKernelGGL((k_one<DotP, body_dot, kBlock>), dim3(nb), dim3(kBlock), 0, s, p);
