@@ -377,15 +377,27 @@ __device__ __forceinline__ void body_correct_velocity_wall(const CorrVelP& P, lo
 // fl(b*b) (GridDotProduct of the unpreconditioned tmp = r) and of b^2 in
 // FP64; float4 groups with a grid stride of per*256 (as body_update), the
 // n % 4 trailing cells spread the same way; one partial per block
-__global__ void __launch_bounds__(kBlock) k_cg_init(Dims d, long long per, const float* __restrict__ rhs,
-                                                    float* __restrict__ x, float* __restrict__ r, int withDot,
-                                                    double* __restrict__ part) {
+struct CgInitP {
+	Dims d;
+	long long per;
+	const float* rhs;
+	float* x;
+	float* r;
+	int withDot;
+	double* part;
+};
+__device__ __forceinline__ void body_cg_init(const CgInitP& P, long long blk, long long slot) {
 	__shared__ double sh[8];
+	const Dims& d = P.d;
+	const long long per = P.per;
+	const float* __restrict__ rhs = P.rhs;
+	float* __restrict__ x = P.x;
+	float* __restrict__ r = P.r;
 	double zr = 0, bb = 0;
 	const long long n4 = d.n >> 2;
 	const long long stride = per * kBlock;
 	const float4 zero4 = make_float4(0.f, 0.f, 0.f, 0.f);
-	for (long long v = blockIdx.x * (long long)kBlock + threadIdx.x; v < n4; v += stride) {
+	for (long long v = blk * kBlock + threadIdx.x; v < n4; v += stride) {
 		const float4 bv = reinterpret_cast<const float4*>(rhs)[v];
 		reinterpret_cast<float4*>(x)[v] = zero4;
 		reinterpret_cast<float4*>(r)[v] = bv;
@@ -395,7 +407,7 @@ __global__ void __launch_bounds__(kBlock) k_cg_init(Dims d, long long per, const
 			bb += (double)e[u] * (double)e[u];
 		}
 	}
-	for (long long c = (n4 << 2) + blockIdx.x * (long long)kBlock + threadIdx.x; c < d.n; c += stride) {
+	for (long long c = (n4 << 2) + blk * kBlock + threadIdx.x; c < d.n; c += stride) {
 		const float b = rhs[c];
 		x[c] = 0.f;
 		r[c] = b;
@@ -405,15 +417,16 @@ __global__ void __launch_bounds__(kBlock) k_cg_init(Dims d, long long per, const
 	const double s0 = block_sum(zr, sh);
 	const double s1 = block_sum(bb, sh);
 	if (threadIdx.x == 0) {
-		part[3 * blockIdx.x] = withDot ? s0 : 0.0;
-		part[3 * blockIdx.x + 1] = s1;
-		part[3 * blockIdx.x + 2] = 0.0;
+		P.part[3 * slot] = P.withDot ? s0 : 0.0;
+		P.part[3 * slot + 1] = s1;
+		P.part[3 * slot + 2] = 0.0;
 	}
 }
 
-// CgState of a new solve (set on the device: no host copy to wait for)
+// CgState of each block's new solve (set on the device: no host copy to wait for)
 __global__ void k_cg_state_init(CgState* st, float acc, int maxIter, int useL2, double relTol) {
 	if (threadIdx.x != 0) return;
+	st += blockIdx.x;
 	CgState z;
 	memset(&z, 0, sizeof(z));
 	z.acc = acc;
@@ -1780,6 +1793,7 @@ struct CgRun {
 		FinP p{st, dpart, fpart, nb, phase, pcNone ? 1 : 0};
 		return p;
 	}
+	CgInitP initP() const { return CgInitP{s->d, per, rhs, x, r, pcNone ? 1 : 0, dpart}; }
 	TrueResP trueResP() const { return TrueResP{s->d, tiles_for(s->d, kLightKZ), code, rhs, x, dpart, scale}; }
 	TrueRedP trueRedP() const { return TrueRedP{st, dpart, (int)tiles_for(s->d, kLightKZ).count()}; }
 };
@@ -1879,8 +1893,7 @@ static int precondition(CgRun& R);
 // doInit of the general kernels: x = 0, r = b, ||b||, sigma = dot(r, r)
 static void cg_init(CgRun& R) {
 	Scene* s = R.s;
-	hipLaunchKernelGGL(k_cg_init, dim3(R.nbU), dim3(kBlock), 0, s->stream, s->d, R.per, (const float*)R.rhs, R.x, R.r,
-	                   R.pcNone ? 1 : 0, R.dpart);
+	launch_one<CgInitP, body_cg_init, kBlock>(s->stream, R.nbU, R.initP());
 	run_finalize_one(s->stream, FinP{R.st, R.dpart, R.fpart, (int)R.nbU, FIN_INIT, 0});
 }
 
@@ -2271,8 +2284,7 @@ static void cg_verify(CgRun& R, double target) {
 }
 
 // after the scene stream has drained: statistics and the divergence error
-static void cg_finish_collect(CgRun& R, mfx_solve_stats* stats) {
-	const CgState* hs = (const CgState*)R.s->hscal;
+static void cg_finish_collect(CgRun& R, mfx_solve_stats* stats, const CgState* hs) {
 	const double bb = hs->bnorm2, rr = hs->trueRR;
 	if (stats) {
 		stats->iterations = hs->iter;
@@ -2332,16 +2344,17 @@ static void cg_drive(CgRun& R, double target, mfx_solve_stats* stats) {
 	}
 	cg_verify(R, target);
 	cg_release(R);
-	cg_finish_collect(R, stats);
+	cg_finish_collect(R, stats, (const CgState*)R.s->hscal);
 }
 
 // GridCg without preconditioner over a scaled Laplace matrix (the other
 // GridCg clients): kind 0 builds cgSolveDiffusion's matrix code, kind 1 the
 // pressure matrix of the flags (cgSolveWE); x is cleared by doInit and
 // solved for rhs.  maxIter = (int)(cgMaxIterFac * max size) * (4 in 2D).
-static void solve_scaled(Scene* s, Grid* flags, float* rhs, float* x, int kind, float scale, float cgAccuracy,
-                         float cgMaxIterFac, mfx_solve_stats* stats) {
-	CgRun R;
+// Shape and options of such a run (no buffers); nsys systems share the
+// scene's partial sums.
+static size_t scaled_shape(CgRun& R, Scene* s, Grid* flags, float* rhs, float* x, float scale, float cgAccuracy,
+                           float cgMaxIterFac, int nsys) {
 	R.t0 = std::chrono::steady_clock::now();
 	R.s = s;
 	R.flags = flags;
@@ -2355,8 +2368,8 @@ static void solve_scaled(Scene* s, Grid* flags, float* rhs, float* x, int kind, 
 	R.nbT = (unsigned)R.t.count();
 	R.nbF = flat_count(d.n);
 	R.nbU = (unsigned)update_tiles(d, &R.per);
-	const unsigned nbMax = std::max(R.nbT, R.nbF);
-	s->ensurePartials(3 * (size_t)nbMax + 16, 2 * (size_t)nbMax + 16);
+	const size_t per = (size_t)std::max(R.nbT, R.nbF) + 8;
+	s->ensurePartials(3 * per * (size_t)nsys + 16, 2 * per * (size_t)nsys + 16);
 	R.dpart = s->dpart;
 	R.fpart = s->fpart;
 	int mx = d.nx > d.ny ? d.nx : d.ny;
@@ -2367,26 +2380,182 @@ static void solve_scaled(Scene* s, Grid* flags, float* rhs, float* x, int kind, 
 	R.scaled = 1;
 	R.scale = scale;
 	R.st = (CgState*)s->dscal;
-	hipLaunchKernelGGL(k_cg_state_init, dim3(1), dim3(64), 0, s->stream, R.st, cgAccuracy, R.maxIter, 0, 0.0);
 	if (!s->code) MFX_HIP(hipMalloc((void**)&s->code, (size_t)d.n));
 	R.code = s->code;
-	const Tiles tc = tiles_for(d, kLightKZ);
-	if (kind == 0)
-		hipLaunchKernelGGL(k_build_code_diff, dim3((unsigned)tc.count()), dim3(kBlock), 0, s->stream, d, tc,
-		                   flags->f8, R.code);
-	else
-		hipLaunchKernelGGL(k_build_code, dim3((unsigned)tc.count()), dim3(kBlock), 0, s->stream, d, tc, flags->f8,
-		                   R.code, (const CgState*)R.st);
 	R.nbM = (unsigned)matvec_tiles(d, &R.kchunk, true);
 	R.npM = (int)zm_dot_parts(d, kMvTY);
+	R.launched = 0;
+	return per;
+}
+static void scaled_code(const CgRun& R, int kind) {
+	Scene* s = R.s;
+	const Tiles tc = tiles_for(s->d, kLightKZ);
+	if (kind == 0)
+		hipLaunchKernelGGL(k_build_code_diff, dim3((unsigned)tc.count()), dim3(kBlock), 0, s->stream, s->d, tc,
+		                   R.flags->f8, R.code);
+	else
+		hipLaunchKernelGGL(k_build_code, dim3((unsigned)tc.count()), dim3(kBlock), 0, s->stream, s->d, tc,
+		                   R.flags->f8, R.code, (const CgState*)R.st);
+}
+static void solve_scaled(Scene* s, Grid* flags, float* rhs, float* x, int kind, float scale, float cgAccuracy,
+                         float cgMaxIterFac, mfx_solve_stats* stats) {
+	CgRun R;
+	scaled_shape(R, s, flags, rhs, x, scale, cgAccuracy, cgMaxIterFac, 1);
+	hipLaunchKernelGGL(k_cg_state_init, dim3(1), dim3(64), 0, s->stream, R.st, cgAccuracy, R.maxIter, 0, 0.0);
+	scaled_code(R, kind);
 	R.r = s->getReal();
 	R.pa = s->getReal();
 	R.pb = s->getReal();
 	R.q = s->getReal();
 	R.z = R.r;
-	R.launched = 0;
 	if (!cg_try_resident(R)) cg_init(R);
 	cg_drive(R, (double)cgAccuracy, stats);
+}
+
+// Several systems of one shape in a launch: blockIdx.y is the system.  Each
+// runs the same workgroups on the same tiles as alone, so its result is the
+// same bit for bit.
+constexpr int kJointMax = 3;
+template <typename P>
+struct JointP {
+	P p[kJointMax];
+};
+template <typename P, void (*BODY)(const P&, long long, long long), int NT>
+__global__ void __launch_bounds__(NT) k_joint(JointP<P> q) {
+	const long long t = xcd_tile(blockIdx.x, gridDim.x);
+	BODY(q.p[blockIdx.y], t, t);
+}
+template <typename P, void (*BODY)(const P&, long long, long long), int NT, typename F>
+static void launch_joint(hipStream_t q, long long nb, const CgRun* R, int nc, F param) {
+	JointP<P> a{};
+	for (int c = 0; c < nc; c++) a.p[c] = param(R[c]);
+	hipLaunchKernelGGL((k_joint<P, BODY, NT>), dim3((unsigned)nb, (unsigned)nc), dim3(NT), 0, q, a);
+}
+
+// The components of a Vec3 / MAC diffusion as one sequence of launches:
+// their matrix is the same, and up to some millions of cells an iteration of
+// one component is four launches of 3 to 12 us that leave most of the GPU
+// idle.  rhs: the components, cstride apart, copied from u before.  Returns
+// false, with nothing queued, where the components are solved one by one:
+// grids of the one-kernel CG, larger grids, and when the further buffers
+// cannot be had.  The line: the systems' vectors have to stay in the 256 MB
+// last-level cache.  Three components, one by one / together: 84^3 984 / 483
+// us, 144^3 1680 / 1258, 176^3 2317 / 2331, 202^3 3310 / 4253.
+constexpr long long kJointCells = 3ll << 22;  // of all components
+static bool joint_diffusion(const Dims& d, int nc) { return nc > 1 && nc * d.n <= kJointCells && !cg_resident_plan(d).V; }
+static bool solve_diffusion_joint(Scene* s, Grid* flags, float* rhs, float* const* u, int nc, float alpha,
+                                  float cgAccuracy, float cgMaxIterFac, mfx_solve_stats* stats) {
+	const Dims& d = s->d;
+	if (!joint_diffusion(d, nc)) return false;
+	float* buf[4 * kJointMax] = {};
+	auto give = [&]() {
+		for (float* b : buf)
+			if (b) s->putReal(b);
+	};
+	try {
+		for (int i = 0; i < 4 * nc; i++) buf[i] = s->getReal();
+	} catch (...) {
+		(void)hipGetLastError();
+		give();
+		return false;
+	}
+	CgRun R[kJointMax];
+	const CgState* hs = (const CgState*)s->hscal;
+	static_assert(kJointMax * sizeof(CgState) <= 4096, "the scene's scalar block");
+	const hipStream_t q = s->stream;
+	try {
+		for (int c = 0; c < nc; c++) {
+			const size_t per = scaled_shape(R[c], s, flags, rhs + c * s->cstride, u[c], alpha, cgAccuracy, cgMaxIterFac, nc);
+			R[c].dpart += 3 * per * (size_t)c;
+			R[c].fpart += 2 * per * (size_t)c;
+			R[c].st += c;
+			R[c].r = buf[4 * c];
+			R[c].z = buf[4 * c];
+			R[c].pa = buf[4 * c + 1];
+			R[c].pb = buf[4 * c + 2];
+			R[c].q = buf[4 * c + 3];
+		}
+		const unsigned nbM = R[0].nbM, nbU = R[0].nbU;
+		const int maxIter = R[0].maxIter, npM = R[0].npM;
+		const long long nLight = tiles_for(d, kLightKZ).count();
+		auto fin = [&](int nb, int phase) {
+			launch_joint<FinP, body_finalize, kFinNT>(q, 1, R, nc, [&](const CgRun& r) { return r.fin(nb, phase); });
+		};
+		auto states = [&]() { MFX_HIP(hipMemcpyAsync(s->hscal, s->dscal, sizeof(CgState) * (size_t)nc, hipMemcpyDeviceToHost, q)); };
+		hipLaunchKernelGGL(k_cg_state_init, dim3((unsigned)nc), dim3(64), 0, q, R[0].st, cgAccuracy, maxIter, 0, 0.0);
+		scaled_code(R[0], 0);
+		launch_joint<CgInitP, body_cg_init, kBlock>(q, nbU, R, nc, [](const CgRun& r) { return r.initP(); });
+		fin((int)nbU, FIN_INIT);
+		if (!s->evState) MFX_HIP(hipEventCreateWithFlags(&s->evState, hipEventDisableTiming));
+		// iterations the slowest system still needs (as cg_iterate_finish)
+		auto left = [&]() {
+			int most = 0;
+			for (int c = 0; c < nc; c++) {
+				const int l = cg_iters_left(hs[c], (double)cgAccuracy, true);
+				if (l < 0) return -1;
+				most = std::max(most, l);
+			}
+			return most;
+		};
+		auto allDone = [&]() {
+			for (int c = 0; c < nc; c++)
+				if (!hs[c].done) return false;
+			return true;
+		};
+		int plan = 4, launched = 0;
+		while (true) {
+			const int nIt = std::min(plan, maxIter - launched);
+			for (int it = 0; it < nIt; it++) {
+				const bool odd = (launched & 1) != 0;
+				{
+					KtScope kt("cg_matvec", q);
+					launch_joint<MatvecP, body_matvec<kMvTY, true>, 64 * kMvTY>(
+					    q, nbM, R, nc, [&](const CgRun& r) { return r.mvp(odd); });
+				}
+				fin(npM, FIN_ALPHA);
+				{
+					KtScope kt("cg_update", q);
+					launch_joint<UpdateP, body_update, kBlock>(q, nbU, R, nc, [&](const CgRun& r) { return r.upd(odd); });
+				}
+				fin((int)nbU, FIN_RES);
+				launched++;
+				if (it == nIt - 2) {
+					states();
+					MFX_HIP(hipEventRecord(s->evState, q));
+				}
+			}
+			if (nIt >= 2 && launched < maxIter) {
+				MFX_HIP(hipEventSynchronize(s->evState));
+				const int l = left();
+				if (l < 0 || l > 1) {
+					plan = cg_plan(l < 0 ? l : l - 1, launched);
+					continue;
+				}
+			}
+			launch_joint<TrueResP, body_true_residual<false, true>, kBlock>(q, nLight, R, nc,
+			                                                               [](const CgRun& r) { return r.trueResP(); });
+			launch_joint<TrueRedP, body_reduce_true_rr, 1024>(q, 1, R, nc, [](const CgRun& r) { return r.trueRedP(); });
+			states();
+			sync(s);
+			if (allDone() || launched >= maxIter) break;
+			plan = cg_plan(left(), launched);
+		}
+	} catch (...) {
+		give();
+		throw;
+	}
+	give();
+	for (int c = 0; c < nc; c++) {
+		try {
+			cg_finish_collect(R[c], stats, hs + c);
+		} catch (...) {
+			// a component that diverges ends the call before the next ones: as they were
+			for (int e = c + 1; e < nc; e++)
+				(void)hipMemcpyAsync(u[e], R[e].rhs, sizeof(float) * (size_t)d.n, hipMemcpyDeviceToDevice, q);
+			throw;
+		}
+	}
+	return true;
 }
 
 static void correct_velocity(Scene* s, Grid* flags, Grid* vel, const float* pressure, const BndDev* bnd = nullptr) {
@@ -2914,7 +3083,8 @@ static void solve_batch(const std::vector<Grid*>& vel, const std::vector<Grid*>&
 		std::vector<std::string> errs((size_t)P);
 		for (int i = 0; i < P; i++) {
 			try {
-				cg_finish_collect(R[(size_t)i], stats ? &stats[i] : nullptr);
+				cg_finish_collect(R[(size_t)i], stats ? &stats[i] : nullptr,
+				                  (const CgState*)R[(size_t)i].s->hscal);
 			} catch (const Error& e) {
 				errs[(size_t)i] = e.what();
 			}
@@ -3281,16 +3451,31 @@ int mfx_cg_solve_diffusion(const mfx_grid* flags, mfx_grid* grid, float alpha, f
 	          "cgSolveDiffusion: Grid Type is not supported (only Real, Vec3, MAC, or Levelset)");
 	Scene* s = f->s;
 	const size_t bytes = sizeof(float) * (size_t)s->d.n;
+	// Vec3 / MAC grids: every component (two in 2D) with the same matrix;
+	// a component of the SoA grid is itself a Real grid, so getComponent
+	// and setComponent are the solve's own input and output
+	const int nc = g->isVec() ? (s->d.is3d ? 3 : 2) : 1;
+	float* u[kJointMax];
+	for (int c = 0; c < nc; c++) u[c] = g->comp(c);
+	if (joint_diffusion(s->d, nc)) {
+		float* rhs3 = s->getVec();
+		bool ok = false;
+		try {
+			for (int c = 0; c < nc; c++)
+				MFX_HIP(hipMemcpyAsync(rhs3 + c * s->cstride, u[c], bytes, hipMemcpyDeviceToDevice, s->stream));
+			ok = solve_diffusion_joint(s, f, rhs3, u, nc, alpha, cgAccuracy, cgMaxIterFac, stats);
+		} catch (...) {
+			s->putVec(rhs3);
+			throw;
+		}
+		s->putVec(rhs3);
+		if (ok) return 0;
+	}
 	float* rhs = s->getReal();
 	try {
-		// Vec3 / MAC grids: every component (two in 2D) with the same matrix;
-		// a component of the SoA grid is itself a Real grid, so getComponent
-		// and setComponent are the solve's own input and output
-		const int nc = g->isVec() ? (s->d.is3d ? 3 : 2) : 1;
 		for (int c = 0; c < nc; c++) {
-			float* u = g->comp(c);
-			MFX_HIP(hipMemcpyAsync(rhs, u, bytes, hipMemcpyDeviceToDevice, s->stream));
-			solve_scaled(s, f, rhs, u, 0, alpha, cgAccuracy, cgMaxIterFac, stats);
+			MFX_HIP(hipMemcpyAsync(rhs, u[c], bytes, hipMemcpyDeviceToDevice, s->stream));
+			solve_scaled(s, f, rhs, u[c], 0, alpha, cgAccuracy, cgMaxIterFac, stats);
 		}
 	} catch (...) {
 		s->putReal(rhs);

@@ -78,3 +78,45 @@ def test_cg_solve_we(manta, oracle, rng, shape, crank):
     assert np.abs(out.toNumpy() - r_out).max() <= 4 * acc
     assert np.array_equal(ut.toNumpy(), out.toNumpy())
     assert np.array_equal(utm1.toNumpy(), ut0)
+
+
+@pytest.mark.parametrize("shape,kind,empty", [((83, 85, 81), "mac", False), ((83, 85, 81), "vec", True),
+                                              ((1031, 530, 1), "mac", True), ((129, 64, 66), "vec", False)])
+def test_diffusion_components_together(manta, oracle, rng, shape, kind, empty):
+    """Above the one-kernel CG's sizes the components of a vector diffusion
+    share their launches: bit for bit what each gives as a Real grid, with the
+    last one's statistics."""
+    n = int(np.prod(shape))
+    flags = _flags(oracle, rng, shape, empty)
+    val = rng.uniform(-1, 1, (n, 3)).astype(np.float32) * np.array([1.0, 0.01, 30.0], np.float32)
+    sc = GpuScene(manta, shape)
+    f = sc.flags(flags)
+    g = sc.vec(val) if kind == "vec" else sc.mac(val)
+    manta.cgSolveDiffusion(flags=f, grid=g, alpha=0.6, cgMaxIterFac=2.0, cgAccuracy=1e-5)
+    st = dict(sc.s._solve_stats)
+    got = g.toNumpy()
+    comps = 2 if shape[2] == 1 else 3
+    for c in range(comps):
+        r = sc.real(val[:, c].copy())
+        manta.cgSolveDiffusion(flags=f, grid=r, alpha=0.6, cgMaxIterFac=2.0, cgAccuracy=1e-5)
+        np.testing.assert_array_equal(got[:, c], r.toNumpy().ravel(), err_msg=str(c))
+    one = sc.s._solve_stats
+    for key in ("iterations", "resNorm", "relResidual", "maxIter", "converged"):
+        assert st[key] == one[key], key
+    np.testing.assert_array_equal(got[:, comps:], val[:, comps:])
+
+
+def test_diffusion_components_diverge(manta, oracle, rng):
+    """A component that diverges ends the call; the later ones keep their
+    values, as when they are solved one after another."""
+    shape = (83, 85, 81)
+    n = int(np.prod(shape))
+    val = rng.uniform(-1, 1, (n, 3)).astype(np.float32)
+    sc = GpuScene(manta, shape)
+    f, g = sc.flags(_flags(oracle, rng, shape, False)), sc.vec(val)
+    r = sc.real(val[:, 0].copy())
+    with pytest.raises(RuntimeError, match="diverged"):
+        manta.cgSolveDiffusion(flags=f, grid=r, alpha=3e38, cgMaxIterFac=2.0, cgAccuracy=1e-5)
+    with pytest.raises(RuntimeError, match="diverged"):
+        manta.cgSolveDiffusion(flags=f, grid=g, alpha=3e38, cgMaxIterFac=2.0, cgAccuracy=1e-5)
+    np.testing.assert_array_equal(g.toNumpy()[:, 1:], val[:, 1:])
