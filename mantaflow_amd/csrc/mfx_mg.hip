@@ -552,17 +552,8 @@ struct __attribute__((packed, aligned(4))) FTriple {
 // row have 2i-1 != x0 and pick their values at a shifted slot.  Fine levels
 // narrower than 3 vertices in x take one load per value.
 template <bool IS3D>
-__device__ __forceinline__ void body_restrict(const RestrictP& P, long long blk, long long) {
-	const CgState* __restrict__ st = P.st;
-	const LvDev& c = P.c;
-	const LvDev& f = P.f;
-	const uint8_t* __restrict__ ctype = P.ctype;
-	const float* __restrict__ rf = P.rf;
-	float* __restrict__ bc = P.bc;
-	if (st->done) return;
-	const VtxPos p = lc_vertex(c, blk);
-	if (!p.in) return;
-	const int i = p.i, j = p.j, k = p.k, v = p.v;
+__device__ __forceinline__ float restrict_value(const LvDev& f, const float* __restrict__ rf,
+                                                const uint8_t* __restrict__ ctype, int v, int i, int j, int k) {
 	float sum = 0.f;
 	if (f.nx >= 3) {
 		constexpr int NZ = IS3D ? 3 : 1;
@@ -593,8 +584,7 @@ __device__ __forceinline__ void body_restrict(const RestrictP& P, long long blk,
 			const int ux = 2 * i + ex - 1, uy = 2 * j + ey - 1, uz = 2 * k + (IS3D ? ez - 1 : 0);
 			if (kx[ex] && ky[ey] && kz[ez]) sum += wgt(ux, uy, uz) * val;
 		}
-		bc[v] = ct ? sum : 0.f;
-		return;
+		return ct ? sum : 0.f;
 	}
 	if (ctype[v]) {
 		// branch-free: per-axis offsets of the fine coordinates 2V-1..2V+1
@@ -628,7 +618,14 @@ __device__ __forceinline__ void body_restrict(const RestrictP& P, long long blk,
 			if (ok[e]) sum += wgt(ux, uy, uz) * rv[e];
 		}
 	}
-	bc[v] = sum;
+	return sum;
+}
+template <bool IS3D>
+__device__ __forceinline__ void body_restrict(const RestrictP& P, long long blk, long long) {
+	if (P.st->done) return;
+	const VtxPos p = lc_vertex(P.c, blk);
+	if (!p.in) return;
+	P.bc[p.v] = restrict_value<IS3D>(P.f, P.rf, P.ctype, p.v, p.i, p.j, p.k);
 }
 
 // r = b - A x on a coarse level (0 on inactive vertices)
@@ -1382,8 +1379,8 @@ constexpr int kSmoothNT = 512;
 // coarse parents of the brick are staged in LDS.  The stencil sum runs as
 // three fused multiply-add chains, one per z layer.  Vertex indices are
 // 32-bit (coarse levels hold fewer than 2^31 vertices).
-template <bool IS3D, typename AT, bool POST>
-__device__ __forceinline__ void body_smooth(const SmoothP& P, long long blk, long long) {
+template <bool IS3D, typename AT, bool POST, bool RESTRICT>
+__device__ __forceinline__ void smooth_tile(const SmoothP& P, const RestrictP* R, long long blk) {
 	const CgState* __restrict__ st = P.st;
 	const LvDev& c = P.c;
 	const AT* __restrict__ A = (const AT*)P.A;
@@ -1419,7 +1416,13 @@ __device__ __forceinline__ void body_smooth(const SmoothP& P, long long blk, lon
 	const bool valid = gx < c.nx && gy < c.ny && gz < c.nz;
 	const int v = valid ? gx + sy * gy + sz * gz : 0;
 	const uint8_t tl = type[v];
-	const float bv = b[v];
+	// RESTRICT: the right-hand side is restricted here instead of by a launch
+	// of its own, and stored for the residual and the way up
+	float bv;
+	if (RESTRICT) {
+		bv = restrict_value<IS3D>(R->f, R->rf, type, v, valid ? gx : 0, valid ? gy : 0, valid ? gz : 0);
+		if (valid) R->bc[v] = bv;
+	} else bv = b[v];
 	// post-smoothing: the region's old iterate and types, asked for before
 	// anything waits
 	constexpr int NIT = (RN + kSmoothNT - 1) / kSmoothNT;
@@ -1539,6 +1542,18 @@ __device__ __forceinline__ void body_smooth(const SmoothP& P, long long blk, lon
 		__syncthreads();
 	}
 	if (valid) xout[v] = xs[me];
+}
+template <bool IS3D, typename AT, bool POST>
+__device__ __forceinline__ void body_smooth(const SmoothP& P, long long blk, long long) {
+	smooth_tile<IS3D, AT, POST, false>(P, nullptr, blk);
+}
+struct RestrictSmoothP {
+	RestrictP r;
+	SmoothP s;
+};
+template <bool IS3D, typename AT>
+__device__ __forceinline__ void body_restrict_smooth(const RestrictSmoothP& P, long long blk, long long) {
+	smooth_tile<IS3D, AT, false, true>(P.s, &P.r, blk);
 }
 
 __device__ __forceinline__ void body_fill(const FillP& P, long long blk, long long) {
@@ -1963,6 +1978,12 @@ MgHierarchy::Steps MgHierarchy::steps(const Dims& d, const uint8_t* code, const 
 	return S_;
 }
 
+// Levels of at most this many smoother bricks restrict inside the smoother
+// (single solves).  There a restriction is a launch of 3 us and its gap; on
+// larger levels the smoother's colour order of vertices costs the rows' loads
+// more than the launch.  Two launches / fused: 17^3 and 33^3 9.3 / 6.5 us,
+// 65^3 (867 bricks) 12.5 / 10.1, 129^3 (5445) 48.3 / 49.9.
+constexpr long long kFuseBricks = 1024;
 int MgHierarchy::vcycle(Scene* s, const uint8_t* code, const float* r, float* z, const CgState* st) {
 	const Dims& d = s->d;
 	const Steps S_ = steps(d, code, r, z, st, s->dpart, true);
@@ -1981,22 +2002,25 @@ int MgHierarchy::vcycle(Scene* s, const uint8_t* code, const float* r, float* z,
 	const int nlv = (int)S_.lv.size();
 	for (int i = 0; i < nlv; i++) {
 		const Steps::Level& v = S_.lv[i];
-		if (is3d) launch_one<RestrictP, body_restrict<true>, 256>(q, v.tiles, v.restrict_);
-		else launch_one<RestrictP, body_restrict<false>, 256>(q, v.tiles, v.restrict_);
-		if (i == nlv - 1) break;
-		if (is3d && bf) {
-			launch_one<SmoothP, body_smooth<true, uint16_t, false>, kSmoothNT>(q, v.blkTiles, v.pre);
-			launch_one<ResidP, body_resid<true, uint16_t>, 256>(q, v.tiles, v.resid);
-		} else if (is3d) {
-			launch_one<SmoothP, body_smooth<true, float, false>, kSmoothNT>(q, v.blkTiles, v.pre);
-			launch_one<ResidP, body_resid<true, float>, 256>(q, v.tiles, v.resid);
-		} else if (bf) {
-			launch_one<SmoothP, body_smooth<false, uint16_t, false>, kSmoothNT>(q, v.blkTiles, v.pre);
-			launch_one<ResidP, body_resid<false, uint16_t>, 256>(q, v.tiles, v.resid);
-		} else {
-			launch_one<SmoothP, body_smooth<false, float, false>, kSmoothNT>(q, v.blkTiles, v.pre);
-			launch_one<ResidP, body_resid<false, float>, 256>(q, v.tiles, v.resid);
+		const bool last = i == nlv - 1, fused = !last && v.blkTiles <= kFuseBricks;
+		if (!fused) {
+			if (is3d) launch_one<RestrictP, body_restrict<true>, 256>(q, v.tiles, v.restrict_);
+			else launch_one<RestrictP, body_restrict<false>, 256>(q, v.tiles, v.restrict_);
 		}
+		if (last) break;
+		auto down = [&](auto d3, auto at) {
+			constexpr bool D = decltype(d3)::value;
+			using AT = decltype(at);
+			if (fused)
+				launch_one<RestrictSmoothP, body_restrict_smooth<D, AT>, kSmoothNT>(q, v.blkTiles,
+				                                                                    RestrictSmoothP{v.restrict_, v.pre});
+			else launch_one<SmoothP, body_smooth<D, AT, false>, kSmoothNT>(q, v.blkTiles, v.pre);
+			launch_one<ResidP, body_resid<D, AT>, 256>(q, v.tiles, v.resid);
+		};
+		if (is3d && bf) down(std::true_type{}, uint16_t{});
+		else if (is3d) down(std::true_type{}, float{});
+		else if (bf) down(std::false_type{}, uint16_t{});
+		else down(std::false_type{}, float{});
 	}
 	launch_one<CoarsestP, body_coarsest, 256>(q, coarsest_tiles(nc), S_.coarsest);
 	for (int i = nlv - 2; i >= 0; i--) {

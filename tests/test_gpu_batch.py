@@ -72,3 +72,20 @@ def test_batch_rejects_shared_solver(manta, oracle):
     g, f, v, p = make_problem(manta, oracle, (16, 16, 16), 0.0, 1)
     with pytest.raises(RuntimeError, match="own solver"):
         manta.solvePressureBatch([(v, p, f), (v, p, f)])
+
+
+@pytest.mark.parametrize("shape,frac", [((150, 150, 40), 0.1), ((140, 133, 150), 0.0), ((150, 149, 152), 0.05),
+                                        ((259, 66, 5), 0.0), ((515, 387, 1), 0.1)])
+def test_single_fused_restriction_equals_batch(manta, oracle, shape, frac):
+    """A single solve restricts inside the smoother on levels of up to 1024
+    bricks, a batch in launches of its own: the same bits with the first
+    level on either side of that line, thin, flat and in 2D."""
+    kw = dict(preconditioner=manta.PcMGStatic, cgAccuracy=1e-4)
+    g1, f1, v1, p1 = make_problem(manta, oracle, shape, frac, 7)
+    g2, f2, v2, p2 = make_problem(manta, oracle, shape, frac, 7)
+    manta.solvePressure(flags=f1, vel=v1, pressure=p1, **kw)
+    manta.solvePressureBatch([(v2, p2, f2)], **kw)
+    s1, s2 = manta.lastSolveStats(g1.s), manta.lastSolveStats(g2.s)
+    assert s1["converged"] and s1["iterations"] == s2["iterations"]
+    np.testing.assert_array_equal(p1.toNumpy(), p2.toNumpy())
+    np.testing.assert_array_equal(v1.toNumpy(), v2.toNumpy())
