@@ -215,9 +215,8 @@ def bench_batched(manta, n2d=32, n3d=32):
     """64 uneven pressure problems: one batched solve vs the problems solved
     one after another on the plain path (same inputs, rel. residual 1e-4).
     The batch is solved ten times untimed (the plane-chunk autotuner's eight
-    trials, then the chosen policy's queued launches and the capture of its
-    two-iteration graph) and the median of three graph replays is
-    reported."""
+    trials, then the chosen policy) and the median of three further solves
+    is reported."""
     from mantaflow_amd import workloads
     probs = workloads.batched_problems(n2d, n3d)
     kw = dict(cgAccuracy=1e-4, preconditioner=manta.PcMGStatic)
