@@ -60,7 +60,7 @@ float* Scene::getReal() {
 	}
 	float* p = nullptr;
 	MFX_HIP(hipMalloc(&p, sizeof(float) * (size_t)d.n));
-	owned.push_back(p);
+	owned.insert(p);
 	return p;
 }
 void Scene::putReal(float* p) { freeReal.push_back(p); }
@@ -72,7 +72,7 @@ float* Scene::getVec() {
 	}
 	float* p = nullptr;
 	MFX_HIP(hipMalloc(&p, sizeof(float) * 3 * cstride));
-	owned.push_back(p);
+	owned.insert(p);
 	return p;
 }
 void Scene::putVec(float* p) { freeVec.push_back(p); }
@@ -149,6 +149,7 @@ Grid* make_grid(Scene* s, int type) {
 		delete g;
 		throw;
 	}
+	s->owned.insert(g->data);
 	s->grids.push_back(g);
 	return g;
 }
@@ -156,6 +157,7 @@ Grid* make_grid(Scene* s, int type) {
 void free_grid(Grid* g) {
 	Scene* s = g->s;
 	hipStreamSynchronize(s->stream);
+	s->owned.erase(g->data);
 	if (g->data) hipFree(g->data);
 	if (g->f8) hipFree(g->f8);
 	if (g->olist) hipFree(g->olist);
@@ -1009,6 +1011,13 @@ int mfx_grid_swap(mfx_grid* x, mfx_grid* y) {
 	          "Grid::swap(): Grid dimensions mismatch.");
 	MFX_CHECK(!a->external && !b->external, "Grid::swap(): Cannot swap if one grid stores externalData.");
 	MFX_CHECK(a->isVec() == b->isVec() && a->isFlags() == b->isFlags(), "Grid::swap(): grid types differ.");
+	if (a->s != b->s) {
+		// the buffers change hands between two scenes
+		a->s->owned.erase(a->data);
+		b->s->owned.erase(b->data);
+		a->s->owned.insert(b->data);
+		b->s->owned.insert(a->data);
+	}
 	std::swap(a->data, b->data);
 	std::swap(a->f8, b->f8);
 	if (a->isFlags()) {

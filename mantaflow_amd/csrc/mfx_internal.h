@@ -8,6 +8,7 @@
 #include <cstdio>
 #include <map>
 #include <memory>
+#include <set>
 #include <stdexcept>
 #include <string>
 #include <vector>
@@ -85,7 +86,10 @@ struct Scene {
 	// pooled temporaries (mirror of FluidSolver::GridStorage)
 	std::vector<float*> freeReal;
 	std::vector<float*> freeVec;
-	std::vector<void*> owned;
+	// every pooled buffer and every grid's data, whoever holds it now:
+	// advection makes a pooled buffer a grid's data and puts the old data into
+	// the pool.  Freed once, by free_grid or with the scene.
+	std::set<void*> owned;
 	// small device workspace for reductions
 	double* dpart = nullptr;    // block partials (doubles)
 	size_t dpartCap = 0;
