@@ -9,6 +9,7 @@
 
 #include "mfx_internal.h"
 #include "mfx_mg.h"
+#include "mfx_resident.h"
 
 namespace mfx {
 
@@ -32,7 +33,10 @@ void set_last_error(const std::string& s) { g_err = s; }
 // scene
 // ---------------------------------------------------------------------------
 Scene::~Scene() {
-	if (stream) hipStreamSynchronize(stream);
+	if (stream) {
+		hipStreamSynchronize(stream);
+		cg_resident_forget(device, stream);
+	}
 	mgStatic.reset();
 	mgDyn.reset();
 	mgMic.reset();

@@ -74,6 +74,7 @@ struct ResWords {
 	unsigned long long* words = nullptr;
 	size_t count = 0;
 	unsigned next = 0;  // 0: the words have not been cleared
+	int rest = 0;       // solves that still run on the general kernels after one gave up
 };
 
 struct Scene {

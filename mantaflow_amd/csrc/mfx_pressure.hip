@@ -1766,6 +1766,7 @@ struct CgRun {
 	uint8_t* code = nullptr;
 	ResWords* res = nullptr;  // exchange words of the one-kernel CG (the scene's when pooled)
 	bool resident = false;    // the iterations ran, or run, as one kernel
+	ResWords& words() const { return res ? *res : s->res; }
 	int pc = 0, maxIter = 0;
 	bool pcNone = true;
 	MgHierarchy* mg = nullptr;
@@ -1900,15 +1901,24 @@ static void cg_init(CgRun& R) {
 // Unpreconditioned solves of grids that fit the one-kernel CG: doInit and
 // every iteration as one launch.  Returns false where the general kernels
 // have to run.  At most 5 s may pass before a workgroup gives up waiting for
-// another (cg_verify then runs the solve on the general kernels).
+// another; cg_verify then runs the solve on the general kernels, and so do the
+// next kResRest solves on the same exchange words, so that a device shared
+// with something that keeps the workgroups apart costs that wait once in so
+// many solves and not in each.
 constexpr long long kResWaitTicks = 5ll * 100000000ll;
+constexpr int kResRest = 1000;
 static long long g_res_wait = kResWaitTicks;
+static std::atomic<long long> g_res_ran{0}, g_res_gaveup{0};
 static bool cg_try_resident(CgRun& R) {
 	Scene* s = R.s;
 	if (!R.pcNone || R.gA0 || R.o.trueResidualEvery > 0) return false;
 	const ResPlan pl = cg_resident_plan(s->d);
 	if (!pl.V) return false;
-	ResWords& w = R.res ? *R.res : s->res;
+	ResWords& w = R.words();
+	if (pl.wg > 1 && w.rest > 0) {
+		w.rest--;
+		return false;
+	}
 	if (pl.wg > 1 && !w.words) {
 		if (R.res) return false;
 		w.count = kResSlotWords + pl.words;
@@ -1928,8 +1938,9 @@ static bool cg_try_resident(CgRun& R) {
 	p.limit = g_res_wait;
 	{
 		KtScope kt("cg_resident", s->stream);
-		cg_resident_run(s->stream, pl, p);
+		if (!cg_resident_run(s->device, s->stream, pl, p)) return false;
 	}
+	g_res_ran++;
 	R.resident = true;
 	return true;
 }
@@ -2267,6 +2278,8 @@ static int cg_restart_plan(const CgState& hs, double target) {
 static void cg_verify(CgRun& R, double target) {
 	if (R.resident && ((const CgState*)R.s->hscal)->pad) {
 		// the one-kernel solve gave up: again, on the general kernels
+		g_res_gaveup++;
+		R.words().rest = kResRest;
 		R.resident = false;
 		R.launched = 0;
 		cg_init(R);
@@ -3124,6 +3137,13 @@ extern "C" long long mfx_testing_resident_wait(long long ticks) {
 	g_res_wait = ticks < 0 ? kResWaitTicks : ticks;
 	return prev;
 }
+// Testing hooks: one-kernel solves queued and given up so far; the number of
+// compute units they count with (0: the device's own).
+extern "C" void mfx_testing_resident_counts(long long* ran, long long* gaveUp) {
+	if (ran) *ran = g_res_ran;
+	if (gaveUp) *gaveUp = g_res_gaveup;
+}
+extern "C" void mfx_testing_resident_cus(int cus) { cg_resident_cus(cus); }
 // Testing hook: set the plane chunks that single solves of a shape use
 // (multiples of 4 up to 64; 0,0 = autotune again).  Returns 0, or -1 for a
 // chunk the z-marching kernels do not accept.

@@ -34,7 +34,14 @@ struct ResP {
 	unsigned epoch;          // first tag
 	long long limit;         // longest wait (wall clock ticks, 100 MHz)
 };
-void cg_resident_run(hipStream_t s, const ResPlan& pl, ResP p);
+// Queues the solve on a stream of `device` (the current one).  Returns false,
+// with nothing queued, where its workgroups do not fit the device together.
+bool cg_resident_run(int device, hipStream_t s, const ResPlan& pl, ResP p);
+// the stream has drained and goes
+void cg_resident_forget(int device, hipStream_t s);
+// compute units of the device as the launches count them (testing: override > 0
+// replaces the device's own number, 0 restores it)
+void cg_resident_cus(int override);
 
 // First tag of a solve of at most maxIter iterations on these exchange words
 // (solves that share them run one after another).

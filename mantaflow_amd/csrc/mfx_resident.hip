@@ -22,12 +22,19 @@
 // own part of the next reduction, that it has read the old value, so one
 // slot per workgroup and reduction is enough.
 //
-// At most kResMaxWG workgroups are launched, far fewer than the GPU holds at
-// once, and every wait is bounded by the clock: a workgroup that waits longer
+// The workgroups of a solve have to be on the GPU together.  At most kResMaxWG
+// are launched, and the solves in flight on a device are kept to as many as
+// leave every workgroup of theirs a compute unit of its own: a workgroup that
+// has not started finds a unit without one of them, whose other work ends by
+// itself (cg_resident_run).  Other processes on the device are not counted, so
+// every wait is bounded by the clock as well: a workgroup that waits longer
 // than `limit` ticks gives up, marks the solve as aborted and leaves; the
-// host then runs the solve again on the general kernels.
+// host then runs the solve again on the general kernels, and the next ones of
+// that solver too (ResWords::rest).
 #include <algorithm>
 #include <limits>
+#include <mutex>
+#include <vector>
 
 #include "mfx_batch.h"
 #include "mfx_internal.h"
@@ -449,14 +456,83 @@ template <int V>
 static void run_multi(hipStream_t s, const ResPlan& pl, const ResP& p) {
 	hipLaunchKernelGGL((k_cg_resident<1024, V, true>), dim3((unsigned)pl.wg), dim3(1024), lds_bytes(pl), s, p);
 }
-void cg_resident_run(hipStream_t s, const ResPlan& pl, ResP p) {
-	p.H = pl.H;
-	if (pl.NT == 512 && pl.V == 4) run_one<512, 4>(s, pl, p);
-	else if (pl.NT == 512) run_one<512, 8>(s, pl, p);
-	else if (pl.wg == 1) run_one<1024, 8>(s, pl, p);
-	else if (pl.V == 2) run_multi<2>(s, pl, p);
+
+// Solves of several workgroups in flight on one device: a lane holds one at a
+// time.  A solve takes the lane its stream used last, else the one unused for
+// longest, and its stream waits (on the device) for the solve that was queued
+// in it before; which lane it gets changes no result.
+struct ResLane {
+	hipEvent_t ev = nullptr;  // end of the lane's last solve
+	hipStream_t last = nullptr;
+	unsigned long long used = 0;
+};
+struct ResDevice {
+	int cus = -1;  // -1: not looked up; 0: a workgroup does not fit a unit
+	std::vector<ResLane> lane;
+	unsigned long long clock = 0;
+};
+static std::mutex g_res_mu;
+static ResDevice g_res_dev[64];
+static int g_res_cus = 0;
+void cg_resident_cus(int override) {
+	std::lock_guard<std::mutex> lk(g_res_mu);
+	g_res_cus = override;
+}
+template <int V>
+static bool fits_unit() {
+	int n = 0;
+	return hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, k_cg_resident<1024, V, true>, 1024, (size_t)kMaxLds) ==
+	           hipSuccess &&
+	       n >= 1;
+}
+static bool run_in_lane(int device, hipStream_t s, const ResPlan& pl, const ResP& p) {
+	if (device < 0 || device >= 64) return false;
+	std::lock_guard<std::mutex> lk(g_res_mu);
+	ResDevice& D = g_res_dev[device];
+	if (D.cus < 0) {
+		int cus = 0;
+		MFX_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device));
+		D.cus = fits_unit<2>() && fits_unit<4>() && fits_unit<8>() ? cus : 0;
+	}
+	const int cus = g_res_cus > 0 ? std::min(g_res_cus, D.cus) : D.cus;
+	if (pl.wg > cus) return false;
+	const size_t lanes = (size_t)std::max(1, cus / kResMaxWG);
+	while (D.lane.size() < lanes) {
+		ResLane l;
+		MFX_HIP(hipEventCreateWithFlags(&l.ev, hipEventDisableTiming));
+		D.lane.push_back(l);
+	}
+	ResLane* l = &D.lane[0];
+	for (size_t i = 0; i < lanes; i++) {
+		ResLane& c = D.lane[i];
+		if (c.last == s) {
+			l = &c;
+			break;
+		}
+		if (c.used < l->used) l = &c;
+	}
+	if (l->last && l->last != s) MFX_HIP(hipStreamWaitEvent(s, l->ev, 0));
+	if (pl.V == 2) run_multi<2>(s, pl, p);
 	else if (pl.V == 4) run_multi<4>(s, pl, p);
 	else run_multi<8>(s, pl, p);
+	l->last = s;
+	l->used = ++D.clock;
+	MFX_HIP(hipEventRecord(l->ev, s));
+	return true;
+}
+void cg_resident_forget(int device, hipStream_t s) {
+	if (device < 0 || device >= 64) return;
+	std::lock_guard<std::mutex> lk(g_res_mu);
+	for (ResLane& l : g_res_dev[device].lane)
+		if (l.last == s) l.last = nullptr;
+}
+bool cg_resident_run(int device, hipStream_t s, const ResPlan& pl, ResP p) {
+	p.H = pl.H;
+	if (pl.wg > 1) return run_in_lane(device, s, pl, p);
+	if (pl.NT == 512 && pl.V == 4) run_one<512, 4>(s, pl, p);
+	else if (pl.NT == 512) run_one<512, 8>(s, pl, p);
+	else run_one<1024, 8>(s, pl, p);
+	return true;
 }
 
 }  // namespace mfx

@@ -8,6 +8,9 @@ the order of the FP64 sums behind the scalars, so the iterates are equal up to
 a rounding of a scalar: the iteration counts must be equal (a stop decided by
 one rounding of the residual norm would move them by one) and the solutions
 within the tolerance the parity tests use for that difference."""
+import ctypes as C
+from contextlib import contextmanager
+
 import numpy as np
 import pytest
 
@@ -105,3 +108,122 @@ def test_resident_nan_diverges(manta, oracle):
         vel[shape[0] * 20 + 20] = np.nan
         with pytest.raises(RuntimeError, match="diverged"):
             _solve(manta, shape, flags, vel, cgAccuracy=1e-4)
+
+
+def _counts():
+    """(one-kernel solves queued, of them given up) so far"""
+    a, b = C.c_longlong(), C.c_longlong()
+    lib().mfx_testing_resident_counts(C.byref(a), C.byref(b))
+    return a.value, b.value
+
+
+@contextmanager
+def _hook(name, value, back):
+    f = getattr(lib(), name)
+    f.argtypes = [type(value)]
+    f(value)
+    try:
+        yield
+    finally:
+        f(type(value)(back))
+
+
+def test_resident_needs_a_unit_per_workgroup(manta, oracle):
+    # 150x130 cells are 10 workgroups, 60x60 one (which waits for nobody)
+    shape, small = (150, 130, 1), (60, 60, 1)
+    flags, vel = _problem(oracle, shape, 12)
+    sflags, svel = _problem(oracle, small, 12)
+    kw = dict(cgAccuracy=1e-4)
+    want = _solve(manta, shape, flags, vel, general=True, **kw)
+    for cus, ran in ((9, 0), (10, 1), (64, 1)):
+        with _hook("mfx_testing_resident_cus", C.c_int(cus), 0):
+            before = _counts()
+            _close(_solve(manta, shape, flags, vel, **kw), want)
+            assert _counts() == (before[0] + ran, before[1]), cus
+    with _hook("mfx_testing_resident_cus", C.c_int(1), 0):
+        before = _counts()
+        _solve(manta, small, sflags, svel, **kw)
+        assert _counts() == (before[0] + 1, before[1])
+
+
+def test_resident_rests_after_giving_up(manta, oracle):
+    shape = (150, 130, 1)
+    flags, vel = _problem(oracle, shape, 10)
+    kw = dict(preconditioner=manta.PcNone, cgAccuracy=1e-4)
+    g = GpuScene(manta, shape)
+    f, v, p = g.flags(flags), g.mac(vel), g.real()
+
+    def solve():
+        v.fromNumpy(vel)
+        before = _counts()
+        manta.solvePressure(flags=f, vel=v, pressure=p, **kw)
+        after = _counts()
+        return p.toNumpy().copy(), (after[0] - before[0], after[1] - before[1])
+
+    whole = solve()
+    assert whole[1] == (1, 0)
+    with _hook("mfx_testing_resident_wait", C.c_longlong(0), -1):
+        gave = solve()
+        assert gave[1] == (1, 1)
+    # the wait was paid once: this solver's next solves do not try again
+    for _ in range(3):
+        again = solve()
+        assert again[1] == (0, 0)
+        np.testing.assert_array_equal(again[0], gave[0])
+    # another solver does
+    h = GpuScene(manta, shape)
+    f, v, p = h.flags(flags), h.mac(vel), h.real()
+    other = solve()
+    assert other[1] == (1, 0)
+    np.testing.assert_array_equal(other[0], whole[0])
+
+
+@pytest.mark.parametrize("cus", [0, 64])
+def test_resident_solves_at_once(manta, oracle, cus):
+    """A batch's unpreconditioned problems start together, each on its own
+    solver's stream: more of them than the device holds at once (or, counted
+    with 64 units, one after another) give the bits of solves alone."""
+    shapes = [(353, 241, 1), (512, 512, 1), (150, 130, 1), (64, 64, 1), (363, 363, 1), (1500, 70, 1)] * 2
+    kw = dict(preconditioner=manta.PcMIC, cgAccuracy=1e-4)
+    single, batch = [], []
+    for k, shape in enumerate(shapes):
+        flags, vel = _problem(oracle, shape, 20 + k)
+        for out in (single, batch):
+            g = GpuScene(manta, shape)
+            out.append((g, g.flags(flags), g.mac(vel), g.real()))
+    for g, f, v, p in single:
+        manta.solvePressure(flags=f, vel=v, pressure=p, **kw)
+    with _hook("mfx_testing_resident_cus", C.c_int(cus), 0):
+        before = _counts()
+        manta.solvePressureBatch([(v, p, f) for g, f, v, p in batch], **kw)
+        assert _counts() == (before[0] + len(shapes), before[1])
+    for (g1, f1, v1, p1), (g2, f2, v2, p2) in zip(single, batch):
+        assert manta.lastSolveStats(g1.s)["iterations"] == manta.lastSolveStats(g2.s)["iterations"]
+        np.testing.assert_array_equal(p1.toNumpy(), p2.toNumpy())
+        np.testing.assert_array_equal(v1.toNumpy(), v2.toNumpy())
+
+
+def test_resident_batch_fallback(manta, oracle):
+    """Workgroups of a batch's problems that give up: those problems run again
+    on the general kernels, the others are not touched."""
+    shapes = [(150, 130, 1), (64, 64, 1), (24, 24, 24), (353, 241, 1)]
+    kw = dict(preconditioner=manta.PcMIC, cgAccuracy=1e-4)
+    want, batch = [], []
+    for k, shape in enumerate(shapes):
+        flags, vel = _problem(oracle, shape, 40 + k)
+        many = shape[2] == 1 and shape != (64, 64, 1)
+        want.append(_solve(manta, shape, flags, vel, general=True, cgAccuracy=1e-4) if many else None)
+        for out in (batch, None):
+            g = GpuScene(manta, shape)
+            f, v, p = g.flags(flags), g.mac(vel), g.real()
+            if out is None and not many:
+                manta.solvePressure(flags=f, vel=v, pressure=p, **kw)
+                want[-1] = p.toNumpy(), v.toNumpy(), manta.lastSolveStats(g.s)
+            elif out is not None:
+                out.append((g, f, v, p))
+    with _hook("mfx_testing_resident_wait", C.c_longlong(0), -1):
+        before = _counts()
+        manta.solvePressureBatch([(v, p, f) for g, f, v, p in batch], **kw)
+        assert _counts() == (before[0] + 3, before[1] + 2)
+    for (g, f, v, p), w in zip(batch, want):
+        _close((p.toNumpy(), v.toNumpy(), manta.lastSolveStats(g.s)), w)
