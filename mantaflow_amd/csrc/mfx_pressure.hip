@@ -1900,12 +1900,12 @@ static void cg_init(CgRun& R) {
 
 // Unpreconditioned solves of grids that fit the one-kernel CG: doInit and
 // every iteration as one launch.  Returns false where the general kernels
-// have to run.  At most 5 s may pass before a workgroup gives up waiting for
-// another; cg_verify then runs the solve on the general kernels, and so do the
+// have to run.  A workgroup that waits 1 s for another (a wait is some
+// microseconds) gives up; cg_verify then runs the solve on the general kernels, and so do the
 // next kResRest solves on the same exchange words, so that a device shared
 // with something that keeps the workgroups apart costs that wait once in so
 // many solves and not in each.
-constexpr long long kResWaitTicks = 5ll * 100000000ll;
+constexpr long long kResWaitTicks = 100000000ll;
 constexpr int kResRest = 1000;
 static long long g_res_wait = kResWaitTicks;
 static std::atomic<long long> g_res_ran{0}, g_res_gaveup{0};

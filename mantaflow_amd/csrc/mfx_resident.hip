@@ -106,11 +106,13 @@ struct ResShared {
 };
 
 // Words [0, NW) of every workgroup's slot with the tag: lane l reads
-// workgroup l's (wavefront 0 only; at most 64 workgroups)
+// workgroup l's (wavefront 0 only; at most 64 workgroups).  The wait is timed
+// from its first poll in vain; a workgroup that has given up does not wait.
 template <int NW>
-__device__ inline void gather(const unsigned long long* slots, int nwg, unsigned tag, long long t0, long long limit,
-                              int* abort, unsigned long long* w) {
+__device__ inline void gather(const unsigned long long* slots, int nwg, unsigned tag, long long limit, int* abort,
+                              unsigned long long* w) {
 	const int l = threadIdx.x;
+	long long since = 0;
 	for (;;) {
 		bool ok = true;
 		if (l < nwg) {
@@ -120,7 +122,9 @@ __device__ inline void gather(const unsigned long long* slots, int nwg, unsigned
 			for (int q = 0; q < NW; q++) ok = ok && (unsigned)(w[q] >> 32) == tag;
 		}
 		if (__all(ok)) return;
-		if (wall_clock64() - t0 > limit) {
+		const long long now = wall_clock64();
+		if (since == 0) since = now;
+		if (*abort || now - since >= limit) {
 			*abort = 1;
 			return;
 		}
@@ -148,7 +152,7 @@ __global__ void __launch_bounds__(NT) k_cg_resident(ResP P) {
 	const bool needRR = relTol > 0 || useL2;
 	unsigned long long* slA = P.xs;
 	unsigned long long* slB = P.xs + (size_t)kResMaxWG * kSlot;
-	const long long t0 = MULTI ? (long long)wall_clock64() : 0;
+	bool gaveUp = false;
 	if (t == 0) S.abort = 0;
 	if (NT < 64 * kMaxNW && t < kMaxNW) {
 		// (the sums run over kMaxNW wavefronts)
@@ -226,7 +230,7 @@ __global__ void __launch_bounds__(NT) k_cg_resident(ResP P) {
 			                                  : m0;
 			if (lane < kWordsB) xstore(slB + (size_t)blockIdx.x * kSlot + lane, tag, word);
 			unsigned long long g[kWordsB];
-			gather<kWordsB>(slB, nwg, tag, t0, P.limit, &S.abort, g);
+			gather<kWordsB>(slB, nwg, tag, P.limit, &S.abort, g);
 			const bool mine = lane < nwg;
 			const double sz_ = wave_sum_to_last(mine ? word_pair(g[0], g[1]) : 0.0);
 			const double sr_ = wave_sum_to_last(mine ? word_pair(g[2], g[3]) : 0.0);
@@ -268,10 +272,13 @@ __global__ void __launch_bounds__(NT) k_cg_resident(ResP P) {
 						hr = P.b[g];
 					} else {
 						unsigned long long u;
-						while ((unsigned)((u = xload(P.xr + g)) >> 32) != tag) {
-							if (wall_clock64() - t0 > P.limit) {
+						long long since = 0;
+						while ((unsigned)((u = xload(P.xr + g)) >> 32) != tag && !gaveUp) {
+							const long long now = wall_clock64();
+							if (since == 0) since = now;
+							if (now - since >= P.limit) {
 								S.abort = 1;
-								break;
+								gaveUp = true;
 							}
 						}
 						hr = __int_as_float((int)(unsigned)u);
@@ -315,7 +322,7 @@ __global__ void __launch_bounds__(NT) k_cg_resident(ResP P) {
 				if (lane < kWordsA)
 					xstore(slA + (size_t)blockIdx.x * kSlot + lane, tag, lane ? (unsigned)(u >> 32) : (unsigned)u);
 				unsigned long long g[kWordsA];
-				gather<kWordsA>(slA, nwg, tag, t0, P.limit, &S.abort, g);
+				gather<kWordsA>(slA, nwg, tag, P.limit, &S.abort, g);
 				const double s = wave_sum_to_last(lane < nwg ? word_pair(g[0], g[1]) : 0.0);
 				if (lane == 63) S.tot[0] = s;
 			}

@@ -227,3 +227,15 @@ def test_resident_batch_fallback(manta, oracle):
         assert _counts() == (before[0] + 3, before[1] + 2)
     for (g, f, v, p), w in zip(batch, want):
         _close((p.toNumpy(), v.toNumpy(), manta.lastSolveStats(g.s)), w)
+
+
+def test_resident_limit_is_per_wait(manta, oracle):
+    """The limit bounds one wait (a few microseconds), not the solve: one that
+    runs several times as long as the limit of 1 ms is not given up."""
+    shape = (353, 241, 1)
+    flags, vel = _problem(oracle, shape, 13)
+    with _hook("mfx_testing_resident_wait", C.c_longlong(100000), -1):
+        before = _counts()
+        got = _solve(manta, shape, flags, vel, cgAccuracy=2e-7, cgMaxIterFac=3.0)
+        assert _counts() == (before[0] + 1, before[1])
+    assert got[2]["seconds"] > 4 * 1e-3, got[2]
