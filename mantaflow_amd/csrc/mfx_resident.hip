@@ -474,7 +474,7 @@ struct ResLane {
 	unsigned long long used = 0;
 };
 struct ResDevice {
-	int cus = -1;  // -1: not looked up; 0: a workgroup does not fit a unit
+	int cus = -1;  // compute units (-1: not looked up)
 	std::vector<ResLane> lane;
 	unsigned long long clock = 0;
 };
@@ -485,21 +485,18 @@ void cg_resident_cus(int override) {
 	std::lock_guard<std::mutex> lk(g_res_mu);
 	g_res_cus = override;
 }
-template <int V>
-static bool fits_unit() {
-	int n = 0;
-	return hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, k_cg_resident<1024, V, true>, 1024, (size_t)kMaxLds) ==
-	           hipSuccess &&
-	       n >= 1;
-}
 static bool run_in_lane(int device, hipStream_t s, const ResPlan& pl, const ResP& p) {
 	if (device < 0 || device >= 64) return false;
 	std::lock_guard<std::mutex> lk(g_res_mu);
 	ResDevice& D = g_res_dev[device];
 	if (D.cus < 0) {
+		// (one workgroup fits a unit: at most 1024 threads by its launch bounds,
+		// at most 64 KiB of LDS.  The runtime's occupancy query is not asked: it
+		// answers 0 once a second runtime is loaded in the process, as torch's is)
+		static_assert(kMaxLds + sizeof(ResShared) + 64 <= 64 * 1024, "LDS of a workgroup");
 		int cus = 0;
 		MFX_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device));
-		D.cus = fits_unit<2>() && fits_unit<4>() && fits_unit<8>() ? cus : 0;
+		D.cus = cus;
 	}
 	const int cus = g_res_cus > 0 ? std::min(g_res_cus, D.cus) : D.cus;
 	if (pl.wg > cus) return false;

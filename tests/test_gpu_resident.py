@@ -9,6 +9,9 @@ a rounding of a scalar: the iteration counts must be equal (a stop decided by
 one rounding of the residual norm would move them by one) and the solutions
 within the tolerance the parity tests use for that difference."""
 import ctypes as C
+import os
+import subprocess
+import sys
 from contextlib import contextmanager
 
 import numpy as np
@@ -16,6 +19,8 @@ import pytest
 
 from mantaflow_amd._abi import lib
 from tests.helpers import GpuScene, make_flags, smooth_vel
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 
 pytestmark = pytest.mark.gpu
 
@@ -239,3 +244,26 @@ def test_resident_limit_is_per_wait(manta, oracle):
         got = _solve(manta, shape, flags, vel, cgAccuracy=2e-7, cgMaxIterFac=3.0)
         assert _counts() == (before[0] + 1, before[1])
     assert got[2]["seconds"] > 4 * 1e-3, got[2]
+
+
+def test_resident_beside_another_runtime():
+    """torch loads a HIP runtime of its own; the one-kernel CG runs all the same
+    (in a child process, so that the other tests keep one runtime)."""
+    prog = """
+import ctypes as C
+from mantaflow_amd import manta
+import torch
+from mantaflow_amd._abi import lib
+s = manta.Solver(name="t", gridSize=manta.vec3(150, 130, 1), dim=2)
+f, v, p = s.create(manta.FlagGrid), s.create(manta.MACGrid), s.create(manta.RealGrid)
+f.initDomain()
+f.fillGrid()
+v.setConst(manta.vec3(0.1, 0.2, 0))
+manta.setWallBcs(flags=f, vel=v)
+manta.solvePressure(flags=f, vel=v, pressure=p, preconditioner=manta.PcNone, cgAccuracy=1e-4)
+ran, gave = C.c_longlong(), C.c_longlong()
+lib().mfx_testing_resident_counts(C.byref(ran), C.byref(gave))
+print("counts", ran.value, gave.value)
+"""
+    r = subprocess.run([sys.executable, "-c", prog], cwd=ROOT, capture_output=True, text=True, timeout=100)
+    assert r.returncode == 0 and "counts 1 0" in r.stdout, r.stdout + r.stderr
