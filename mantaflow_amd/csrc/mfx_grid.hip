@@ -56,14 +56,23 @@ Scene::~Scene() {
 	if (stream) hipStreamDestroy(stream);
 }
 
+// Testing hook: the allocation of a scene's working memory after `after` more
+// fails (< 0: none does).
+static std::atomic<int> g_fail_alloc{-1};
+static void* scene_alloc(size_t bytes) {
+	if (g_fail_alloc >= 0 && g_fail_alloc-- == 0) MFX_HIP(hipErrorOutOfMemory);
+	void* p = nullptr;
+	MFX_HIP(hipMalloc(&p, bytes));
+	return p;
+}
+
 float* Scene::getReal() {
 	if (!freeReal.empty()) {
 		float* p = freeReal.back();
 		freeReal.pop_back();
 		return p;
 	}
-	float* p = nullptr;
-	MFX_HIP(hipMalloc(&p, sizeof(float) * (size_t)d.n));
+	float* p = (float*)scene_alloc(sizeof(float) * (size_t)d.n);
 	owned.insert(p);
 	return p;
 }
@@ -74,22 +83,26 @@ float* Scene::getVec() {
 		freeVec.pop_back();
 		return p;
 	}
-	float* p = nullptr;
-	MFX_HIP(hipMalloc(&p, sizeof(float) * 3 * cstride));
+	float* p = (float*)scene_alloc(sizeof(float) * 3 * cstride);
 	owned.insert(p);
 	return p;
 }
 void Scene::putVec(float* p) { freeVec.push_back(p); }
 
 void Scene::ensurePartials(size_t nd, size_t nf) {
+	// (without the larger buffer there is none: the old one is gone)
 	if (nd > dpartCap) {
 		if (dpart) MFX_HIP(hipFree(dpart));
-		MFX_HIP(hipMalloc(&dpart, sizeof(double) * nd));
+		dpart = nullptr;
+		dpartCap = 0;
+		dpart = (double*)scene_alloc(sizeof(double) * nd);
 		dpartCap = nd;
 	}
 	if (nf > fpartCap) {
 		if (fpart) MFX_HIP(hipFree(fpart));
-		MFX_HIP(hipMalloc(&fpart, sizeof(float) * nf));
+		fpart = nullptr;
+		fpartCap = 0;
+		fpart = (float*)scene_alloc(sizeof(float) * nf);
 		fpartCap = nf;
 	}
 }
@@ -814,6 +827,9 @@ static inline Scene* S(mfx_scene* s) { return static_cast<Scene*>(s); }
 static inline Grid* G(const mfx_grid* g) { return const_cast<Grid*>(static_cast<const Grid*>(g)); }
 
 #define NEED(p, what) MFX_CHECK((p) != nullptr, std::string(what) + " must not be null")
+
+// (not part of the public interface)
+extern "C" void mfx_testing_fail_alloc(int after) { g_fail_alloc = after; }
 
 extern "C" {
 

@@ -92,3 +92,35 @@ def test_swap_between_solvers_moves_ownership(manta):
         if rep == 1:
             check_mem = _free_memory()
     assert check_mem - _free_memory() < 4 * n
+
+
+def test_partial_sums_after_a_failed_growth(manta, oracle):
+    """The buffers of partial sums grow with the first solve.  When that fails
+    the old ones are gone: the next calls allocate again."""
+    shape = (32, 30, 24)
+    n = 32 * 30 * 24
+    rng = np.random.default_rng(4)
+    flags = oracle.init_domain(shape)
+    oracle.fill_grid(shape, flags)
+    vel, vals = rand_vel(rng, n, 0.5), rng.uniform(-1, 1, n).astype(np.float32)
+    oracle.set_wall_bcs(shape, flags, vel)
+    kw = dict(cgAccuracy=1e-4, preconditioner=manta.PcNone)
+    out = []
+    for fail in (False, True):
+        g = GpuScene(manta, shape)
+        f, v, p, r = g.flags(flags), g.mac(vel), g.real(), g.real(vals)
+        assert r.getMaxAbs() == np.abs(vals).max()
+        if fail:
+            # the right-hand side is had, the partial sums are not
+            lib().mfx_testing_fail_alloc(1)
+            try:
+                with pytest.raises(RuntimeError, match="memory"):
+                    manta.solvePressure(flags=f, vel=v, pressure=p, **kw)
+            finally:
+                lib().mfx_testing_fail_alloc(-1)
+            assert r.getMaxAbs() == np.abs(vals).max()
+        manta.solvePressure(flags=f, vel=v, pressure=p, **kw)
+        assert r.getMaxAbs() == np.abs(vals).max()
+        out.append((p.toNumpy(), v.toNumpy()))
+    np.testing.assert_array_equal(out[0][0], out[1][0])
+    np.testing.assert_array_equal(out[0][1], out[1][1])
