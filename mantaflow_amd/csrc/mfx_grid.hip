@@ -77,6 +77,10 @@ float* Scene::getReal() {
 	return p;
 }
 void Scene::putReal(float* p) { freeReal.push_back(p); }
+void Scene::dropReal(float* p) {
+	owned.erase(p);
+	(void)hipFree(p);
+}
 float* Scene::getVec() {
 	if (!freeVec.empty()) {
 		float* p = freeVec.back();

@@ -121,6 +121,7 @@ struct Scene {
 	~Scene();
 	float* getReal();
 	void putReal(float* p);
+	void dropReal(float* p);  // back to the device instead of the pool (hipFree waits for what is queued)
 	float* getVec();
 	void putVec(float* p);
 	void ensurePartials(size_t nd, size_t nf);

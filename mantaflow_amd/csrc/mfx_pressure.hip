@@ -2445,49 +2445,56 @@ static void launch_joint(hipStream_t q, long long nb, const CgRun* R, int nc, F 
 	hipLaunchKernelGGL((k_joint<P, BODY, NT>), dim3((unsigned)nb, (unsigned)nc), dim3(NT), 0, q, a);
 }
 
-// The components of a Vec3 / MAC diffusion as one sequence of launches:
+// The components u of a Vec3 / MAC diffusion as one sequence of launches:
 // their matrix is the same, and up to some millions of cells an iteration of
 // one component is four launches of 3 to 12 us that leave most of the GPU
-// idle.  rhs: the components, cstride apart, copied from u before.  Returns
-// false, with nothing queued, where the components are solved one by one:
-// grids of the one-kernel CG, larger grids, and when the further buffers
-// cannot be had.  The line: the systems' vectors have to stay in the 256 MB
-// last-level cache.  Three components, one by one / together: 84^3 984 / 483
-// us, 144^3 1680 / 1258, 176^3 2317 / 2331, 202^3 3310 / 4253.
+// idle.  Returns false, with nothing queued, where the components are solved
+// one by one: grids of the one-kernel CG, larger grids, and when the further
+// buffers cannot be had.  The line: the systems' vectors have to stay in the
+// 256 MB last-level cache.  Three components, one by one / together: 84^3 984
+// / 483 us, 144^3 1680 / 1258, 176^3 2317 / 2331, 202^3 3310 / 4253.
 constexpr long long kJointCells = 3ll << 22;  // of all components
+constexpr int kScaledBufs = 4;                // CG vectors of one component
 static bool joint_diffusion(const Dims& d, int nc) { return nc > 1 && nc * d.n <= kJointCells && !cg_resident_plan(d).V; }
-static bool solve_diffusion_joint(Scene* s, Grid* flags, float* rhs, float* const* u, int nc, float alpha,
-                                  float cgAccuracy, float cgMaxIterFac, mfx_solve_stats* stats) {
+static bool solve_diffusion_joint(Scene* s, Grid* flags, float* const* u, int nc, float alpha, float cgAccuracy,
+                                  float cgMaxIterFac, mfx_solve_stats* stats) {
 	const Dims& d = s->d;
 	if (!joint_diffusion(d, nc)) return false;
-	float* buf[4 * kJointMax] = {};
+	std::vector<float*> buf;
+	CgRun R[kJointMax];
 	auto give = [&]() {
-		for (float* b : buf)
-			if (b) s->putReal(b);
+		for (float* b : buf) s->putReal(b);
 	};
 	try {
-		for (int i = 0; i < 4 * nc; i++) buf[i] = s->getReal();
+		for (int i = 0; i < (kScaledBufs + 1) * nc; i++) buf.push_back(s->getReal());
+		for (int c = 0; c < nc; c++) {
+			float** b = &buf[(size_t)((kScaledBufs + 1) * c)];
+			const size_t per = scaled_shape(R[c], s, flags, b[4], u[c], alpha, cgAccuracy, cgMaxIterFac, nc);
+			R[c].dpart += 3 * per * (size_t)c;
+			R[c].fpart += 2 * per * (size_t)c;
+			R[c].st += c;
+			R[c].r = R[c].z = b[0];
+			R[c].pa = b[1];
+			R[c].pb = b[2];
+			R[c].q = b[3];
+		}
 	} catch (...) {
+		// one component needs its vectors and a right-hand side; the rest goes
+		// back to the device, not to the pool
 		(void)hipGetLastError();
+		while (buf.size() > kScaledBufs + 1) {
+			s->dropReal(buf.back());
+			buf.pop_back();
+		}
 		give();
 		return false;
 	}
-	CgRun R[kJointMax];
 	const CgState* hs = (const CgState*)s->hscal;
 	static_assert(kJointMax * sizeof(CgState) <= 4096, "the scene's scalar block");
 	const hipStream_t q = s->stream;
 	try {
-		for (int c = 0; c < nc; c++) {
-			const size_t per = scaled_shape(R[c], s, flags, rhs + c * s->cstride, u[c], alpha, cgAccuracy, cgMaxIterFac, nc);
-			R[c].dpart += 3 * per * (size_t)c;
-			R[c].fpart += 2 * per * (size_t)c;
-			R[c].st += c;
-			R[c].r = buf[4 * c];
-			R[c].z = buf[4 * c];
-			R[c].pa = buf[4 * c + 1];
-			R[c].pb = buf[4 * c + 2];
-			R[c].q = buf[4 * c + 3];
-		}
+		for (int c = 0; c < nc; c++)
+			MFX_HIP(hipMemcpyAsync(R[c].rhs, u[c], sizeof(float) * (size_t)d.n, hipMemcpyDeviceToDevice, q));
 		const unsigned nbM = R[0].nbM, nbU = R[0].nbU;
 		const int maxIter = R[0].maxIter, npM = R[0].npM;
 		const long long nLight = tiles_for(d, kLightKZ).count();
@@ -3477,20 +3484,7 @@ int mfx_cg_solve_diffusion(const mfx_grid* flags, mfx_grid* grid, float alpha, f
 	const int nc = g->isVec() ? (s->d.is3d ? 3 : 2) : 1;
 	float* u[kJointMax];
 	for (int c = 0; c < nc; c++) u[c] = g->comp(c);
-	if (joint_diffusion(s->d, nc)) {
-		float* rhs3 = s->getVec();
-		bool ok = false;
-		try {
-			for (int c = 0; c < nc; c++)
-				MFX_HIP(hipMemcpyAsync(rhs3 + c * s->cstride, u[c], bytes, hipMemcpyDeviceToDevice, s->stream));
-			ok = solve_diffusion_joint(s, f, rhs3, u, nc, alpha, cgAccuracy, cgMaxIterFac, stats);
-		} catch (...) {
-			s->putVec(rhs3);
-			throw;
-		}
-		s->putVec(rhs3);
-		if (ok) return 0;
-	}
+	if (solve_diffusion_joint(s, f, u, nc, alpha, cgAccuracy, cgMaxIterFac, stats)) return 0;
 	float* rhs = s->getReal();
 	try {
 		for (int c = 0; c < nc; c++) {

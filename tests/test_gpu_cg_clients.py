@@ -4,9 +4,12 @@
 with obstacles and empty cells.  The CG runs the same iteration as the
 oracle; reductions are summed in another order, so iteration counts agree
 within one and solutions within the CG tolerance (stated per test)."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
+from mantaflow_amd._abi import check, lib
 from oracle import EMPTY, FLUID, OBSTACLE
 from tests.helpers import GpuScene, make_flags
 
@@ -120,3 +123,29 @@ def test_diffusion_components_diverge(manta, oracle, rng):
     with pytest.raises(RuntimeError, match="diverged"):
         manta.cgSolveDiffusion(flags=f, grid=g, alpha=3e38, cgMaxIterFac=2.0, cgAccuracy=1e-5)
     np.testing.assert_array_equal(g.toNumpy()[:, 1:], val[:, 1:])
+
+
+def test_diffusion_without_the_further_buffers(manta, oracle, rng):
+    """When a buffer that only the joint solve needs cannot be had, the
+    components are solved one after another: the same bits, no error, and no
+    more buffers kept than that takes."""
+    shape = (83, 85, 81)
+    n = int(np.prod(shape))
+    flags = _flags(oracle, rng, shape, False)
+    val = rng.uniform(-1, 1, (n, 3)).astype(np.float32)
+    want, sizes = None, []
+    for after in (-1, 0, 1, 4, 5, 9, 14, 15, 16):  # 15 vectors, then the partial sums
+        sc = GpuScene(manta, shape)
+        f, g = sc.flags(flags), sc.vec(val)
+        lib().mfx_testing_fail_alloc(after)
+        try:
+            manta.cgSolveDiffusion(flags=f, grid=g, alpha=0.6, cgMaxIterFac=2.0, cgAccuracy=1e-5)
+        finally:
+            lib().mfx_testing_fail_alloc(-1)
+        got = g.toNumpy().copy()
+        want = got if want is None else want
+        np.testing.assert_array_equal(got, want, err_msg=str(after))
+        b = C.c_size_t()
+        check(lib().mfx_scene_memory(sc.s._h, C.byref(b)))
+        sizes.append(b.value)
+    assert all(sizes[0] - b == 4 * 10 * n for b in sizes[1:]), sizes
