@@ -59,7 +59,7 @@ Scene::~Scene() {
 // Testing hook: the allocation of a scene's working memory after `after` more
 // fails (< 0: none does).
 static std::atomic<int> g_fail_alloc{-1};
-static void* scene_alloc(size_t bytes) {
+void* scene_alloc(size_t bytes) {
 	if (g_fail_alloc >= 0 && g_fail_alloc-- == 0) MFX_HIP(hipErrorOutOfMemory);
 	void* p = nullptr;
 	MFX_HIP(hipMalloc(&p, bytes));

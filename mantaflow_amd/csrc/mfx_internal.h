@@ -77,6 +77,9 @@ struct ResWords {
 	int rest = 0;       // solves that still run on the general kernels after one gave up
 };
 
+// device memory a scene works in (throws when there is none)
+void* scene_alloc(size_t bytes);
+
 struct Scene {
 	Dims d;
 	int dim;

@@ -1921,8 +1921,15 @@ static bool cg_try_resident(CgRun& R) {
 	}
 	if (pl.wg > 1 && !w.words) {
 		if (R.res) return false;
-		w.count = kResSlotWords + pl.words;
-		MFX_HIP(hipMalloc((void**)&w.words, sizeof(unsigned long long) * w.count));
+		const size_t count = kResSlotWords + pl.words;
+		try {
+			w.words = (unsigned long long*)scene_alloc(sizeof(unsigned long long) * count);
+		} catch (const Error&) {
+			// (8 bytes a cell that the general kernels do without)
+			(void)hipGetLastError();
+			return false;
+		}
+		w.count = count;
 	}
 	ResP p;
 	p.d = s->d;

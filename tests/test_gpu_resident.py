@@ -246,6 +246,29 @@ def test_resident_limit_is_per_wait(manta, oracle):
     assert got[2]["seconds"] > 4 * 1e-3, got[2]
 
 
+def test_resident_without_its_words(manta, oracle):
+    """The exchange words are the one buffer the general kernels do not need:
+    without them the solve runs on those, and takes the words when it can."""
+    shape = (150, 130, 1)
+    flags, vel = _problem(oracle, shape, 14)
+    g = GpuScene(manta, shape)
+    f, v, p = g.flags(flags), g.mac(vel), g.real()
+    out = []
+    for every, after, ran in (((1 << 30), -1, 0), (0, 0, 0), (0, -1, 1)):
+        v.fromNumpy(vel)
+        g.s.mfxTrueResidualEvery = every
+        before = _counts()
+        lib().mfx_testing_fail_alloc(after)
+        try:
+            manta.solvePressure(flags=f, vel=v, pressure=p, preconditioner=manta.PcNone, cgAccuracy=1e-4)
+        finally:
+            lib().mfx_testing_fail_alloc(-1)
+        assert _counts()[0] - before[0] == ran
+        out.append((p.toNumpy().copy(), v.toNumpy().copy(), dict(manta.lastSolveStats(g.s))))
+    np.testing.assert_array_equal(out[1][0], out[0][0])
+    _close(out[2], out[0])
+
+
 def test_resident_beside_another_runtime():
     """torch loads a HIP runtime of its own; the one-kernel CG runs all the same
     (in a child process, so that the other tests keep one runtime)."""
