@@ -927,6 +927,8 @@ int mfx_scene_memory(const mfx_scene* s, size_t* bytes) {
 	for (Grid* g : sc->grids) b += (g->isVec() ? 3 * sc->cstride * 4 : (size_t)sc->d.n * 4) + (g->f8 ? sc->d.n : 0);
 	b += (sc->freeReal.size()) * (size_t)sc->d.n * 4;
 	b += (sc->freeVec.size()) * 3 * sc->cstride * 4;
+	for (const auto* m : {&sc->mgStatic, &sc->mgDyn, &sc->mgMic}) b += *m ? (*m)->bytes() : 0;
+	b += sc->res.count * sizeof(unsigned long long);
 	*bytes = b;
 	API_END
 }

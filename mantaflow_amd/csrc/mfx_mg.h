@@ -74,6 +74,7 @@ public:
 	int levels() const { return (int)L.size(); }
 	// (-1: the last build did not finish)
 	int precision() const { return ready ? prec : -1; }
+	size_t bytes() const { return arena ? arenaBytes : 0; }  // device memory held
 
 private:
 	bool is3d = true;
@@ -87,6 +88,7 @@ private:
 	int nc = 0;
 	bool ready = false;
 	void* arena = nullptr;       // all of the hierarchy's device memory
+	size_t arenaBytes = 0;
 	void* hbuf = nullptr;        // pinned: what a build reads and writes on the host
 	size_t hostBytes = 0, readBytes = 0;
 	float* zero = nullptr;       // vectors that start a hierarchy at 0

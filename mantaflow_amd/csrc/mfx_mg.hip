@@ -1659,7 +1659,6 @@ void MgHierarchy::layout(Scene* s) {
 	const int nl = (int)L.size();
 	const size_t ncMax = (size_t)L[nl - 1].n;
 	// two passes over the same list: sizes, then addresses
-	size_t total = 0;
 	for (int pass = 0; pass < 2; pass++) {
 		size_t off = 0;
 		auto take = [&](auto*& p, size_t count) {
@@ -1711,8 +1710,8 @@ void MgHierarchy::layout(Scene* s) {
 		take(cpos, ncMax);
 		take(cpin, ncMax);
 		if (!pass) {
-			total = off;
-			MFX_HIP(hipMalloc(&arena, total));
+			arenaBytes = off;
+			MFX_HIP(hipMalloc(&arena, arenaBytes));
 		}
 	}
 	hostBytes = std::max(readBytes, ncMax) + 256 + ((uint8_t*)(cpin + ncMax) - (uint8_t*)cidx);

@@ -2031,14 +2031,18 @@ static void cg_setup(CgRun& R, Scene* s, Grid* flags, float* rhs, float* x, cons
 	R.npM = (int)zm_dot_parts(d, kMvTY);
 
 	if (!R.pcNone) {
+		// (a solve with a hierarchy that is kept for its matrix gives back the
+		// dynamic one, which would only be memory then)
 		if (o.preconditioner == MFX_PC_MGDYNAMIC) {
 			s->mgStatic.reset();
 			if (!s->mgDyn) s->mgDyn.reset(new MgHierarchy());
 			s->mgDyn->build(s, R.code, o.precision);
 			R.mg = s->mgDyn.get();
 		} else if (o.preconditioner == MFX_PC_MIC) {
+			s->mgDyn.reset();
 			R.mg = mic_hierarchy(s, flags, R.code, R.fixing, o.precision);
 		} else {
+			s->mgDyn.reset();
 			if (!s->mgStatic || s->mgStatic->precision() != o.precision) {
 				s->mgStatic.reset(new MgHierarchy());
 				s->mgStatic->build(s, R.code, o.precision);

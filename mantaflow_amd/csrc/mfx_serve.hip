@@ -23,6 +23,7 @@
 #include <vector>
 
 #include "mfx_internal.h"
+#include "mfx_mg.h"
 
 struct mfx_scene : public mfx::Scene {};
 struct mfx_grid : public mfx::Grid {};
@@ -189,6 +190,10 @@ void worker_loop(mfx_server* sv) {
 		std::vector<mfx_serve_result> res;
 		for (const Request& r : batch) res.push_back(make_result(r));
 		run_tick(sv, batch, res);
+		// a finished request holds nothing of the budget: the hierarchy that a
+		// dynamic solve would find again is given back (the next one builds it anyway)
+		if (sv->opts.solve.preconditioner == MFX_PC_MGDYNAMIC)
+			for (const Request& r : batch) r.scene->mgDyn.reset();
 		const double t = sv->now();
 		lk.lock();
 		for (size_t i = 0; i < batch.size(); ++i) {
