@@ -1765,7 +1765,9 @@ struct CgRun {
 	float* fpart = nullptr;
 	uint8_t* code = nullptr;
 	ResWords* res = nullptr;  // exchange words of the one-kernel CG (the scene's when pooled)
-	bool resident = false;    // the iterations ran, or run, as one kernel
+	bool resident = false;    // the iterations ran, or run, as one kernel:
+	ResPlan resPlan;
+	ResP resP{};
 	ResWords& words() const { return res ? *res : s->res; }
 	int pc = 0, maxIter = 0;
 	bool pcNone = true;
@@ -1801,8 +1803,8 @@ struct CgRun {
 
 // matrix, preconditioner, buffers, CgState and GridCg::doInit
 // (conjugategrad.cpp:210-235, pressure.cpp:349-433).  With batchInit the
-// initial V-cycle and sigma = dot(z, r) are left to the caller's batched
-// launches (FIN_BETA0 afterwards).
+// one-kernel CG, or the initial V-cycle and sigma = dot(z, r), are left to the
+// caller's batched launches (FIN_BETA0 afterwards).
 // Autotuner of the z-marching plane chunk.  The first time a 3D grid shape
 // is solved alone, the CG matvec and the level-0 multigrid down-sweep are
 // timed (HIP events, three launches after one warm-up) for chunks of 4..64
@@ -1908,12 +1910,12 @@ static void cg_init(CgRun& R) {
 constexpr long long kResWaitTicks = 100000000ll;
 constexpr int kResRest = 1000;
 static long long g_res_wait = kResWaitTicks;
-static std::atomic<long long> g_res_ran{0}, g_res_gaveup{0};
-static bool cg_try_resident(CgRun& R) {
+static std::atomic<long long> g_res_ran{0}, g_res_gaveup{0}, g_res_launches{0};
+static bool cg_plan_resident(CgRun& R) {
 	Scene* s = R.s;
 	if (!R.pcNone || R.gA0 || R.o.trueResidualEvery > 0) return false;
 	const ResPlan pl = cg_resident_plan(s->d);
-	if (!pl.V) return false;
+	if (!cg_resident_fits(s->device, pl)) return false;
 	ResWords& w = R.words();
 	if (pl.wg > 1 && w.rest > 0) {
 		w.rest--;
@@ -1931,8 +1933,9 @@ static bool cg_try_resident(CgRun& R) {
 		}
 		w.count = count;
 	}
-	ResP p;
+	ResP& p = R.resP;
 	p.d = s->d;
+	p.H = pl.H;
 	p.st = R.st;
 	p.code = R.code;
 	p.b = R.rhs;
@@ -1943,12 +1946,16 @@ static bool cg_try_resident(CgRun& R) {
 	p.xr = w.words ? w.words + kResSlotWords : nullptr;
 	p.epoch = cg_resident_tags(w, s->stream, pl, R.maxIter);
 	p.limit = g_res_wait;
-	{
-		KtScope kt("cg_resident", s->stream);
-		if (!cg_resident_run(s->device, s->stream, pl, p)) return false;
-	}
-	g_res_ran++;
+	R.resPlan = pl;
 	R.resident = true;
+	g_res_ran++;
+	return true;
+}
+static bool cg_try_resident(CgRun& R) {
+	if (!cg_plan_resident(R)) return false;
+	KtScope kt("cg_resident", R.s->stream);
+	cg_resident_run(R.s->device, R.s->stream, R.resPlan, R.resP);
+	g_res_launches++;
 	return true;
 }
 
@@ -2061,7 +2068,7 @@ static void cg_setup(CgRun& R, Scene* s, Grid* flags, float* rhs, float* x, cons
 
 	// doInit: x = 0, r = b, bnorm; preconditioned: z = M r, sigma = dot(z, r)
 	R.launched = 0;
-	if (cg_try_resident(R)) return;
+	if (batchInit ? cg_plan_resident(R) : cg_try_resident(R)) return;
 	cg_init(R);
 	if (R.gA0 && !R.pcNone) {
 		R.gS = s->getReal();
@@ -2466,11 +2473,13 @@ static void launch_joint(hipStream_t q, long long nb, const CgRun* R, int nc, F 
 // / 483 us, 144^3 1680 / 1258, 176^3 2317 / 2331, 202^3 3310 / 4253.
 constexpr long long kJointCells = 3ll << 22;  // of all components
 constexpr int kScaledBufs = 4;                // CG vectors of one component
-static bool joint_diffusion(const Dims& d, int nc) { return nc > 1 && nc * d.n <= kJointCells && !cg_resident_plan(d).V; }
+static bool joint_diffusion(const Scene* s, int nc) {
+	return nc > 1 && nc * s->d.n <= kJointCells && !cg_resident_fits(s->device, cg_resident_plan(s->d));
+}
 static bool solve_diffusion_joint(Scene* s, Grid* flags, float* const* u, int nc, float alpha, float cgAccuracy,
                                   float cgMaxIterFac, mfx_solve_stats* stats) {
 	const Dims& d = s->d;
-	if (!joint_diffusion(d, nc)) return false;
+	if (!joint_diffusion(s, nc)) return false;
 	std::vector<float*> buf;
 	CgRun R[kJointMax];
 	auto give = [&]() {
@@ -2609,7 +2618,13 @@ static void correct_velocity(Scene* s, Grid* flags, Grid* vel, const float* pres
 // is one launch per CG/MG phase over a work list that holds the tiles of all
 // problems, so small problems share launches with large ones.  Each problem
 // keeps its own device CgState, so converged problems drop out at once
-// (their workgroups return on st->done).
+// (their workgroups return on st->done).  Unpreconditioned problems of the
+// one-kernel CG share launches too, a problem to a run of workgroups, beside
+// the others' iterations, so that each has the bits of its solve alone.  A
+// launch each, on their own streams, ran four at a time (the hardware queues).
+// 64 problems of 64^2 / 32 of 128^2 / 16 of 353x241: iterated in the work
+// lists 4098 / 6701 / 13947 us, a launch each 4746 / 9478 / 7386, together
+// 1042 / 1588 / 5596.
 // ---------------------------------------------------------------------------
 namespace {
 
@@ -2667,14 +2682,22 @@ struct BatchSolve {
 	Step<CoarsestP> crs;
 	Step<L0UpP> l0up[2];
 	Step<DotP> dot;
-	// finish: true residual partials, their sums, the velocity correction
-	Step<TrueResP> tres;
-	Step<TrueRedP> tred;
+	// one-kernel solves by kind
+	Step<ResP> one[kResKinds];
+	std::vector<ResPlan> plan[kResKinds];
+	// finish: true residual partials, their sums (of the iterated problems and
+	// of the one-kernel ones), the velocity correction
+	Step<TrueResP> tres[2];
+	Step<TrueRedP> tred[2];
 	Step<CorrVelP> corr;
 	bool anyMg = false;
 	uint8_t* dmem = nullptr;
 	CgState** dStates = nullptr;
 
+	void true_residuals(hipStream_t s, int resident) {
+		run_true_residual_many(s, tres[resident].n(), tres[resident].dItems, tres[resident].dParams);
+		run_reduce_true_rr_many(s, tred[resident].n(), tred[resident].dItems, tred[resident].dParams);
+	}
 	// an iteration of every problem, in the two parts of a single solve's
 	void part_a(hipStream_t s, int parity) {
 		run_matvec_many(s, mv[parity].n(), mv[parity].dItems, mv[parity].dParams);
@@ -2852,8 +2875,14 @@ static void solve_batch(const std::vector<Grid*>& vel, const std::vector<Grid*>&
 		B.fill = Step<FillP>((size_t)P);
 		B.crs = Step<CoarsestP>((size_t)P);
 		B.dot = Step<DotP>((size_t)P);
-		B.tres = Step<TrueResP>((size_t)P);
-		B.tred = Step<TrueRedP>((size_t)P);
+		for (int res = 0; res < 2; res++) {
+			B.tres[res] = Step<TrueResP>((size_t)P);
+			B.tred[res] = Step<TrueRedP>((size_t)P);
+		}
+		for (int k = 0; k < kResKinds; k++) {
+			B.one[k] = Step<ResP>((size_t)P);
+			B.plan[k].resize((size_t)P);
+		}
 		B.corr = Step<CorrVelP>((size_t)P);
 		for (int d3 = 0; d3 < 2; d3++) {
 			B.down[d3] = Step<L0DownP>((size_t)P);
@@ -2867,10 +2896,27 @@ static void solve_batch(const std::vector<Grid*>& vel, const std::vector<Grid*>&
 			tkey.push_back(d.nz);
 		}
 		const int policy = batch_policy(tkey);
-		int maxIt = 0;
+		int maxIt = 0, nIter = 0;  // of the problems that iterate in the work lists
 		for (int i = 0; i < P; i++) {
 			CgRun& r = R[(size_t)i];
 			const Dims& d = r.s->d;
+			MFX_CHECK(!r.scaled && !r.gA0 && d.n >= 3, "batched solve: unexpected system kind");
+			const long long nLight = tiles_for(d, kLightKZ).count();
+			const int res = r.resident ? 1 : 0;
+			B.tres[res].params[(size_t)i] = r.trueResP();
+			B.tres[res].add_tiles(i, nLight);
+			B.tred[res].params[(size_t)i] = r.trueRedP();
+			B.tred[res].add_tiles(i, 1);
+			B.corr.params[(size_t)i] = CorrVelP{d, tiles_for(d, kLightKZ), flg[(size_t)i]->f8, pres[(size_t)i]->real(),
+			                                    vel[(size_t)i]->comp(0), vel[(size_t)i]->comp(1), vel[(size_t)i]->comp(2)};
+			B.corr.add_tiles(i, nLight);
+			if (r.resident) {
+				B.one[r.resPlan.kind].params[(size_t)i] = r.resP;
+				B.one[r.resPlan.kind].add_tiles(i, r.resPlan.wg);
+				B.plan[r.resPlan.kind][(size_t)i] = r.resPlan;
+				continue;
+			}
+			nIter++;
 			maxIt = std::max(maxIt, r.maxIter);
 			bool tuned = false;
 			int fMv = 0, fL0 = 0;
@@ -2884,15 +2930,6 @@ static void solve_batch(const std::vector<Grid*>& vel, const std::vector<Grid*>&
 				B.up[par].params[(size_t)i] = r.upd(par == 1);
 				B.up[par].add_tiles(i, r.nbU);
 			}
-			MFX_CHECK(!r.scaled && !r.gA0 && d.n >= 3, "batched solve: unexpected system kind");
-			const long long nLight = tiles_for(d, kLightKZ).count();
-			B.tres.params[(size_t)i] = r.trueResP();
-			B.tres.add_tiles(i, nLight);
-			B.tred.params[(size_t)i] = r.trueRedP();
-			B.tred.add_tiles(i, 1);
-			B.corr.params[(size_t)i] = CorrVelP{d, tiles_for(d, kLightKZ), flg[(size_t)i]->f8, pres[(size_t)i]->real(),
-			                                    vel[(size_t)i]->comp(0), vel[(size_t)i]->comp(1), vel[(size_t)i]->comp(2)};
-			B.corr.add_tiles(i, nLight);
 			B.fa.params[(size_t)i] = r.fin(r.npM, FIN_ALPHA);
 			B.fa.add_tiles(i, 1);
 			B.fr.params[(size_t)i] = r.fin((int)r.nbU, FIN_RES);
@@ -2956,8 +2993,11 @@ static void solve_batch(const std::vector<Grid*>& vel, const std::vector<Grid*>&
 			f(B.fill);
 			f(B.crs);
 			f(B.dot);
-			f(B.tres);
-			f(B.tred);
+			for (int res = 0; res < 2; res++) {
+				f(B.tres[res]);
+				f(B.tred[res]);
+			}
+			for (auto& x : B.one) f(x);
 			f(B.corr);
 			for (int d3 = 0; d3 < 2; d3++) {
 				f(B.down[d3]);
@@ -2969,8 +3009,13 @@ static void solve_batch(const std::vector<Grid*>& vel, const std::vector<Grid*>&
 			}
 		};
 		placeAll([&](auto& st) { st.place(A); });
+		// the states' order: the problems that iterate, then the one-kernel ones
 		std::vector<CgState*> states((size_t)P);
-		for (int i = 0; i < P; i++) states[(size_t)i] = R[(size_t)i].st;
+		std::vector<int> pos((size_t)P);
+		for (int i = 0, a = 0, b = nIter; i < P; i++) {
+			pos[(size_t)i] = R[(size_t)i].resident ? b++ : a++;
+			states[(size_t)pos[(size_t)i]] = R[(size_t)i].st;
+		}
 		const size_t stOff = A.add(states.data(), sizeof(CgState*) * (size_t)P);
 		std::vector<CgState> gatherInit((size_t)P);
 		const size_t gatherOff = A.add(gatherInit.data(), sizeof(CgState) * (size_t)P);
@@ -3000,6 +3045,20 @@ static void solve_batch(const std::vector<Grid*>& vel, const std::vector<Grid*>&
 		B.dStates = (CgState**)(B.dmem + stOff);
 		// the batch stream waits for every problem's set-up
 		for (int i = 1; i < P; i++) MFX_HIP(hipStreamWaitEvent(q, vel[(size_t)i]->s->ev, 0));
+		// the one-kernel solves, beside the iterations on the stream of one of
+		// them (one that is not the batch stream, where there is one); sr->ev is
+		// their end
+		Scene* sr = nullptr;
+		for (int i = 0; i < P; i++)
+			if (R[(size_t)i].resident) sr = vel[(size_t)i]->s;
+		if (sr) {
+			MFX_HIP(hipEventRecord(s0->ev, q));  // the lists are up, every set-up is done
+			if (sr != s0) MFX_HIP(hipStreamWaitEvent(sr->stream, s0->ev, 0));
+			KtScope kt("cg_resident", sr->stream);
+			for (int k = 0; k < kResKinds; k++)
+				g_res_launches += cg_resident_run_many(s0->device, sr->stream, k, B.plan[k], B.one[k].dItems, B.one[k].dParams);
+			MFX_HIP(hipEventRecord(sr->ev, sr->stream));
+		}
 		// initial V-cycle of every preconditioned problem, sigma = dot(z, r)
 		if (B.anyMg) {
 			B.enqueue_vcycle(q);
@@ -3015,16 +3074,18 @@ static void solve_batch(const std::vector<Grid*>& vel, const std::vector<Grid*>&
 		CgState* hst = (CgState*)s0->hstage;  // pinned, P states
 		const double target = o.relTol > 0 ? o.relTol : (double)o.cgAccuracy;
 		if (!s0->evState) MFX_HIP(hipEventCreateWithFlags(&s0->evState, hipEventDisableTiming));
-		auto copy_states = [&]() {
-			hipLaunchKernelGGL(k_gather_states, dim3((P + 255) / 256), dim3(256), 0, q, P, (CgState* const*)B.dStates,
+		// the first n states
+		auto copy_states = [&](int n) {
+			hipLaunchKernelGGL(k_gather_states, dim3((n + 255) / 256), dim3(256), 0, q, n, (CgState* const*)B.dStates,
 			                   dGather);
-			MFX_HIP(hipMemcpyAsync(hst, dGather, sizeof(CgState) * (size_t)P, hipMemcpyDeviceToHost, q));
+			MFX_HIP(hipMemcpyAsync(hst, dGather, sizeof(CgState) * (size_t)n, hipMemcpyDeviceToHost, q));
 		};
 		// the most iterations any problem still needs (-1: unknown for some)
 		auto iters_left = [&]() {
 			int most = 0;
 			for (int i = 0; i < P; i++) {
-				const int left = cg_iters_left(hst[i], target, R[(size_t)i].pcNone);
+				if (R[(size_t)i].resident) continue;
+				const int left = cg_iters_left(hst[pos[(size_t)i]], target, R[(size_t)i].pcNone);
 				if (left < 0) return -1;
 				most = std::max(most, left);
 			}
@@ -3041,7 +3102,7 @@ static void solve_batch(const std::vector<Grid*>& vel, const std::vector<Grid*>&
 					owesB = true;
 					its++;
 					if (it == nIt - 2) {
-						copy_states();
+						copy_states(nIter);
 						MFX_HIP(hipEventRecord(s0->evState, q));
 					}
 				}
@@ -3058,26 +3119,33 @@ static void solve_batch(const std::vector<Grid*>& vel, const std::vector<Grid*>&
 					owesB = false;
 				}
 				// every problem's true residual and its sum, all states to the host
-				run_true_residual_many(q, B.tres.n(), B.tres.dItems, B.tres.dParams);
-				run_reduce_true_rr_many(q, B.tred.n(), B.tred.dItems, B.tred.dParams);
-				copy_states();
+				B.true_residuals(q, 0);
+				copy_states(nIter);
 				sync(s0);
 				const int left = iters_left();
 				if (left == 0 || its >= limit) return;
 				plan = cg_plan(left, its);
 			}
 		};
-		const auto tIter = std::chrono::steady_clock::now();
-		iterate(4, maxIt);
-		batch_policy_done(tkey, policy,
-		                  std::chrono::duration<double>(std::chrono::steady_clock::now() - tIter).count());
+		if (nIter) {
+			const auto tIter = std::chrono::steady_clock::now();
+			iterate(4, maxIt);
+			batch_policy_done(tkey, policy,
+			                  std::chrono::duration<double>(std::chrono::steady_clock::now() - tIter).count());
+		}
+		if (sr) {
+			MFX_HIP(hipStreamWaitEvent(q, sr->ev, 0));
+			B.true_residuals(q, 1);
+			copy_states(P);
+			sync(s0);
+		}
 		// each problem's state into its scene's host mirror (as a single solve
 		// leaves it), then the relTol check on the true residual: the
 		// preconditioned problems that need it restart together
 		auto mirror = [&]() {
 			for (int i = 0; i < P; i++) {
-				std::memcpy(vel[(size_t)i]->s->hscal, hst + i, sizeof(CgState));
-				R[(size_t)i].launched = hst[i].iter;
+				std::memcpy(vel[(size_t)i]->s->hscal, hst + pos[(size_t)i], sizeof(CgState));
+				R[(size_t)i].launched = hst[pos[(size_t)i]].iter;
 			}
 		};
 		mirror();
@@ -3089,8 +3157,9 @@ static void solve_batch(const std::vector<Grid*>& vel, const std::vector<Grid*>&
 				again[(size_t)i] = !r.pcNone && cg_needs_restart(r) ? 1 : 0;
 				if (!again[(size_t)i]) continue;
 				n++;
-				plan = std::max(plan, cg_restart_plan(hst[i], target));
-				limit = std::max(limit, r.maxIter - hst[i].iter);
+				const CgState& st = hst[pos[(size_t)i]];
+				plan = std::max(plan, cg_restart_plan(st, target));
+				limit = std::max(limit, r.maxIter - st.iter);
 			}
 			if (!n) break;
 			for (int i = 0; i < P; i++)
@@ -3155,8 +3224,9 @@ extern "C" long long mfx_testing_resident_wait(long long ticks) {
 	g_res_wait = ticks < 0 ? kResWaitTicks : ticks;
 	return prev;
 }
-// Testing hooks: one-kernel solves queued and given up so far; the number of
-// compute units they count with (0: the device's own).
+// Testing hooks: one-kernel solves queued and given up so far, launches of
+// them; the number of compute units they count with (0: the device's own).
+extern "C" long long mfx_testing_resident_launches() { return g_res_launches; }
 extern "C" void mfx_testing_resident_counts(long long* ran, long long* gaveUp) {
 	if (ran) *ran = g_res_ran;
 	if (gaveUp) *gaveUp = g_res_gaveup;

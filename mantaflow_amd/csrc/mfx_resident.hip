@@ -34,6 +34,7 @@
 #include <algorithm>
 #include <limits>
 #include <mutex>
+#include <type_traits>
 #include <vector>
 
 #include "mfx_batch.h"
@@ -133,16 +134,16 @@ __device__ inline void gather(const unsigned long long* slots, int nwg, unsigned
 
 }  // namespace
 
-// NT threads of V cells; MULTI: several workgroups
+// Workgroup wg of nwg, of NT threads of V cells; MULTI: several workgroups
 template <int NT, int V, bool MULTI>
-__global__ void __launch_bounds__(NT) k_cg_resident(ResP P) {
+__device__ __forceinline__ void body_cg_resident(const ResP& P, int wg, int nwg) {
 	extern __shared__ float ps[];  // p of cells c0-H .. c0+C+H-1
 	__shared__ ResShared S;
 	constexpr int C = NT * V;
 	const Dims& d = P.d;
 	const int t = threadIdx.x, lane = t & 63, w = t >> 6;
-	const int H = P.H, nwg = (int)gridDim.x;
-	const long long n = d.n, c0 = (long long)blockIdx.x * C;
+	const int H = P.H;
+	const long long n = d.n, c0 = (long long)wg * C;
 	const int cnt = (int)min((long long)C, n - c0);
 	const int sx = 1, sy = d.nx, sz = (int)d.sz;
 	CgState* st = P.st;
@@ -228,7 +229,7 @@ __global__ void __launch_bounds__(NT) k_cg_resident(ResP P) {
 			                      : lane == 2 ? (unsigned)ru
 			                      : lane == 3 ? (unsigned)(ru >> 32)
 			                                  : m0;
-			if (lane < kWordsB) xstore(slB + (size_t)blockIdx.x * kSlot + lane, tag, word);
+			if (lane < kWordsB) xstore(slB + (size_t)wg * kSlot + lane, tag, word);
 			unsigned long long g[kWordsB];
 			gather<kWordsB>(slB, nwg, tag, P.limit, &S.abort, g);
 			const bool mine = lane < nwg;
@@ -320,7 +321,7 @@ __global__ void __launch_bounds__(NT) k_cg_resident(ResP P) {
 			if (w == 0) {
 				const unsigned long long u = __builtin_bit_cast(unsigned long long, sum16(S.a));
 				if (lane < kWordsA)
-					xstore(slA + (size_t)blockIdx.x * kSlot + lane, tag, lane ? (unsigned)(u >> 32) : (unsigned)u);
+					xstore(slA + (size_t)wg * kSlot + lane, tag, lane ? (unsigned)(u >> 32) : (unsigned)u);
 				unsigned long long g[kWordsA];
 				gather<kWordsA>(slA, nwg, tag, P.limit, &S.abort, g);
 				const double s = wave_sum_to_last(lane < nwg ? word_pair(g[0], g[1]) : 0.0);
@@ -366,7 +367,7 @@ __global__ void __launch_bounds__(NT) k_cg_resident(ResP P) {
 			else resNorm = maxR < 0.f ? 3.402823466e+38f : maxR;  // (no finite or infinite value: all NaN)
 			conv = resNorm < acc;
 		}
-		if (blockIdx.x == 0 && t == 0 && iter - 1 < 64) st->hist[iter - 1] = resNorm;
+		if (wg == 0 && t == 0 && iter - 1 < 64) st->hist[iter - 1] = resNorm;
 		if (conv) {
 			sigma = resNorm;
 			converged = done = true;
@@ -392,7 +393,7 @@ __global__ void __launch_bounds__(NT) k_cg_resident(ResP P) {
 		}
 		return;
 	}
-	if (blockIdx.x == 0 && t == 0) {
+	if (wg == 0 && t == 0) {
 		st->sigma = sigma;
 		st->alpha = alpha;
 		st->beta = beta;
@@ -406,10 +407,40 @@ __global__ void __launch_bounds__(NT) k_cg_resident(ResP P) {
 		st->done = 1;
 	}
 }
+template <int NT, int V, bool MULTI>
+__global__ void __launch_bounds__(NT) k_cg_resident(ResP p) {
+	body_cg_resident<NT, V, MULTI>(p, (int)blockIdx.x, (int)gridDim.x);
+}
+// the workgroups of several solves, from workgroup `base` of the list
+template <int NT, int V, bool MULTI>
+__global__ void __launch_bounds__(NT) k_cg_resident_many(WorkList wl, const ResP* __restrict__ params, int base) {
+	const int b = base + (int)blockIdx.x, i = worklist_prob(wl, (unsigned)b), b0 = wl.start[i];
+	const ResP p = params[i];
+	body_cg_resident<NT, V, MULTI>(p, b - b0, wl.start[i + 1] - b0);
+}
 
 static __global__ void k_words_clear(unsigned long long* p, long long n) {
 	for (long long i = blockIdx.x * (long long)blockDim.x + threadIdx.x; i < n; i += (long long)gridDim.x * blockDim.x)
 		p[i] = 0;
+}
+
+struct ResKind {
+	int nt, v;  // threads, cells per thread
+	bool multi;
+};
+constexpr ResKind kResKind[kResKinds] = {{512, 4, false}, {512, 8, false}, {1024, 8, false},
+                                         {1024, 2, true}, {1024, 4, true}, {1024, 8, true}};
+// f(kind as a constant)
+template <typename F>
+static void with_kind(int kind, F&& f) {
+	switch (kind) {
+	case 0: f(std::integral_constant<int, 0>{}); break;
+	case 1: f(std::integral_constant<int, 1>{}); break;
+	case 2: f(std::integral_constant<int, 2>{}); break;
+	case 3: f(std::integral_constant<int, 3>{}); break;
+	case 4: f(std::integral_constant<int, 4>{}); break;
+	default: f(std::integral_constant<int, 5>{}); break;
+	}
 }
 
 ResPlan cg_resident_plan(const Dims& d) {
@@ -422,19 +453,15 @@ ResPlan cg_resident_plan(const Dims& d) {
 	// cells each.  Beyond, runs of as few cells as the workgroup limit allows:
 	// an iteration then is the two exchanges (4.0 us at 128^2, 4.7 at 353x241
 	// with 2048 cells a workgroup, 4.9 with 4096, 6.1 with 8192).
-	struct {
-		int nt, v;
-		bool multi;
-	} const kinds[] = {{512, 4, false}, {512, 8, false}, {1024, 8, false}, {1024, 2, true}, {1024, 4, true}, {1024, 8, true}};
-	for (const auto& k : kinds) {
+	for (int kind = 0; kind < kResKinds; kind++) {
+		const ResKind& k = kResKind[kind];
 		const long long c = (long long)k.nt * k.v;
 		if (!fits(c) || d.n > c * (k.multi ? kResMaxWG : 1)) continue;
-		r.NT = k.nt;
-		r.V = k.v;
+		r.kind = kind;
 		r.wg = (int)((d.n + c - 1) / c);
 		break;
 	}
-	if (!r.V) return r;
+	if (!r.wg) return r;
 	r.H = (int)H;
 	r.words = r.wg > 1 ? (size_t)d.n : 0;
 	return r;
@@ -454,20 +481,16 @@ unsigned cg_resident_tags(ResWords& w, hipStream_t s, const ResPlan& pl, int max
 	return e;
 }
 
-static size_t lds_bytes(const ResPlan& pl) { return ((size_t)pl.NT * pl.V + 2 * (size_t)pl.H) * sizeof(float); }
-template <int NT, int V>
-static void run_one(hipStream_t s, const ResPlan& pl, const ResP& p) {
-	hipLaunchKernelGGL((k_cg_resident<NT, V, false>), dim3(1), dim3(NT), lds_bytes(pl), s, p);
-}
-template <int V>
-static void run_multi(hipStream_t s, const ResPlan& pl, const ResP& p) {
-	hipLaunchKernelGGL((k_cg_resident<1024, V, true>), dim3((unsigned)pl.wg), dim3(1024), lds_bytes(pl), s, p);
+static size_t lds_bytes(const ResPlan& pl) {
+	const ResKind& k = kResKind[pl.kind];
+	return ((size_t)k.nt * k.v + 2 * (size_t)pl.H) * sizeof(float);
 }
 
 // Solves of several workgroups in flight on one device: a lane holds one at a
-// time.  A solve takes the lane its stream used last, else the one unused for
-// longest, and its stream waits (on the device) for the solve that was queued
-// in it before; which lane it gets changes no result.
+// time, or a batch all of them.  A solve takes the lane its stream used last,
+// else the one unused for longest, and its stream waits (on the device) for
+// the solve that was queued in it before; which lane it gets changes no
+// result.
 struct ResLane {
 	hipEvent_t ev = nullptr;  // end of the lane's last solve
 	hipStream_t last = nullptr;
@@ -485,9 +508,9 @@ void cg_resident_cus(int override) {
 	std::lock_guard<std::mutex> lk(g_res_mu);
 	g_res_cus = override;
 }
-static bool run_in_lane(int device, hipStream_t s, const ResPlan& pl, const ResP& p) {
-	if (device < 0 || device >= 64) return false;
-	std::lock_guard<std::mutex> lk(g_res_mu);
+// compute units of the device (g_res_mu held; 0: not known)
+static int units(int device) {
+	if (device < 0 || device >= 64) return 0;
 	ResDevice& D = g_res_dev[device];
 	if (D.cus < 0) {
 		// (one workgroup fits a unit: at most 1024 threads by its launch bounds,
@@ -498,31 +521,33 @@ static bool run_in_lane(int device, hipStream_t s, const ResPlan& pl, const ResP
 		MFX_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device));
 		D.cus = cus;
 	}
-	const int cus = g_res_cus > 0 ? std::min(g_res_cus, D.cus) : D.cus;
-	if (pl.wg > cus) return false;
-	const size_t lanes = (size_t)std::max(1, cus / kResMaxWG);
-	while (D.lane.size() < lanes) {
+	return g_res_cus > 0 ? std::min(g_res_cus, D.cus) : D.cus;
+}
+bool cg_resident_fits(int device, const ResPlan& pl) {
+	if (pl.wg < 2) return pl.wg == 1;
+	std::lock_guard<std::mutex> lk(g_res_mu);
+	return pl.wg <= units(device);
+}
+// the device's lanes (g_res_mu held)
+static std::vector<ResLane*> lanes(int device) {
+	ResDevice& D = g_res_dev[device];
+	const size_t n = (size_t)std::max(1, units(device) / kResMaxWG);
+	while (D.lane.size() < n) {
 		ResLane l;
 		MFX_HIP(hipEventCreateWithFlags(&l.ev, hipEventDisableTiming));
 		D.lane.push_back(l);
 	}
-	ResLane* l = &D.lane[0];
-	for (size_t i = 0; i < lanes; i++) {
-		ResLane& c = D.lane[i];
-		if (c.last == s) {
-			l = &c;
-			break;
-		}
-		if (c.used < l->used) l = &c;
-	}
+	std::vector<ResLane*> r;
+	for (size_t i = 0; i < n; i++) r.push_back(&D.lane[i]);
+	return r;
+}
+static void enter_lane(ResLane* l, hipStream_t s) {
 	if (l->last && l->last != s) MFX_HIP(hipStreamWaitEvent(s, l->ev, 0));
-	if (pl.V == 2) run_multi<2>(s, pl, p);
-	else if (pl.V == 4) run_multi<4>(s, pl, p);
-	else run_multi<8>(s, pl, p);
+}
+static void leave_lane(int device, ResLane* l, hipStream_t s) {
 	l->last = s;
-	l->used = ++D.clock;
+	l->used = ++g_res_dev[device].clock;
 	MFX_HIP(hipEventRecord(l->ev, s));
-	return true;
 }
 void cg_resident_forget(int device, hipStream_t s) {
 	if (device < 0 || device >= 64) return;
@@ -530,13 +555,71 @@ void cg_resident_forget(int device, hipStream_t s) {
 	for (ResLane& l : g_res_dev[device].lane)
 		if (l.last == s) l.last = nullptr;
 }
-bool cg_resident_run(int device, hipStream_t s, const ResPlan& pl, ResP p) {
-	p.H = pl.H;
-	if (pl.wg > 1) return run_in_lane(device, s, pl, p);
-	if (pl.NT == 512 && pl.V == 4) run_one<512, 4>(s, pl, p);
-	else if (pl.NT == 512) run_one<512, 8>(s, pl, p);
-	else run_one<1024, 8>(s, pl, p);
-	return true;
+
+void cg_resident_run(int device, hipStream_t s, const ResPlan& pl, const ResP& p) {
+	auto launch = [&]() {
+		with_kind(pl.kind, [&](auto k) {
+			constexpr ResKind K = kResKind[decltype(k)::value];
+			hipLaunchKernelGGL((k_cg_resident<K.nt, K.v, K.multi>), dim3((unsigned)pl.wg), dim3(K.nt), lds_bytes(pl), s, p);
+		});
+	};
+	if (!kResKind[pl.kind].multi) {
+		launch();
+		return;
+	}
+	std::lock_guard<std::mutex> lk(g_res_mu);
+	ResLane* l = nullptr;
+	for (ResLane* c : lanes(device)) {
+		if (c->last == s) {
+			l = c;
+			break;
+		}
+		if (!l || c->used < l->used) l = c;
+	}
+	enter_lane(l, s);
+	launch();
+	leave_lane(device, l, s);
+}
+
+// Solves of one workgroup are one launch whatever their number.  Of the
+// others as many share a launch as there are units for their workgroups, with
+// no other solve in flight (all lanes held).
+int cg_resident_run_many(int device, hipStream_t s, int kind, const std::vector<ResPlan>& pl, WorkList items,
+                         const ResP* params) {
+	size_t lds = 0;
+	for (const ResPlan& q : pl)
+		if (q.wg) lds = std::max(lds, lds_bytes(q));
+	auto launch = [&](int base, int wgs) {
+		with_kind(kind, [&](auto k) {
+			constexpr ResKind K = kResKind[decltype(k)::value];
+			hipLaunchKernelGGL((k_cg_resident_many<K.nt, K.v, K.multi>), dim3((unsigned)wgs), dim3(K.nt), lds, s, items,
+			                   params, base);
+		});
+	};
+	int base = 0, wgs = 0, launches = 0;
+	if (!kResKind[kind].multi) {
+		for (const ResPlan& q : pl) wgs += q.wg;
+		if (wgs) launch(0, wgs);
+		return wgs ? 1 : 0;
+	}
+	std::lock_guard<std::mutex> lk(g_res_mu);
+	const int most = units(device);
+	const std::vector<ResLane*> all = lanes(device);
+	for (ResLane* l : all) enter_lane(l, s);
+	auto flush = [&]() {
+		if (!wgs) return;
+		launch(base, wgs);
+		launches++;
+		base += wgs;
+		wgs = 0;
+	};
+	for (const ResPlan& q : pl) {
+		if (wgs + q.wg > most) flush();
+		wgs += q.wg;
+	}
+	flush();
+	for (ResLane* l : all) leave_lane(device, l, s);
+	return launches;
 }
 
 }  // namespace mfx

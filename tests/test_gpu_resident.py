@@ -122,6 +122,12 @@ def _counts():
     return a.value, b.value
 
 
+def _launches():
+    f = lib().mfx_testing_resident_launches
+    f.restype = C.c_longlong
+    return f()
+
+
 @contextmanager
 def _hook(name, value, back):
     f = getattr(lib(), name)
@@ -183,11 +189,13 @@ def test_resident_rests_after_giving_up(manta, oracle):
     np.testing.assert_array_equal(other[0], whole[0])
 
 
-@pytest.mark.parametrize("cus", [0, 64])
-def test_resident_solves_at_once(manta, oracle, cus):
-    """A batch's unpreconditioned problems start together, each on its own
-    solver's stream: more of them than the device holds at once (or, counted
-    with 64 units, one after another) give the bits of solves alone."""
+# by threads and cells per thread: 42, 10, 52, 42, 10, 52 workgroups, 64, 33,
+# 64, 33 and twice one; a launch holds as many as there are units (256)
+@pytest.mark.parametrize("cus,launches", [(0, 3), (64, 9)])
+def test_resident_solves_at_once(manta, oracle, cus, launches):
+    """A batch's unpreconditioned problems share launches, as many as the
+    device (or 64 units of it) holds at once, and give the bits of solves
+    alone."""
     shapes = [(353, 241, 1), (512, 512, 1), (150, 130, 1), (64, 64, 1), (363, 363, 1), (1500, 70, 1)] * 2
     kw = dict(preconditioner=manta.PcMIC, cgAccuracy=1e-4)
     single, batch = [], []
@@ -199,11 +207,36 @@ def test_resident_solves_at_once(manta, oracle, cus):
     for g, f, v, p in single:
         manta.solvePressure(flags=f, vel=v, pressure=p, **kw)
     with _hook("mfx_testing_resident_cus", C.c_int(cus), 0):
-        before = _counts()
+        before, n = _counts(), _launches()
         manta.solvePressureBatch([(v, p, f) for g, f, v, p in batch], **kw)
         assert _counts() == (before[0] + len(shapes), before[1])
+        assert _launches() - n == launches
     for (g1, f1, v1, p1), (g2, f2, v2, p2) in zip(single, batch):
         assert manta.lastSolveStats(g1.s)["iterations"] == manta.lastSolveStats(g2.s)["iterations"]
+        np.testing.assert_array_equal(p1.toNumpy(), p2.toNumpy())
+        np.testing.assert_array_equal(v1.toNumpy(), v2.toNumpy())
+
+
+@pytest.mark.parametrize("relTol", [0.0, 1e-3])
+def test_resident_beside_iterated_problems(manta, oracle, relTol):
+    """One-kernel problems first, last and among problems with a preconditioner
+    and an unpreconditioned one too large for it: each as alone."""
+    shapes = [(40, 40, 1), (24, 22, 20), (150, 130, 1), (33, 30, 28), (800, 700, 1), (90, 90, 1), (64, 64, 1)]
+    kw = dict(preconditioner=manta.PcMIC, cgAccuracy=1e-3)
+    single, batch = [], []
+    for k, shape in enumerate(shapes):
+        flags, vel = _problem(oracle, shape, 60 + k)
+        for out in (single, batch):
+            g = GpuScene(manta, shape)
+            g.s.mfxRelTol = relTol
+            out.append((g, g.flags(flags), g.mac(vel), g.real()))
+    for g, f, v, p in single:
+        manta.solvePressure(flags=f, vel=v, pressure=p, **kw)
+    manta.solvePressureBatch([(v, p, f) for g, f, v, p in batch], **kw)
+    for (g1, f1, v1, p1), (g2, f2, v2, p2) in zip(single, batch):
+        s1, s2 = manta.lastSolveStats(g1.s), manta.lastSolveStats(g2.s)
+        for key in ("iterations", "resNorm", "relResidual", "converged"):
+            assert s1[key] == s2[key], (key, s1, s2)
         np.testing.assert_array_equal(p1.toNumpy(), p2.toNumpy())
         np.testing.assert_array_equal(v1.toNumpy(), v2.toNumpy())
 
