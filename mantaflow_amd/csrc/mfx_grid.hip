@@ -77,10 +77,6 @@ float* Scene::getReal() {
 	return p;
 }
 void Scene::putReal(float* p) { freeReal.push_back(p); }
-void Scene::dropReal(float* p) {
-	owned.erase(p);
-	(void)hipFree(p);
-}
 float* Scene::getVec() {
 	if (!freeVec.empty()) {
 		float* p = freeVec.back();
@@ -92,6 +88,10 @@ float* Scene::getVec() {
 	return p;
 }
 void Scene::putVec(float* p) { freeVec.push_back(p); }
+void Scene::drop(float* p) {
+	owned.erase(p);
+	(void)hipFree(p);
+}
 
 void Scene::ensurePartials(size_t nd, size_t nf) {
 	// (without the larger buffer there is none: the old one is gone)

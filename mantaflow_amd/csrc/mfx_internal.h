@@ -124,9 +124,9 @@ struct Scene {
 	~Scene();
 	float* getReal();
 	void putReal(float* p);
-	void dropReal(float* p);  // back to the device instead of the pool (hipFree waits for what is queued)
 	float* getVec();
 	void putVec(float* p);
+	void drop(float* p);  // back to the device instead of the pool (hipFree waits for what is queued)
 	void ensurePartials(size_t nd, size_t nf);
 };
 

@@ -2480,16 +2480,20 @@ static bool solve_diffusion_joint(Scene* s, Grid* flags, float* const* u, int nc
                                   float cgMaxIterFac, mfx_solve_stats* stats) {
 	const Dims& d = s->d;
 	if (!joint_diffusion(s, nc)) return false;
+	float* rhs = nullptr;  // the components' right-hand sides
 	std::vector<float*> buf;
 	CgRun R[kJointMax];
 	auto give = [&]() {
+		if (rhs) s->putVec(rhs);
 		for (float* b : buf) s->putReal(b);
 	};
 	try {
-		for (int i = 0; i < (kScaledBufs + 1) * nc; i++) buf.push_back(s->getReal());
+		rhs = s->getVec();
+		for (int i = 0; i < kScaledBufs * nc; i++) buf.push_back(s->getReal());
 		for (int c = 0; c < nc; c++) {
-			float** b = &buf[(size_t)((kScaledBufs + 1) * c)];
-			const size_t per = scaled_shape(R[c], s, flags, b[4], u[c], alpha, cgAccuracy, cgMaxIterFac, nc);
+			float** b = &buf[(size_t)(kScaledBufs * c)];
+			const size_t per =
+			    scaled_shape(R[c], s, flags, rhs + c * s->cstride, u[c], alpha, cgAccuracy, cgMaxIterFac, nc);
 			R[c].dpart += 3 * per * (size_t)c;
 			R[c].fpart += 2 * per * (size_t)c;
 			R[c].st += c;
@@ -2502,8 +2506,10 @@ static bool solve_diffusion_joint(Scene* s, Grid* flags, float* const* u, int nc
 		// one component needs its vectors and a right-hand side; the rest goes
 		// back to the device, not to the pool
 		(void)hipGetLastError();
+		if (rhs) s->drop(rhs);
+		rhs = nullptr;
 		while (buf.size() > kScaledBufs + 1) {
-			s->dropReal(buf.back());
+			s->drop(buf.back());
 			buf.pop_back();
 		}
 		give();
