@@ -282,13 +282,31 @@ __global__ void k_mult_add(float* __restrict__ g, const float* __restrict__ a, c
 		g[i] = g[i] * a[i] + b[i];
 }
 
+// An operation queued on s's stream with a further grid: equal sizes, and where
+// that is another solver's, whose stream knows nothing of this one, its queue
+// has drained before and the operation is done when it returns.
+struct With {
+	Scene* s;
+	bool wait = false;
+	explicit With(Scene* scene) : s(scene) {}
+	void operator()(const Grid* o, const char* msg = "different grid resolutions") {
+		if (!o || o->s == s) return;
+		MFX_CHECK(o->s->d.nx == s->d.nx && o->s->d.ny == s->d.ny && o->s->d.nz == s->d.nz, msg);
+		sync(o->s);
+		wait = true;
+	}
+	void done() const {
+		if (wait) sync(s);
+	}
+};
+
 static void elementwise(Grid* g, const Grid* other, int op, const float* v, const float* v2) {
 	Scene* s = g->s;
 	long long n = s->d.n;
 	unsigned nb = flat_blocks(n);
+	With with(s);
 	if (other) {
-		MFX_CHECK(other->s->d.nx == s->d.nx && other->s->d.ny == s->d.ny && other->s->d.nz == s->d.nz,
-		          "different grid resolutions");
+		with(other);
 		MFX_CHECK((other->type & (kTypeVec3 | kTypeInt | kTypeReal)) == (g->type & (kTypeVec3 | kTypeInt | kTypeReal)),
 		          "grid types do not match");
 	}
@@ -306,6 +324,7 @@ static void elementwise(Grid* g, const Grid* other, int op, const float* v, cons
 		float a = v ? v[0] : 0.f, b = v2 ? v2[0] : 0.f;
 		launch_elementwise_f(s, g->real(), other ? (const float*)other->real() : nullptr, n, op, a, b);
 	}
+	with.done();
 }
 
 // ---------------------------------------------------------------------------
@@ -1017,14 +1036,14 @@ int mfx_grid_copy(mfx_grid* dst, const mfx_grid* src) {
 	NEED(dst, "grid");
 	NEED(src, "grid");
 	Grid *a = G(dst), *b = G(src);
-	MFX_CHECK(a->s->d.nx == b->s->d.nx && a->s->d.ny == b->s->d.ny && a->s->d.nz == b->s->d.nz,
-	          "different grid resolutions");
-	MFX_CHECK(a->isVec() == b->isVec(), "copyFrom: grid types do not match");
 	Scene* s = a->s;
-	if (a->s != b->s) MFX_HIP(hipStreamSynchronize(b->s->stream));
+	With with(s);
+	with(b);
+	MFX_CHECK(a->isVec() == b->isVec(), "copyFrom: grid types do not match");
 	size_t bytes = a->isVec() ? 3 * s->cstride * 4 : (size_t)s->d.n * 4;
 	MFX_HIP(hipMemcpyAsync(a->data, b->data, bytes, hipMemcpyDeviceToDevice, s->stream));
 	if (a->isFlags()) flags_repack(a);
+	with.done();
 	API_END
 }
 
@@ -1033,8 +1052,9 @@ int mfx_grid_swap(mfx_grid* x, mfx_grid* y) {
 	NEED(x, "grid");
 	NEED(y, "grid");
 	Grid *a = G(x), *b = G(y);
-	MFX_CHECK(a->s->d.nx == b->s->d.nx && a->s->d.ny == b->s->d.ny && a->s->d.nz == b->s->d.nz,
-	          "Grid::swap(): Grid dimensions mismatch.");
+	With with(a->s);
+	with(b, "Grid::swap(): Grid dimensions mismatch.");
+	with.done();
 	MFX_CHECK(!a->external && !b->external, "Grid::swap(): Cannot swap if one grid stores externalData.");
 	MFX_CHECK(a->isVec() == b->isVec() && a->isFlags() == b->isFlags(), "Grid::swap(): grid types differ.");
 	if (a->s != b->s) {
@@ -1105,10 +1125,10 @@ int mfx_grid_mult_add(mfx_grid* g, const mfx_grid* a, const mfx_grid* b) {
 	Grid *x = G(g), *y = G(a), *z = G(b);
 	MFX_CHECK(x->isReal() && y->isReal() && z->isReal(), "mult+add: needs Real grids");
 	MFX_CHECK(z != x, "mult+add: the added grid must not be the result grid");
-	for (const Grid* o : {y, z})
-		MFX_CHECK(o->s->d.nx == x->s->d.nx && o->s->d.ny == x->s->d.ny && o->s->d.nz == x->s->d.nz,
-		          "different grid resolutions");
 	Scene* s = x->s;
+	With with(s);
+	with(y);
+	with(z);
 	const long long n = s->d.n;
 	float* gp = x->real();
 	const float *ap = y->real(), *bp = z->real();
@@ -1117,6 +1137,7 @@ int mfx_grid_mult_add(mfx_grid* g, const mfx_grid* a, const mfx_grid* b) {
 		                   (const float4*)ap, (const float4*)bp, n / 4);
 	else
 		hipLaunchKernelGGL(k_mult_add, dim3(flat_blocks(n)), dim3(256), 0, s->stream, gp, ap, bp, n);
+	with.done();
 	API_END
 }
 int mfx_grid_add_scaled(mfx_grid* g, const mfx_grid* a, const float* factor) {
@@ -1183,7 +1204,8 @@ int mfx_grid_max_diff(const mfx_grid* a, const mfx_grid* b, double* out) {
 	Grid *x = G(a), *y = G(b);
 	Scene* s = x->s;
 	MFX_CHECK(x->isVec() == y->isVec() && x->isInt() == y->isInt(), "gridMaxDiff: grid types differ");
-	if (x->s != y->s) MFX_HIP(hipStreamSynchronize(y->s->stream));
+	With with(s);
+	with(y);
 	unsigned nb = flat_blocks(s->d.n, 256, 4096);
 	s->ensurePartials(nb, 0);
 	int mode = x->isInt() ? 1 : (x->isVec() ? 2 : 0);
@@ -1207,8 +1229,11 @@ int mfx_get_component(const mfx_grid* vec, mfx_grid* real, int c) {
 	MFX_CHECK(c >= 0 && c < 3, "component out of range");
 	Grid *v = G(vec), *r = G(real);
 	MFX_CHECK(v->isVec() && r->isReal(), "getComponent: needs a Vec3 source and a Real target");
+	With with(v->s);
+	with(r);
 	hipLaunchKernelGGL(k_copy, dim3(flat_blocks(v->s->d.n)), dim3(256), 0, v->s->stream, r->real(),
 	                   (const float*)v->comp(c), v->s->d.n);
+	with.done();
 	API_END
 }
 int mfx_set_component(const mfx_grid* real, mfx_grid* vec, int c) {
@@ -1218,8 +1243,11 @@ int mfx_set_component(const mfx_grid* real, mfx_grid* vec, int c) {
 	MFX_CHECK(c >= 0 && c < 3, "component out of range");
 	Grid *v = G(vec), *r = G(real);
 	MFX_CHECK(v->isVec() && r->isReal(), "setComponent: needs a Real source and a Vec3 target");
+	With with(v->s);
+	with(r);
 	hipLaunchKernelGGL(k_copy, dim3(flat_blocks(v->s->d.n)), dim3(256), 0, v->s->stream, v->comp(c),
 	                   (const float*)r->real(), v->s->d.n);
+	with.done();
 	API_END
 }
 int mfx_copy_mac_to_vec3(const mfx_grid* mac, mfx_grid* vec) {
@@ -1228,9 +1256,12 @@ int mfx_copy_mac_to_vec3(const mfx_grid* mac, mfx_grid* vec) {
 	NEED(vec, "grid");
 	Grid *m = G(mac), *v = G(vec);
 	MFX_CHECK(m->isVec() && v->isVec(), "copyMacToVec3: needs Vec3 grids");
+	With with(m->s);
+	with(v);
 	for (int c = 0; c < 3; c++)
 		hipLaunchKernelGGL(k_copy, dim3(flat_blocks(m->s->d.n)), dim3(256), 0, m->s->stream, v->comp(c),
 		                   (const float*)m->comp(c), m->s->d.n);
+	with.done();
 	API_END
 }
 
@@ -1282,6 +1313,8 @@ int mfx_flags_count_cells(const mfx_grid* gg, int flag, int bnd, mfx_grid* mask,
 	Grid* g = G(gg);
 	Scene* s = g->s;
 	MFX_CHECK(!mask || G(mask)->isReal(), "countCells: mask must be a Real grid");
+	With with(s);
+	if (mask) with(G(mask));
 	unsigned nb = flat_blocks(s->d.n, 256, 4096);
 	s->ensurePartials(nb, 0);
 	hipLaunchKernelGGL(k_count_cells, dim3(nb), dim3(256), 0, s->stream, (const int*)g->data, s->d, flag, bnd,
@@ -1328,12 +1361,16 @@ int mfx_reset_outflow(mfx_grid* gg, mfx_grid* phi, mfx_grid* real) {
 	MFX_CHECK(!phi || G(phi)->isReal(), "resetOutflow: phi must be a Real grid");
 	MFX_CHECK(!real || G(real)->isReal(), "resetOutflow: real must be a Real grid");
 	Scene* s = g->s;
+	With with(s);
+	if (phi) with(G(phi));
+	if (real) with(G(real));
 	flags_touched(g);
 	// (the outflow flags themselves are not changed here: the list stays valid)
 	const unsigned* count = nullptr;
 	const unsigned* list = outflow_list(g, &count);
 	hipLaunchKernelGGL(k_reset_outflow, dim3(kOutflowListBlocks), dim3(256), 0, s->stream, g->ints(), g->f8,
 	                   phi ? G(phi)->real() : nullptr, real ? G(real)->real() : nullptr, list, count);
+	with.done();
 	API_END
 }
 
@@ -1378,12 +1415,15 @@ int mfx_apply_shape(mfx_grid* gg, int kind, const float* a, const float* b, floa
 	else if (g->isMAC()) mode = 3;
 	else if (g->isVec()) mode = 2;
 	else mode = 1;
+	With with(s);
+	if (respectFlags) with(G(respectFlags));
 	const uint8_t* resp = respectFlags ? G(respectFlags)->f8 : nullptr;
 	hipLaunchKernelGGL(k_apply_shape, dim3(flat_blocks(s->d.n)), dim3(256), 0, s->stream, sh, s->d, mode,
 	                   g->isInt() ? nullptr : g->comp(0), g->isVec() ? g->comp(1) : nullptr,
 	                   g->isVec() ? g->comp(2) : nullptr, g->isInt() ? g->ints() : nullptr, value[0],
 	                   g->isVec() ? value[1] : 0.f, g->isVec() ? value[2] : 0.f, resp);
 	if (g->isFlags()) flags_repack(g);
+	with.done();
 	API_END
 }
 

@@ -124,3 +124,67 @@ def test_partial_sums_after_a_failed_growth(manta, oracle):
         out.append((p.toNumpy(), v.toNumpy()))
     np.testing.assert_array_equal(out[0][0], out[1][0])
     np.testing.assert_array_equal(out[0][1], out[1][1])
+
+
+def test_grids_of_two_solvers(manta):
+    """An operation on grids of two solvers (equal sizes are all that the
+    reference asks for) comes after what either has queued, and before what
+    either queues next."""
+    shape = (160, 150, 140)
+    n = 160 * 150 * 140
+    a, b = GpuScene(manta, shape), GpuScene(manta, shape)
+    x, v = a.real(), a.vec()
+    y, w = b.real(), b.vec()
+    one = manta.vec3(1, 1, 1)
+
+    def queue():
+        # some hundred microseconds of work on the first solver's stream
+        x.setConst(0.0)
+        v.setConst(manta.vec3(0, 0, 0))
+        for _ in range(40):
+            x.addConst(1.0)
+            v.addConst(one)
+
+    def copy():
+        y.copyFrom(x)
+
+    def add():
+        y.add(x)
+
+    def mult():
+        y.mult(x)
+
+    def component():
+        manta.getComponent(v, y, 1)
+
+    def back():
+        manta.setComponent(x, w, 2)
+
+    def swap():
+        check(lib().mfx_grid_swap(y._h, x._h))
+
+    for op, start, want in ((copy, 0.0, 40.0), (add, 2.0, 42.0), (mult, 0.5, 20.0), (component, 0.0, 40.0),
+                            (back, 0.0, 0.0), (swap, 0.0, 40.0)):
+        y.setConst(start)
+        w.setConst(manta.vec3(0, 0, 0))
+        queue()
+        op()
+        x.setConst(-1.0)
+        v.setConst(manta.vec3(-1, -1, -1))
+        assert (y.toNumpy() == want).all(), op.__name__
+        if op is back:
+            got = w.toNumpy().reshape(n, 3)
+            assert (got[:, 2] == 40.0).all() and not got[:, :2].any()
+
+
+def test_two_solvers_of_unequal_size(manta):
+    """Component copies and resetOutflow's grids are as large as their partner."""
+    a, b = GpuScene(manta, (16, 12, 10)), GpuScene(manta, (16, 12, 11))
+    v, r = a.vec(), b.real()
+    f = b.s.create(manta.FlagGrid)
+    f.initDomain()
+    small = a.real()
+    for call in (lambda: manta.getComponent(v, r, 0), lambda: manta.setComponent(r, v, 0),
+                 lambda: manta.resetOutflow(flags=f, real=small)):
+        with pytest.raises(RuntimeError, match="different grid resolutions"):
+            call()
