@@ -16,8 +16,8 @@
 //    sequential bucket-heap selection (:520-578) keeps the interpolation full
 //    rank; here rank-deficient directions are harmless because
 //  * the coarsest level is solved exactly by a dense generalised inverse in
-//    FP64 (Cholesky of the active operator with zero pivots dropped, built once
-//    per hierarchy on the host, applied as a GEMV on the GPU) instead of a
+//    FP64 (blocked symmetric sweep of the active operator with zero pivots
+//    dropped, on the GPU once per hierarchy, applied as a GEMV) instead of a
 //    sequential FP64 Jacobi-PCG (:796-902).  This also makes the V-cycle well
 //    defined for pure-Neumann problems without pinning a pressure value.
 //  * level 0 is matrix-free: its stencil comes from the per-cell matrix code.

@@ -37,7 +37,6 @@
 #include <atomic>
 #include <exception>
 #include <thread>
-#include <deque>
 #include <cmath>
 #include <cstring>
 
@@ -3254,6 +3253,12 @@ extern "C" int mfx_testing_set_zmarch_chunks(int nx, int ny, int nz, int mv, int
 
 struct mfx_grid : public Grid {};
 struct mfx_scene : public Scene {};
+// Testing hook: the first tag not used yet on a scene's exchange words.
+extern "C" unsigned mfx_testing_resident_next(mfx_scene* s, unsigned next) {
+	const unsigned prev = s->res.next;
+	if (next) s->res.next = next;
+	return prev;
+}
 static inline Grid* G(const mfx_grid* g) { return const_cast<Grid*>(static_cast<const Grid*>(g)); }
 
 #define API_BEGIN try {

@@ -71,12 +71,6 @@ __device__ inline double sum16(const double* sh) {
 	const unsigned hi = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)(u >> 32), 15);
 	return __builtin_bit_cast(double, ((unsigned long long)hi << 32) | lo);
 }
-__device__ inline double last_lane(double v) {
-	const unsigned long long u = __builtin_bit_cast(unsigned long long, v);
-	const unsigned lo = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)u, 63);
-	const unsigned hi = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)(u >> 32), 63);
-	return __builtin_bit_cast(double, ((unsigned long long)hi << 32) | lo);
-}
 // maximum over the wavefront, valid in lane 63 (the moves of wave_sum_to_last;
 // a lane that a move does not write keeps its own value)
 template <int CTRL, int ROWS>

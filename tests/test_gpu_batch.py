@@ -42,12 +42,11 @@ def test_batch_equals_single(manta, oracle, pc):
         np.testing.assert_array_equal(v1.toNumpy(), v2.toNumpy())
 
 
-def test_batch_repeated_direct_capture_replay(manta, oracle):
+def test_batch_repeated_over_chunk_policies(manta, oracle):
     """The same batch solved twelve times in a row: the chunk autotuner's
-    eight trial solves (four plane-chunk policies, queued launches), then the
-    chosen policy's queued launches, the capture of its two-iteration graph
-    and the replays.  Every pass starts from the same velocity and must give
-    results bit-identical to single solves."""
+    eight trial solves (four plane-chunk policies), then the chosen policy.
+    Every pass starts from the same velocity and must give results
+    bit-identical to single solves."""
     kw = dict(preconditioner=manta.PcMGStatic, cgAccuracy=1e-4)
     single, batch, vel0 = [], [], []
     for k, (shape, frac) in enumerate(PROBLEMS):

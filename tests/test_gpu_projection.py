@@ -193,6 +193,54 @@ def test_zmarch_matvec_tile_edges(manta, oracle, shape):
         setc(*shape, 0, 0)
 
 
+@pytest.mark.parametrize("at", [0.0, 0.37, 1.0])
+@pytest.mark.parametrize("nz", [1020, 1028, 4100])
+def test_scalar_reduction_adds_every_partial_once(manta, oracle, nz, at):
+    """Two iterations of plain CG on 70x20 columns (4 partial sums per 4
+    planes, around once and four times the 1024 threads of the scalar
+    reduction; the smallest holds 45 of 1.2 to 5 million cells) against FP64
+    numpy: a partial dropped or added twice moves alpha or beta by 9e-6 at
+    least, most by 1e-3.  Float rounding leaves some 1e-7 in a scalar and in
+    the iterate.  A spike in the right-hand side puts the largest residual
+    into the first, a middle or the last of the blocks."""
+    shape = (70, 20, nz)
+    flags = oracle.init_domain(shape)
+    flags.reshape(nz, 20, 70)[1:-1, 1:-1, 1:-1] = 1
+    fluid = flags.reshape(nz, 20, 70) == 1
+    b = np.where(fluid, np.random.default_rng(nz).uniform(0.5, 1.5, fluid.shape), 0).astype(np.float32)
+    cells = np.flatnonzero(fluid.ravel())
+    b.ravel()[cells[int(at * (cells.size - 1))]] = 40.0
+
+    diag = np.zeros(fluid.shape)
+    for ax in range(3):
+        for sh in (1, -1):
+            diag += np.roll(fluid, sh, ax)
+    def A(x):
+        out = diag * x
+        for ax in range(3):
+            for sh in (1, -1):
+                out -= np.roll(x, sh, ax)
+        return np.where(fluid, out, 0.0)
+    x, r = np.zeros(fluid.shape), b.astype(np.float64)
+    p, sigma = r.copy(), (r * r).sum()
+    for _ in range(2):
+        q = A(p)
+        alpha = sigma / (q * p).sum()
+        x += alpha * p
+        r -= alpha * q
+        p, sigma = r + (r * r).sum() / sigma * p, (r * r).sum()
+
+    g = GpuScene(manta, shape)
+    f, v, rhs, pr = g.flags(flags), g.mac(), g.real(b.ravel()), g.real()
+    manta.solvePressureSystem(rhs=rhs, vel=v, pressure=pr, flags=f, cgAccuracy=1e-6, cgMaxIterFac=2.5 / nz,
+                              preconditioner=manta.PcNone)
+    st = manta.lastSolveStats(g.s)
+    got = pr.toNumpy().reshape(fluid.shape).astype(np.float64)
+    assert st["iterations"] == 2
+    assert np.linalg.norm(got - x) <= 5e-6 * np.linalg.norm(x)
+    assert abs(st["resNorm"] - np.abs(r).max()) <= 1e-5 * np.abs(r).max()
+
+
 @pytest.mark.parametrize("nz", [1020, 1028, 4100])
 def test_scalar_reduction_partial_counts(manta, oracle, nz):
     """65x17 columns leave 4 partial sums per 4 planes: fewer than, just more

@@ -96,15 +96,40 @@ def test_resident_fallback(manta, oracle, shape):
     flags, vel = _problem(oracle, shape, 10)
     kw = dict(cgAccuracy=1e-4)
     want = _solve(manta, shape, flags, vel, general=True, **kw)
-    wait = lib().mfx_testing_resident_wait
-    import ctypes as C
-    wait.restype, wait.argtypes = C.c_longlong, [C.c_longlong]
-    wait(0)
-    try:
-        _close(_solve(manta, shape, flags, vel, **kw), want)
-    finally:
-        wait(-1)
+    before = _counts()
+    with _hook("mfx_testing_resident_wait", C.c_longlong(0), -1):
+        got = _solve(manta, shape, flags, vel, **kw)
+    assert _counts() == (before[0] + 1, before[1] + 1)
+    _close(got, want)
+    np.testing.assert_array_equal(got[0], want[0])
     _close(_solve(manta, shape, flags, vel, **kw), want)
+    assert _counts() == (before[0] + 2, before[1] + 1)
+
+
+def test_resident_tags_wrap(manta, oracle):
+    """The words carry 32-bit tags; before they run out the words are cleared
+    and the count starts again.  The solve that ends at the last tag and the
+    ones after it give the bits of the first."""
+    shape = (150, 130, 1)
+    flags, vel = _problem(oracle, shape, 15)
+    g = GpuScene(manta, shape)
+    f, v, p = g.flags(flags), g.mac(vel), g.real()
+    tag = lib().mfx_testing_resident_next
+    tag.restype, tag.argtypes = C.c_uint, [C.c_void_p, C.c_uint]
+    seen, out = [], []
+    for k in range(4):
+        if k == 1:
+            need = seen[0] - 1  # tags of one solve
+            tag(g.s._h, 2 ** 32 - 1 - need)
+        v.fromNumpy(vel)
+        before = _counts()
+        manta.solvePressure(flags=f, vel=v, pressure=p, preconditioner=manta.PcNone, cgAccuracy=1e-4)
+        assert _counts() == (before[0] + 1, before[1])
+        seen.append(tag(g.s._h, 0))
+        out.append(p.toNumpy().copy())
+    assert seen[1] == 2 ** 32 - 1 and seen[2] == 1 + need and seen[3] == 1 + 2 * need
+    for o in out[1:]:
+        np.testing.assert_array_equal(o, out[0])
 
 
 def test_resident_nan_diverges(manta, oracle):
