@@ -69,7 +69,9 @@ int mfx_scene_set_dt(mfx_scene* s, float dt);
 int mfx_scene_get_dt(const mfx_scene* s, float* dt);
 /* wait for all work queued on the scene's stream */
 int mfx_scene_sync(mfx_scene* s);
-/* bytes of device memory held by the scene (grids, temporaries, MG cache) */
+/* bytes of device memory held by the scene: grids, pooled temporaries, multigrid
+ * hierarchies (PcMGStatic's and PcMIC's are kept for their matrix, PcMGDynamic's
+ * until a solve uses another kind or mfx_release_mg) */
 int mfx_scene_memory(const mfx_scene* s, size_t* bytes);
 
 /* ----------------------------------------------------------------- grids */
@@ -248,8 +250,9 @@ int mfx_solve_pressure_batch(int count, mfx_grid* const* vel, mfx_grid* const* p
  * with preconditioner MFX_PC_NONE (or MFX_PC_MIC in 2D), bit-identical to it,
  * with the right-hand side, CG vectors, matrix code and partial sums in one
  * library-held device array instead of pooled allocations.  No counterpart in
- * the reference; it is for callers that cannot allocate device memory (code
- * under HIP graph capture, tight serving loops).  Limits: at most 2^20 cells
+ * the reference; it is for callers that cannot allocate device memory (tight
+ * serving loops).  It waits for its stream, as every solve does, so it cannot be
+ * captured into a HIP graph.  Limits: at most 2^20 cells
  * and 65536 partial-sum slots per launch (rejected with an error beyond).
  * Every call on a GPU shares that GPU's array, so calls that overlap on one
  * GPU (two scenes, two threads) race; serialise them.  Other preconditioners

@@ -2469,7 +2469,10 @@ static void launch_joint(hipStream_t q, long long nb, const CgRun* R, int nc, F 
 // one by one: grids of the one-kernel CG, larger grids, and when the further
 // buffers cannot be had.  The line: the systems' vectors have to stay in the
 // 256 MB last-level cache.  Three components, one by one / together: 84^3 984
-// / 483 us, 144^3 1680 / 1258, 176^3 2317 / 2331, 202^3 3310 / 4253.
+// / 483 us, 144^3 1680 / 1258, 176^3 2317 / 2331, 202^3 3310 / 4253.  The lower
+// line is where the one-kernel CG ends; it runs the components one by one in
+// 365 us at 32^3, 454 at 48^3, 578 at 64^3 and 673 at 75x75x46 (general kernels,
+// one by one: 1270 to 1390), a joint solve of 68^3 takes 502.
 constexpr long long kJointCells = 3ll << 22;  // of all components
 constexpr int kScaledBufs = 4;                // CG vectors of one component
 static bool joint_diffusion(const Scene* s, int nc) {

@@ -11,7 +11,7 @@
 // row, in 3D one plane, on each side) is in LDS, and only the two dot
 // products and the residuals along the run's ends leave the workgroup.  An
 // iteration is bound by the latency of its reductions: 64^2 (one workgroup)
-// 15.6 -> 2.2 us, 353x241 (42 workgroups) 15.3 -> 4.7 us, 24^3 (7) 5.3 us.
+// 15.6 -> 2.05 us, 353x241 (42 workgroups) 15.3 -> 4.6 us, 24^3 (7) 4.8 us.
 //
 // Workgroups meet through memory twice per iteration without a grid barrier:
 // every word exchanged carries the number of the iteration it belongs to in
@@ -442,11 +442,15 @@ ResPlan cg_resident_plan(const Dims& d) {
 	const long long H = d.is3d ? d.sz : (long long)d.nx;
 	auto fits = [&](long long c) { return (c + 2 * H) * (long long)sizeof(float) <= kMaxLds; };
 	// One workgroup up to 8192 cells, where a second one costs more in waits
-	// than it saves in arithmetic (64^2: 2.2 us an iteration, 3.9 with two;
-	// 90^2: 3.2 against 4.0), of as few threads as hold the grid at up to 8
+	// than it saves in arithmetic (64^2: 2.1 us an iteration, 3.9 with two;
+	// 90^2: 3.0 against 4.0), of as few threads as hold the grid at up to 8
 	// cells each.  Beyond, runs of as few cells as the workgroup limit allows:
-	// an iteration then is the two exchanges (4.0 us at 128^2, 4.7 at 353x241
-	// with 2048 cells a workgroup, 4.9 with 4096, 6.1 with 8192).
+	// an iteration then is the two exchanges (4.2 us at 128^2, 4.6 at 353x241
+	// with 2048 cells a workgroup, 4.9 with 4096, 6.1 with 8192).  Where a plane
+	// or a row is half a run and more, the words of the runs' ends add to it, and
+	// it still takes less than the general kernels' four launches, a whole solve
+	// per iteration: 48^3 7.4 us against 15.4, 64^3 9.8 / 15.4, 75x75x46 11.5 /
+	// 15.3, 60x59x146 12.4 / 16.2, 3500x140 10.8 / 16.3.
 	for (int kind = 0; kind < kResKinds; kind++) {
 		const ResKind& k = kResKind[kind];
 		const long long c = (long long)k.nt * k.v;
