@@ -12,6 +12,7 @@ import ctypes as C
 import os
 import subprocess
 import sys
+from concurrent.futures import ThreadPoolExecutor
 from contextlib import contextmanager
 
 import numpy as np
@@ -240,6 +241,36 @@ def test_resident_solves_at_once(manta, oracle, cus, launches):
         assert manta.lastSolveStats(g1.s)["iterations"] == manta.lastSolveStats(g2.s)["iterations"]
         np.testing.assert_array_equal(p1.toNumpy(), p2.toNumpy())
         np.testing.assert_array_equal(v1.toNumpy(), v2.toNumpy())
+
+
+@pytest.mark.parametrize("cus", [0, 128, 64])
+def test_resident_solves_on_threads(manta, oracle, cus):
+    """Solvers on threads of their own, each on its own stream, solve at once,
+    again and again: more workgroups than fit together (297; counted with 128
+    and 64 units two solves and one at a time).  None gives up waiting and each
+    result is that of the solve alone."""
+    shapes = [(353, 241, 1), (512, 512, 1), (150, 130, 1), (363, 363, 1), (1500, 70, 1), (70, 60, 40), (48, 48, 48)]
+    work = []
+    for k, shape in enumerate(shapes):
+        flags, vel = _problem(oracle, shape, 80 + k)
+        g = GpuScene(manta, shape)
+        f, v, p = g.flags(flags), g.mac(vel), g.real()
+
+        def solve(f=f, v=v, p=p, vel=vel):
+            v.fromNumpy(vel)
+            manta.solvePressure(flags=f, vel=v, pressure=p, preconditioner=manta.PcNone, cgAccuracy=1e-4)
+            return p.toNumpy().copy(), v.toNumpy().copy()
+        work.append((g, solve, solve()))
+    with _hook("mfx_testing_resident_cus", C.c_int(cus), 0):
+        before = _counts()
+        with ThreadPoolExecutor(len(work)) as ex:
+            runs = [ex.submit(lambda s=solve: [s() for _ in range(4)]) for _, solve, _ in work]
+            got = [r.result(timeout=60) for r in runs]
+        assert _counts() == (before[0] + 4 * len(work), before[1])
+    for (_, _, want), out in zip(work, got):
+        for o in out:
+            np.testing.assert_array_equal(o[0], want[0])
+            np.testing.assert_array_equal(o[1], want[1])
 
 
 @pytest.mark.parametrize("relTol", [0.0, 1e-3])
