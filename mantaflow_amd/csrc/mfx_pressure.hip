@@ -1900,12 +1900,13 @@ static void cg_init(CgRun& R) {
 }
 
 // Unpreconditioned solves of grids that fit the one-kernel CG: doInit and
-// every iteration as one launch.  Returns false where the general kernels
-// have to run.  A workgroup that waits 1 s for another (a wait is some
-// microseconds) gives up; cg_verify then runs the solve on the general kernels, and so do the
-// next kResRest solves on the same exchange words, so that a device shared
-// with something that keeps the workgroups apart costs that wait once in so
-// many solves and not in each.
+// every iteration as one launch, here or with other problems of a batch.
+// cg_plan_resident returns false where the general kernels have to run.  A
+// workgroup that waits 1 s for another (a wait is some microseconds) gives up;
+// cg_verify then runs the solve on the general kernels, and so do the next
+// kResRest solves on the same exchange words, so that a device shared with
+// something that keeps the workgroups apart costs that wait once in so many
+// solves and not in each.
 constexpr long long kResWaitTicks = 100000000ll;
 constexpr int kResRest = 1000;
 static long long g_res_wait = kResWaitTicks;
